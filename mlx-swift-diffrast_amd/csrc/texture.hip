@@ -67,8 +67,29 @@ __device__ __forceinline__ int apply_boundary(int t, int size, int mode, float& 
   return r;
 }
 
+// t mod size and (t + 1) mod size, both in [0, size).  While |t| < 2^22 the
+// quotient comes from a float product whose error is below one (t is exact
+// in fp32, the reciprocal good to an ulp), corrected by one step; the
+// integer remainder it replaces is a 25-instruction sequence per tap
+// (bilinear wrap, 4 x 1000^2 x 3: forward 40 -> 38 us).
+__device__ __forceinline__ void wrap_pair(int t, int size, int& i0, int& i1) {
+  if ((unsigned)t + (1u << 22) < (1u << 23)) {
+    const int q = f2i(floorf((float)t * __builtin_amdgcn_rcpf((float)size)));
+    int r = t - q * size;
+    r += r < 0 ? size : 0;
+    r -= r >= size ? size : 0;
+    i0 = r;
+    i1 = r + 1 == size ? 0 : r + 1;
+  } else {
+    float unused;
+    i0 = apply_boundary(t, size, DR_BOUNDARY_WRAP, unused);
+    i1 = apply_boundary(t + 1, size, DR_BOUNDARY_WRAP, unused);
+  }
+}
+
 struct Bilin {
   int ix0, ix1, iy0, iy1;
+  int tx0, ty0;  // ix0, iy0 before the boundary mode
   float fx, fy, m00, m10, m01, m11, w00, w10, w01, w11;
 };
 
@@ -81,11 +102,18 @@ __device__ __forceinline__ Bilin bilin(float u, float v, int Wk, int Hk, int mod
   const int tx1 = tx0 + 1, ty1 = ty0 + 1;
   b.fx = tx - (float)tx0;
   b.fy = ty - (float)ty0;
-  float ox0, ox1, oy0, oy1;
-  b.ix0 = apply_boundary(tx0, Wk, mode, ox0);
-  b.ix1 = apply_boundary(tx1, Wk, mode, ox1);
-  b.iy0 = apply_boundary(ty0, Hk, mode, oy0);
-  b.iy1 = apply_boundary(ty1, Hk, mode, oy1);
+  b.tx0 = tx0;
+  b.ty0 = ty0;
+  float ox0 = 0.0f, ox1 = 0.0f, oy0 = 0.0f, oy1 = 0.0f;
+  if (mode == DR_BOUNDARY_WRAP) {
+    wrap_pair(tx0, Wk, b.ix0, b.ix1);
+    wrap_pair(ty0, Hk, b.iy0, b.iy1);
+  } else {
+    b.ix0 = apply_boundary(tx0, Wk, mode, ox0);
+    b.ix1 = apply_boundary(tx1, Wk, mode, ox1);
+    b.iy0 = apply_boundary(ty0, Hk, mode, oy0);
+    b.iy1 = apply_boundary(ty1, Hk, mode, oy1);
+  }
   b.m00 = (1.0f - ox0) * (1.0f - oy0);
   b.m10 = (1.0f - ox1) * (1.0f - oy0);
   b.m01 = (1.0f - ox0) * (1.0f - oy1);
@@ -749,18 +777,35 @@ __global__ void __launch_bounds__(256) k_tex_bwd(TexBwdArgs A, int total_tiles) 
 // ---------------------------------------------------------------------------
 // Windowed backward for the sampled filters (linear, linear-mipmap-*), C in
 // 1..4.  Per 16x16 pixel tile the texel bounding box of the footprints on
-// the two lowest levels in use is taken, and contributions are summed into
-// dense fp64 LDS windows over those boxes (direct indexing, no hashing; the
-// two windows share one pool).  The windows are written out row by row, so
-// consecutive lanes issue atomics to consecutive addresses.  Big groups of lanes on one footprint (the
-// background texel) go to the per-wave accumulator; taps on other levels,
-// or boxes too large for a window, go to the LDS hash table.
+// each level in use is taken, and contributions are summed into dense fp64
+// LDS windows over those boxes (direct indexing, no hashing; the windows
+// share one pool).  The windows are written out row by row, so consecutive
+// lanes issue atomics to consecutive addresses.  Groups of lanes on one
+// footprint (empty pixels) go to the per-wave accumulator; a box the pool
+// cannot hold goes through it in bands of rows (bilinear), or its taps go to
+// memory a texel row at a time.  Before, such taps went through a small LDS
+// hash table and mostly from there to one device atomic per value (bilinear,
+// 4 x 1000^2 x 3 at 1-3 texels a pixel: 960 us, now 218; at 8 x 1024^2
+// trilinear with 1.3% of them, no change: 237 us).
 // ---------------------------------------------------------------------------
 
 constexpr int kWinWaves = 4;                  // waves per workgroup; a tile is 16 x (4 * kWinWaves) pixels
-constexpr int kWinTexels = 192 * kWinWaves;  // texels of the two windows together
-constexpr int kWinFallback = 32 * kWinWaves;  // LDS hash table entries
 constexpr int kWinThreads = 64 * kWinWaves;
+
+// Texels of a tile's windows together: what five workgroups per CU leave of
+// the LDS at four channels.  The bilinear filter has one slot a pixel and no
+// level to absorb minification, so up to three channels it takes as many as
+// the 10-bit window fields address (4 x 1000^2 x 3 at 1-3 texels a pixel:
+// backward 338 -> 289 us against 768, before the bands).
+template <int FILTER, int CT>
+constexpr int win_texels() {
+  return FILTER == DR_FILTER_LINEAR && CT < 4 ? 1008 : 192 * kWinWaves;
+}
+
+// Most bands of a box larger than the pool (bilinear): 289 -> 218 us at the
+// same sizes; two, four, six or ten allowed differ by the noise (218-226),
+// since a box of more than a few thousand texels holds few taps each.
+constexpr int kWinBands = 4;
 
 struct TapSlot {
   int k;         // level
@@ -780,24 +825,55 @@ __device__ __forceinline__ void slot_box(const TapSlot& q, int& x0, int& x1, int
 }
 
 
+// The wrap mode's window coordinates are the texel coordinates before the
+// wrap (reduced to texels when the window is written out), so a footprint
+// across the texture's border, and a tiled texture's pixels on both sides of
+// a repeat, stay neighbours: with wrapped coordinates their box spans the
+// texture, no window holds it, and the tile's taps all went to the hash
+// table and to device atomics.  Coordinates too far out for the packed
+// 16-bit boxes are taken wrapped, which is the same texel.
+constexpr int kWinCoordMax = 32000;
+__device__ __forceinline__ int win_coord(int t, int wrapped) {
+  return (unsigned)t + kWinCoordMax <= 2u * kWinCoordMax ? t : wrapped;
+}
+// The texel of window coordinate t.
+template <int BND>
+__device__ __forceinline__ int win_texel(int t, int size) {
+  if (BND != DR_BOUNDARY_WRAP) return t;
+  const int r = t % size;
+  return r < 0 ? r + size : r;
+}
+
+// t mod size for t >= 0, mostly below 2 * size.
+__device__ __forceinline__ int wrap_up(int t, int size) {
+  if (t >= size) t -= size;
+  return t < size ? t : t % size;
+}
+
+// Weight `tap` (0..3: 00, 10, 01, 11) of the wave-uniform lane `leader`.
+__device__ __forceinline__ float leader_weight(const TapSlot& q, int leader, int tap) {
+  const int a = __builtin_amdgcn_readlane(__float_as_int(q.w00), leader);
+  const int b = __builtin_amdgcn_readlane(__float_as_int(q.w10), leader);
+  const int c = __builtin_amdgcn_readlane(__float_as_int(q.w01), leader);
+  const int d = __builtin_amdgcn_readlane(__float_as_int(q.w11), leader);
+  return __int_as_float(tap == 0 ? a : tap == 1 ? b : tap == 2 ? c : d);
+}
+
 template <int FILTER, int CT, int BND, bool BIAS>
 // Five waves per SIMD (the register budget this asks for costs a few
 // spilled values; measured cheaper than four or six).
 __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, int total_tiles) {
+  constexpr int kWinTexels = win_texels<FILTER, CT>();
   // channel-major (win[c * kWinTexels + texel]): a wave's run tails on
   // neighbouring texels then add 8 bytes apart, spread over the banks,
   // rather than 8 * CT bytes apart on a few of them
   __shared__ double win[kWinTexels * CT];
   __shared__ __align__(16) int s_lmask[kWinWaves];  // per wave: the levels in use (bit mask)
   __shared__ int2 s_lbox[kWinWaves][kMaxLevels];     // per wave and level: packed box
-  __shared__ int s_tab_used[2];    // per tile parity: the table took entries
-  __shared__ LdsTable<CT, kWinFallback> tab;
   FootAcc<CT> acc;
   acc_init(acc);
   const int tid = threadIdx.x;
   for (int i = tid; i < kWinTexels * CT; i += kWinThreads) win[i] = 0.0;
-  lds_table_clear(tab);
-  if (tid < 2) s_tab_used[tid] = 0;
   __syncthreads();
 
   const MipDesc& md = A.md;
@@ -897,7 +973,12 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
       float w00 = b.w00, w10 = b.w10, w01 = b.w01, w11 = b.w11;
       if (b.ix1 == b.ix0) { w00 += w10; w01 += w11; w10 = 0.0f; w11 = 0.0f; }
       if (b.iy1 == b.iy0) { w00 += w01; w10 += w11; w01 = 0.0f; w11 = 0.0f; }
-      q[li].ix0 = b.ix0; q[li].ix1 = b.ix1; q[li].iy0 = b.iy0; q[li].iy1 = b.iy1;
+      if (BND == DR_BOUNDARY_WRAP) {
+        q[li].ix0 = win_coord(b.tx0, b.ix0); q[li].ix1 = q[li].ix0 + 1;
+        q[li].iy0 = win_coord(b.ty0, b.iy0); q[li].iy1 = q[li].iy0 + 1;
+      } else {
+        q[li].ix0 = b.ix0; q[li].ix1 = b.ix1; q[li].iy0 = b.iy0; q[li].iy1 = b.iy1;
+      }
       const bool on = valid && q[li].scale != 0.0f;
       q[li].w00 = on ? w00 : 0.0f; q[li].w10 = on ? w10 : 0.0f;
       q[li].w01 = on ? w01 : 0.0f; q[li].w11 = on ? w11 : 0.0f;
@@ -969,7 +1050,25 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
       // spanning both, which the windows cannot hold (their taps then went to
       // the hash table: 0.299 -> 0.294 ms at 8 x 1024^2); other footprints,
       // however many lanes share them, take the windows' run sums
-      const bool flat = on0 && q[0].ix0 == q[0].ix1 && q[0].iy0 == q[0].iy1;
+      // Wrap mode: an empty pixel's footprint (uv = 0) is the texture's four
+      // corner texels, so pixels of one uv are grouped instead: those at uv
+      // (0, 0), and any whose left or right neighbour has the same uv (a
+      // background given another constant).  One uv on one level has one set
+      // of weights, so the group's cotangents are summed and then weighted
+      // (4 x 1000^2 x 3, bilinear, 55% of the pixels empty: 960 -> 92 us with
+      // the windows' unwrapped coordinates).
+      bool flat;
+      if (BND == DR_BOUNDARY_WRAP) {
+        const int ux = __float_as_int(uvp.x), uy = __float_as_int(uvp.y);
+        // (every lane executes the shifts)
+        const int lx = dpp_shift<0x111>(ux), ly = dpp_shift<0x111>(uy);
+        const int rx = dpp_shift<0x101>(ux), ry = dpp_shift<0x101>(uy);
+        const bool left = (lane & 15) != 0 && lx == ux && ly == uy;
+        const bool right = (lane & 15) != 15 && rx == ux && ry == uy;
+        flat = on0 && ((uvp.x == 0.0f && uvp.y == 0.0f) || left || right);
+      } else {
+        flat = on0 && q[0].ix0 == q[0].ix1 && q[0].iy0 == q[0].iy1;
+      }
       uint64_t pending = __ballot(flat);
 #pragma unroll 1
       for (int probe = 0; probe < 2 && pending; ++probe) {
@@ -977,17 +1076,24 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
         const uint64_t lkey = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(key >> 32), leader) << 32) |
                               (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)key, leader);
         const uint32_t lkey2 = (uint32_t)__builtin_amdgcn_readlane((int)key2, leader);
-        const bool same = flat && !hot && key == lkey && key2 == lkey2;
+        bool same;
+        if (BND == DR_BOUNDARY_WRAP)
+          same = flat && !hot && q[0].k == __builtin_amdgcn_readlane(q[0].k, leader) &&
+                 __float_as_int(uvp.x) == __builtin_amdgcn_readlane(__float_as_int(uvp.x), leader) &&
+                 __float_as_int(uvp.y) == __builtin_amdgcn_readlane(__float_as_int(uvp.y), leader);
+        else
+          same = flat && !hot && key == lkey && key2 == lkey2;
         const uint64_t members = __ballot(same);
         pending &= ~members;
         const int lk = __builtin_amdgcn_readlane(q[0].k, leader);
         float* base = dlevel_ptr(lk);
         const int lW = mip_w(md, lk);
         float* lp[4];
-        const int lix0 = __builtin_amdgcn_readlane(q[0].ix0, leader);
-        const int lix1 = __builtin_amdgcn_readlane(q[0].ix1, leader);
-        const int liy0 = __builtin_amdgcn_readlane(q[0].iy0, leader);
-        const int liy1 = __builtin_amdgcn_readlane(q[0].iy1, leader);
+        const int lH = mip_h(md, lk);
+        const int lix0 = win_texel<BND>(__builtin_amdgcn_readlane(q[0].ix0, leader), lW);
+        const int lix1 = win_texel<BND>(__builtin_amdgcn_readlane(q[0].ix1, leader), lW);
+        const int liy0 = win_texel<BND>(__builtin_amdgcn_readlane(q[0].iy0, leader), lH);
+        const int liy1 = win_texel<BND>(__builtin_amdgcn_readlane(q[0].iy1, leader), lH);
         lp[0] = base + ((int64_t)liy0 * lW + lix0) * CT;
         lp[1] = base + ((int64_t)liy0 * lW + lix1) * CT;
         lp[2] = base + ((int64_t)liy1 * lW + lix0) * CT;
@@ -1001,14 +1107,22 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
           acc.v = 0.0f;
           acc.on = true;
         }
-        // all the weight is on tap 0 (one texel): four sums, one per channel
+        // all the weight is on tap 0 (one texel; wrap mode: the group has one
+        // set of four weights): four sums, one per channel
         float x[4];
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-          x[c] = (c < CT && same) ? q[0].w00 * (g[c < CT ? c : 0] * q[0].scale) : 0.0f;
+        for (int c = 0; c < 4; ++c) {
+          const float gc = g[c < CT ? c : 0] * q[0].scale;
+          x[c] = (c < CT && same) ? (BND == DR_BOUNDARY_WRAP ? gc : q[0].w00 * gc) : 0.0f;
+        }
         const float z = wave_sum4(x);  // lane l: total of value l & 3
         const float zc = __shfl(z, (lane >> 2) & 3, kWave);
-        if (lane < 4 * CT && (lane & 3) == 0) acc.v += zc;  // lane 4c: channel c, tap 0
+        if (BND == DR_BOUNDARY_WRAP) {  // lane 4c + t: channel c, tap t
+          const float wt = leader_weight(q[0], leader, lane & 3);
+          if (lane < 4 * CT) acc.v += wt * zc;
+        } else {
+          if (lane < 4 * CT && (lane & 3) == 0) acc.v += zc;  // lane 4c: channel c, tap 0
+        }
         if (same) hot = true;
       }
     }
@@ -1017,7 +1131,6 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
     //    cover every level any wave uses ------------------------------------
     const bool use0 = !hot && (q[0].w00 != 0.0f || q[0].w10 != 0.0f || q[0].w01 != 0.0f || q[0].w11 != 0.0f);
     const bool use1 = q[1].w00 != 0.0f || q[1].w10 != 0.0f || q[1].w01 != 0.0f || q[1].w11 != 0.0f;
-    const int par = it & 1;
     {
       const int lm = wave_or((use0 ? 1 << q[0].k : 0) | (use1 ? 1 << q[1].k : 0));
 #pragma unroll 1
@@ -1041,7 +1154,6 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
       if (lane == 0) s_lmask[wave] = lm;
     }
     __syncthreads();
-    if (tid == 0) s_tab_used[par ^ 1] = 0;  // read by every thread before the last barrier
     // Level L's window, in lane L of each 16-lane row: the union of the
     // waves' boxes on L and its place in the pool (levels in ascending
     // order; a box larger than the pool is left out).  A lane then takes
@@ -1081,13 +1193,41 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
       incl += t;
       const bool usable = present && area == fit && incl <= kWinTexels;
       static_assert(kWinTexels < 1024, "window sides and offsets are 10-bit fields");
-      wxy = x0 | (y0 << 16);
+      wxy = pack16(x0, y0);
       wsz = usable ? (x1 - x0 + 1) | ((y1 - y0 + 1) << 10) | ((incl - fit + 1) << 20) : 0;
     }
 
     // -- accumulate: runs of one footprint along a pixel row are summed
     //    first (lanes of one LDS atomic on one address are serialised), the
     //    run's last lane adds the totals ----------------------------------------
+    // Slot li's run totals v (tap-major, 4 * CT values, all zero in a lane
+    // that is not the tail of a run of `u` lanes' footprints); whether this
+    // lane is one.  Every lane executes it.
+    auto run_totals = [&](int li, bool u, float (&v)[4 * CT]) -> bool {
+      const float sc = mip ? q[li].scale : 1.0f;
+      // level and the four texel coordinates (each < 32767 on the window
+      // path) fix the taps; an unused slot gets a key no footprint has
+      const uint64_t key =
+          !u ? (0x7FFFull << 45) | (uint64_t)lane
+          : BND == DR_BOUNDARY_WRAP  // (the second coordinates follow from the first)
+             ? ((uint64_t)q[li].k << 60) | ((uint64_t)(uint16_t)q[li].ix0 << 16) |
+                   (uint16_t)q[li].iy0
+             : ((uint64_t)q[li].k << 60) | ((uint64_t)q[li].ix0 << 45) |
+                   ((uint64_t)q[li].ix1 << 30) | ((uint64_t)q[li].iy0 << 15) |
+                   (uint64_t)q[li].iy1;
+      const RowRun run = row_run(key);
+      const int maxlen = wave_max(run.li - run.s + 1);  // longest run in the wave
+      const float wt[4] = {q[li].w00, q[li].w10, q[li].w01, q[li].w11};
+      float gs[CT];
+#pragma unroll
+      for (int c = 0; c < CT; ++c) gs[c] = !u ? 0.0f : g[c] * sc;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int c = 0; c < CT; ++c) v[t * CT + c] = wt[t] * gs[c];
+      row_run_scan_n(run, v, maxlen);
+      return u && run.tail;
+    };
 #pragma unroll
     for (int li = 0; li < 2; ++li) {
       const bool u = li == 0 ? use0 : use1;
@@ -1096,36 +1236,15 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
       // the window of level k (every lane executes the permutes)
       const int sxy = __builtin_amdgcn_ds_bpermute(k << 2, wxy);
       const int ssz = __builtin_amdgcn_ds_bpermute(k << 2, wsz);
-      const float sc = mip ? q[li].scale : 1.0f;
-      // level and the four texel coordinates (each < 32767 on the window
-      // path) fix the taps; an unused slot gets a key no footprint has
-      const uint64_t key =
-          !u ? (0x7FFFull << 45) | (uint64_t)lane
-             : ((uint64_t)k << 60) | ((uint64_t)q[li].ix0 << 45) | ((uint64_t)q[li].ix1 << 30) |
-                   ((uint64_t)q[li].iy0 << 15) | (uint64_t)q[li].iy1;
-      const RowRun run = row_run(key);
-      const int maxlen = wave_max(run.li - run.s + 1);  // longest run in the wave
-      const bool adds = u && run.tail;
-      const bool in_win = ssz != 0;
-      // the 16 values (tap-major) of the footprint, then one segmented scan
-      // over all of them
-      const float wt[4] = {q[li].w00, q[li].w10, q[li].w01, q[li].w11};
-      float gs[CT];
-#pragma unroll
-      for (int c = 0; c < CT; ++c) gs[c] = !u ? 0.0f : g[c] * sc;
       float v[4 * CT];
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int c = 0; c < CT; ++c) v[t * CT + c] = wt[t] * gs[c];
-      row_run_scan_n(run, v, maxlen);
-      if (adds && in_win) {
+      const bool adds = run_totals(li, u, v);
+      if (adds && ssz != 0) {
         // window indices of the four taps.  The box holds every tap with a
         // nonzero weight in some lane of the run; a tap whose weight is zero
         // in all of them (a texel column or row with zero weight, outside
         // the image for the zero boundary) may lie outside it, and its
         // coordinates are clamped into the box, where it adds 0.
-        const int wx = sxy & 0xffff, wy = sxy >> 16;
+        const int wx = unpack16_lo(sxy), wy = unpack16_hi(sxy);
         const int ww = ssz & 0x3ff, wh = (ssz >> 10) & 0x3ff, sbase = (ssz >> 20) - 1;
         const int cx0 = min(max(q[li].ix0 - wx, 0), ww - 1);
         const int cx1 = min(max(q[li].ix1 - wx, 0), ww - 1);
@@ -1138,34 +1257,21 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
           for (int c = 0; c < CT; ++c)
             atomicAdd(win + c * kWinTexels + o[t], (double)v[t * CT + c]);
       }
-      if (adds && !in_win) {  // boxes that the pool could not hold
-        s_tab_used[par] = 1;
-        float* base = dlevel_ptr(k);
-        const int Wk = mip_w(md, k);
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const int tx_ = (t & 1) ? q[li].ix1 : q[li].ix0;
-          const int ty_ = (t & 2) ? q[li].iy1 : q[li].iy0;
-          lds_table_add(tab, base + ((int64_t)ty_ * Wk + tx_) * CT, &v[t * CT]);
-        }
-      }
     }
     __syncthreads();
 
     // -- write the windows out, row by row -----------------------------------
-#pragma unroll 1
-    for (int rem = lmask; rem != 0; rem &= rem - 1) {  // uniform
-      const int k = __builtin_ctz(rem);
-      const int sz = __builtin_amdgcn_readlane(wsz, k);
-      if (sz == 0) continue;
-      const int xy = __builtin_amdgcn_readlane(wxy, k);
-      const int bx0 = xy & 0xffff, by0 = xy >> 16, bw = sz & 0x3ff, bh = (sz >> 10) & 0x3ff;
-      const int base_k = (sz >> 20) - 1;
+    // Level k's window of bw x bh texels from window coordinates (x0, y0),
+    // at `at` in the pool, added to the level and cleared.
+    auto flush_window = [&](int k, int x0, int y0, int bw, int bh, int at) {
       float* base = dlevel_ptr(k);
-      const int Wk = mip_w(md, k);
+      const int Wk = mip_w(md, k), Hk = mip_h(md, k);
+      // (wrap mode: the first texel reduced into the texture; a window's
+      // later columns and rows wrap from there)
+      const int bx0 = win_texel<BND>(x0, Wk), by0 = win_texel<BND>(y0, Hk);
       const int row = bw * CT;
       const int total = row * bh;
-      double* wb = win + base_k;
+      double* wb = win + at;
       // consecutive lanes take consecutive channels of a texel, so the
       // device atomics of a row share cache lines; (r, cpos) of element i
       // advance by a uniform step instead of a division per element
@@ -1176,7 +1282,12 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
         double* e = wb + c * kWinTexels + r * bw + tx;
         const double v = *e;
         if (v != 0.0) {
-          unsafeAtomicAdd(base + ((int64_t)(by0 + r) * Wk + bx0) * CT + cpos, (float)v);
+          if (BND == DR_BOUNDARY_WRAP) {
+            const int X = wrap_up(bx0 + tx, Wk), Y = wrap_up(by0 + r, Hk);
+            unsafeAtomicAdd(base + ((int64_t)Y * Wk + X) * CT + c, (float)v);
+          } else {
+            unsafeAtomicAdd(base + ((int64_t)(by0 + r) * Wk + bx0) * CT + cpos, (float)v);
+          }
           *e = 0.0;
         }
         r += dr;
@@ -1186,8 +1297,116 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
           ++r;
         }
       }
+    };
+    int nowin = 0;  // levels without a window (uniform)
+#pragma unroll 1
+    for (int rem = lmask; rem != 0; rem &= rem - 1) {  // uniform
+      const int k = __builtin_ctz(rem);
+      const int sz = __builtin_amdgcn_readlane(wsz, k);
+      if (sz == 0) {
+        nowin |= 1 << k;
+        continue;
+      }
+      const int xy = __builtin_amdgcn_readlane(wxy, k);
+      flush_window(k, unpack16_lo(xy), unpack16_hi(xy), sz & 0x3ff, (sz >> 10) & 0x3ff,
+                   (sz >> 20) - 1);
     }
-    if (s_tab_used[par]) lds_table_flush(tab);  // uniform; contains a barrier
+    // -- bilinear: a box larger than the pool (a texture minified by up to a
+    //    few texels a pixel) goes through it in bands of whole rows: a band's
+    //    rows share cache-line requests, where the direct way below costs two
+    //    requests a pixel whatever the box
+    if (!mip && nowin != 0) {  // uniform: level 0 alone is in use
+      int px = pack16(32767, 32767), py = px;
+#pragma unroll
+      for (int w = 0; w < kWinWaves; ++w) {
+        const int mw = w == 0 ? wm.x : w == 1 ? wm.y : w == 2 ? wm.z : wm.w;
+        if (mw & 1) {
+          px = pk16_min(px, s_lbox[w][0].x);
+          py = pk16_min(py, s_lbox[w][0].y);
+        }
+      }
+      px = __builtin_amdgcn_readfirstlane(px);
+      py = __builtin_amdgcn_readfirstlane(py);
+      const int x0 = unpack16_lo(px), y0 = unpack16_lo(py);
+      const int bw = -unpack16_hi(px) - x0 + 1, bh = -unpack16_hi(py) - y0 + 1;
+      const int rows = bw <= kWinTexels ? kWinTexels / bw : 0;
+      if (rows * kWinBands >= bh) {  // (rows 0: too wide)
+        float v[4 * CT];
+        const bool adds = run_totals(0, use0, v);
+        const int cx0 = min(max(q[0].ix0 - x0, 0), bw - 1);
+        const int cx1 = min(max(q[0].ix1 - x0, 0), bw - 1);
+        // (a zero-weight row outside the box is clamped into it: adds 0)
+        const int cy0 = min(max(q[0].iy0 - y0, 0), bh - 1);
+        const int cy1 = min(max(q[0].iy1 - y0, 0), bh - 1);
+#pragma unroll 1
+        for (int b0 = 0; b0 < bh; b0 += rows) {
+          const int nr = min(rows, bh - b0);
+          __syncthreads();  // the pool is written out (and cleared)
+#pragma unroll
+          for (int row = 0; row < 2; ++row) {
+            const int r = (row == 0 ? cy0 : cy1) - b0;
+            if (adds && (unsigned)r < (unsigned)nr) {
+#pragma unroll
+              for (int c = 0; c < CT; ++c) {
+                atomicAdd(win + c * kWinTexels + r * bw + cx0, (double)v[row * 2 * CT + c]);
+                atomicAdd(win + c * kWinTexels + r * bw + cx1, (double)v[row * 2 * CT + CT + c]);
+              }
+            }
+          }
+          __syncthreads();
+          flush_window(0, x0, y0 + b0, bw, nr, 0);
+        }
+        nowin = 0;
+      }
+    }
+    // -- levels without a window: each run's two texel rows straight to
+    //    memory.  A wave lays a row's 2 * CT totals of its 64 lanes out in
+    //    its part of the pool and issues them with consecutive lanes on
+    //    consecutive addresses (one cache-line request a row instead of one a
+    //    value: the atomic units take requests, about 21 G/s), so a minified
+    //    texture without mip levels costs two requests a pixel
+    if (nowin != 0) {
+      __syncthreads();  // the windows are written out: the pool is free and zero
+      double* st = win + wave * (kWinTexels * CT / kWinWaves);
+      static_assert(kWinTexels / kWinWaves >= 2 * 64, "a wave's row of totals fits its part");
+#pragma unroll 1
+      for (int rem = nowin; rem != 0; rem &= rem - 1) {  // uniform
+        const int k = __builtin_ctz(rem);
+        float* base = dlevel_ptr(k);
+        const int Wk = mip_w(md, k), Hk = mip_h(md, k);
+#pragma unroll
+        for (int li = 0; li < (mip ? 2 : 1); ++li) {
+          const bool u = (li == 0 ? use0 : use1) && q[li].k == k;
+          if (__ballot(u) == 0) continue;
+          float v[4 * CT];
+          const bool adds = run_totals(li, u, v);
+          const int X0 = win_texel<BND>(q[li].ix0, Wk), X1 = win_texel<BND>(q[li].ix1, Wk);
+#pragma unroll
+          for (int row = 0; row < 2; ++row) {
+            const int Y = win_texel<BND>(row == 0 ? q[li].iy0 : q[li].iy1, Hk);
+            const uint32_t off = ((uint32_t)Y * (uint32_t)Wk + (uint32_t)X0) * CT;
+#pragma unroll
+            for (int j = 0; j < 2 * CT; ++j)
+              st[lane * 2 * CT + j] = adds ? (double)v[row * 2 * CT + j] : 0.0;
+            __builtin_amdgcn_wave_barrier();  // (LDS is ordered within a wave)
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+#pragma unroll 1
+            for (int i = 0; i < 2 * CT; ++i) {
+              const int e = (i * 64 + lane) / (2 * CT), j = (i * 64 + lane) - e * 2 * CT;
+              const uint32_t eo = (uint32_t)__builtin_amdgcn_ds_bpermute(e << 2, (int)off);
+              const int ed = __builtin_amdgcn_ds_bpermute(e << 2, X1 - X0);
+              const float x = (float)st[i * 64 + lane];
+              if (x != 0.0f)
+                unsafeAtomicAdd(base + eo + (j < CT ? j : ed * CT + j - CT), x);
+            }
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+          }
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < 2 * CT; ++j) st[lane * 2 * CT + j] = 0.0;  // before the next barrier
+    }
   }
   acc_flush(acc);
 }

@@ -1,0 +1,79 @@
+"""texture's backward paths on smooth uv fields (what a rendered surface
+gives), against the CPU oracle, at the sizes where a path changes: wrap
+windows across the texture's border and repeats; boxes that fill the LDS
+pool, take it in bands, or are written to memory directly."""
+import numpy as np
+import pytest
+
+import oracle as O
+from parity import assert_fwd_close, assert_grad_close, dev, host, torch_dev
+
+pytestmark = pytest.mark.gpu
+
+
+def smooth_uv(rng, N, Hi, Wi, scale, offset, background):
+    """An affine field over `scale` repeats from `offset`, its derivatives,
+    and a patch and single pixels of one constant uv (empty pixels)."""
+    y, x = np.meshgrid((np.arange(Hi) + 0.5) / Hi, (np.arange(Wi) + 0.5) / Wi, indexing="ij")
+    M = rng.normal(size=(N, 2, 2)) * scale
+    uv = np.stack([np.stack([M[n, 0, 0] * x + M[n, 0, 1] * y, M[n, 1, 0] * x + M[n, 1, 1] * y], -1)
+                   for n in range(N)]) + offset
+    da = np.stack([np.broadcast_to([M[n, 0, 0] / Wi, M[n, 0, 1] / Hi, M[n, 1, 0] / Wi,
+                                    M[n, 1, 1] / Hi], (Hi, Wi, 4)) for n in range(N)]).copy()
+    empty = np.zeros((N, Hi, Wi), bool)
+    empty[:, : Hi // 2, : Wi // 3] = True
+    empty[:, ::7, ::5] = True
+    uv[empty], da[empty] = background, 0.0
+    return uv.astype(np.float32), da.astype(np.float32)
+
+
+def check(rng, tex, uv, da, filt, bnd, rtol=1e-4):
+    from diffrast import DiffRast
+    mip = "mipmap" in filt
+    t, u = dev(tex).requires_grad_(True), dev(uv).requires_grad_(True)
+    d = dev(da).requires_grad_(True) if mip else None
+    kw = dict(filterMode=filt, boundaryMode=bnd)
+    out = DiffRast.texture(t, u, uvDA=d, **kw)
+    ref = O.texture(tex, uv, uvDA=da if mip else None, **kw)
+    assert_fwd_close(host(out), ref)
+    g = rng.normal(size=ref.shape).astype(np.float32)
+    out.backward(dev(g))
+    d_tex, d_uv, d_da, _ = O.texture_vjp(tex, uv, g, uvDA=da if mip else None, **kw)
+    assert_grad_close(host(t.grad), d_tex, "d_tex", rtol=rtol)
+    assert_grad_close(host(u.grad), d_uv, "d_uv", rtol=rtol)
+    if mip:
+        assert_grad_close(host(d.grad), d_da, "d_uvDA", rtol=rtol)
+
+
+# texture sizes of one texel a side, odd ones, one smaller and one larger
+# than a tile's footprint; offsets beyond the packed window coordinates
+# (taken wrapped) and around zero; the background at uv (0, 0) (four corner
+# texels in wrap mode) and at another constant
+@pytest.mark.parametrize("Ht,Wt", [(1, 1), (1, 7), (5, 3), (40, 72), (512, 256)])
+@pytest.mark.parametrize("offset,background", [(0.0, (0.0, 0.0)), (-3.5, (0.3, 0.7)),
+                                               (40000.0, (0.0, 0.0))])
+@pytest.mark.parametrize("filt,C", [("linear", 1), ("linear", 3), ("linear-mipmap-linear", 4)])
+def test_wrap_windows(Ht, Wt, offset, background, filt, C):
+    torch_dev()
+    rng = np.random.default_rng(Ht * 1000 + Wt + C)
+    uv, da = smooth_uv(rng, 2, 35, 53, 1.5, offset, background)
+    tex = rng.random((1, Ht, Wt, C)).astype(np.float32)
+    check(rng, tex, uv, da, filt, "wrap")
+
+
+# texels a pixel: a tile's box of 16 x 16 pixels grows from one window (0.5)
+# over several bands (2 to 4) to the direct way (12); C = 4 has a smaller pool
+@pytest.mark.parametrize("texels", [0.5, 2.0, 3.0, 4.0, 12.0])
+@pytest.mark.parametrize("bnd", ["wrap", "clamp", "zero"])
+@pytest.mark.parametrize("filt,C", [("linear", 1), ("linear", 3), ("linear", 4),
+                                    ("linear-mipmap-linear", 2)])
+def test_minified_boxes(texels, bnd, filt, C):
+    torch_dev()
+    rng = np.random.default_rng(int(texels * 10) + C)
+    Hi, Wi, Ht, Wt = 49, 60, 256, 320
+    scale = texels * Wi / Wt / 1.5
+    uv, da = smooth_uv(rng, 2, Hi, Wi, scale, 0.4, (0.0, 0.0))
+    if "mipmap" in filt:  # the LOD of a magnified surface: level 0 at any footprint spread
+        da *= 1e-3
+    tex = rng.random((1, Ht, Wt, C)).astype(np.float32)
+    check(rng, tex, uv, da, filt, bnd)
