@@ -395,6 +395,42 @@ __device__ __forceinline__ void acc_flush(FootAcc<CT>& a) {
   a.on = false;
 }
 
+// The accumulators of a workgroup's W waves at its end (every thread calls
+// it): those of one footprint are added up in fp64 and written once.  The
+// empty pixels' footprint collects one addition per value from every
+// workgroup of the persistent grid, and the atomics on one address are
+// serialised (about 80 M/s) just as the workgroups end: one per workgroup
+// instead of one per wave (bilinear, 4 x 1000^2 x 3: 215 -> 193 us; 8 x 1024^2
+// trilinear, whose waves end further apart: no change).
+template <int CT, int W>
+struct FootAccLds {
+  uint64_t p[W][4];
+  float v[W][4 * CT];
+};
+
+template <int CT, int W>
+__device__ __forceinline__ void acc_flush_group(const FootAcc<CT>& a, FootAccLds<CT, W>& s) {
+  const int wave = (int)threadIdx.x >> 6, l = lane_id();
+  if (l < 4) {
+    float* q = l == 0 ? a.p[0] : l == 1 ? a.p[1] : l == 2 ? a.p[2] : a.p[3];
+    s.p[wave][l] = a.on ? (uint64_t)q : 0ull;
+  }
+  if (l < 4 * CT) s.v[wave][l] = a.on ? a.v : 0.0f;
+  __syncthreads();
+  if (!a.on) return;
+  auto same = [&](int w) {
+    return s.p[w][0] == s.p[wave][0] && s.p[w][1] == s.p[wave][1] &&
+           s.p[w][2] == s.p[wave][2] && s.p[w][3] == s.p[wave][3];
+  };
+  for (int w = 0; w < wave; ++w)
+    if (same(w)) return;  // an earlier wave writes this footprint
+  if (l >= 4 * CT) return;
+  double sum = 0.0;
+  for (int w = wave; w < W; ++w)
+    if (same(w)) sum += (double)s.v[w][l];
+  if (sum != 0.0) unsafeAtomicAdd((float*)s.p[wave][l & 3] + (l >> 2), (float)sum);
+}
+
 // Adds the wave sums of val[0..M) (M <= 16) to the accumulator.
 template <int CT, int M>
 __device__ __forceinline__ void acc_add(FootAcc<CT>& a, const float (&val)[M], bool member) {
@@ -761,6 +797,7 @@ __device__ __forceinline__ void tex_bwd_tile(const TexBwdArgs& A, int bidx,
 template <int FILTER, bool CUBE, int CT>
 __global__ void __launch_bounds__(256) k_tex_bwd(TexBwdArgs A, int total_tiles) {
   __shared__ TexTable<CT> tab;
+  __shared__ FootAccLds<(CT > 0 ? CT : 1), 4> s_acc;
   FootAcc<(CT > 0 ? CT : 1)> acc0;
   acc_init(acc0);
   lds_table_clear(tab);
@@ -771,7 +808,7 @@ __global__ void __launch_bounds__(256) k_tex_bwd(TexBwdArgs A, int total_tiles) 
     lds_table_flush(tab);
     __syncthreads();
   }
-  acc_flush(acc0);
+  acc_flush_group(acc0, s_acc);
 }
 
 // ---------------------------------------------------------------------------
@@ -785,27 +822,34 @@ __global__ void __launch_bounds__(256) k_tex_bwd(TexBwdArgs A, int total_tiles) 
 // cannot hold goes through it in bands of rows (bilinear), or its taps go to
 // memory a texel row at a time.  Before, such taps went through a small LDS
 // hash table and mostly from there to one device atomic per value (bilinear,
-// 4 x 1000^2 x 3 at 1-3 texels a pixel: 960 us, now 218; at 8 x 1024^2
-// trilinear with 1.3% of them, no change: 237 us).
+// 4 x 1000^2 x 3 at 1-3 texels a pixel: 960 us, now 189; at 8 x 1024^2
+// trilinear with 1.3% of them, no change: 238 us).
 // ---------------------------------------------------------------------------
 
 constexpr int kWinWaves = 4;                  // waves per workgroup; a tile is 16 x (4 * kWinWaves) pixels
 constexpr int kWinThreads = 64 * kWinWaves;
 
 // Texels of a tile's windows together: what five workgroups per CU leave of
-// the LDS at four channels.  The bilinear filter has one slot a pixel and no
+// the LDS at four channels (8 x 1024^2, trilinear: 237.8 us with 928, 239.7
+// with 768, 313.8 with 992, where only four fit).  The bilinear filter has one slot a pixel and no
 // level to absorb minification, so up to three channels it takes as many as
 // the 10-bit window fields address (4 x 1000^2 x 3 at 1-3 texels a pixel:
 // backward 338 -> 289 us against 768, before the bands).
 template <int FILTER, int CT>
 constexpr int win_texels() {
-  return FILTER == DR_FILTER_LINEAR && CT < 4 ? 1008 : 192 * kWinWaves;
+  return FILTER == DR_FILTER_LINEAR && CT < 4 ? 1008 : 232 * kWinWaves;
 }
 
 // Most bands of a box larger than the pool (bilinear): 289 -> 218 us at the
 // same sizes; two, four, six or ten allowed differ by the noise (218-226),
 // since a box of more than a few thousand texels holds few taps each.
 constexpr int kWinBands = 4;
+
+// Runs of a wave up to which the direct way adds lane by lane (1 x 512^2,
+// trilinear, one tile a workgroup: 21 us for the kernel, 34 with the hash
+// table; the bilinear case above takes the staged way: 189 us, 349 lane by
+// lane).
+constexpr int kWinFewRuns = 12;
 
 struct TapSlot {
   int k;         // level
@@ -870,6 +914,7 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
   __shared__ double win[kWinTexels * CT];
   __shared__ __align__(16) int s_lmask[kWinWaves];  // per wave: the levels in use (bit mask)
   __shared__ int2 s_lbox[kWinWaves][kMaxLevels];     // per wave and level: packed box
+  __shared__ FootAccLds<CT, kWinWaves> s_acc;
   FootAcc<CT> acc;
   acc_init(acc);
   const int tid = threadIdx.x;
@@ -1364,51 +1409,69 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
     //    its part of the pool and issues them with consecutive lanes on
     //    consecutive addresses (one cache-line request a row instead of one a
     //    value: the atomic units take requests, about 21 G/s), so a minified
-    //    texture without mip levels costs two requests a pixel
+    //    texture without mip levels costs two requests a pixel.  A few runs
+    //    (a mixed tile's) are added lane by lane: fewer instructions.
     if (nowin != 0) {
       __syncthreads();  // the windows are written out: the pool is free and zero
       double* st = win + wave * (kWinTexels * CT / kWinWaves);
       static_assert(kWinTexels / kWinWaves >= 2 * 64, "a wave's row of totals fits its part");
-#pragma unroll 1
-      for (int rem = nowin; rem != 0; rem &= rem - 1) {  // uniform
-        const int k = __builtin_ctz(rem);
-        float* base = dlevel_ptr(k);
+      bool staged = false;
+#pragma unroll
+      for (int li = 0; li < (mip ? 2 : 1); ++li) {
+        const int k = q[li].k;
+        const bool u = (li == 0 ? use0 : use1) && ((nowin >> k) & 1);
+        if (__ballot(u) == 0) continue;
+        float v[4 * CT];
+        const bool adds = run_totals(li, u, v);
         const int Wk = mip_w(md, k), Hk = mip_h(md, k);
+        const int X0 = win_texel<BND>(q[li].ix0, Wk), X1 = win_texel<BND>(q[li].ix1, Wk);
+        const int Y0 = win_texel<BND>(q[li].iy0, Hk), Y1 = win_texel<BND>(q[li].iy1, Hk);
+        float* const lv = dlevel_ptr(k);
+        const uint32_t o0 = ((uint32_t)Y0 * (uint32_t)Wk + (uint32_t)X0) * CT;
+        const uint32_t o1 = ((uint32_t)Y1 * (uint32_t)Wk + (uint32_t)X0) * CT;
+        const int dx = (X1 - X0) * CT;
+        if (__popcll(__ballot(adds)) <= kWinFewRuns) {
+          if (adds) {
 #pragma unroll
-        for (int li = 0; li < (mip ? 2 : 1); ++li) {
-          const bool u = (li == 0 ? use0 : use1) && q[li].k == k;
-          if (__ballot(u) == 0) continue;
-          float v[4 * CT];
-          const bool adds = run_totals(li, u, v);
-          const int X0 = win_texel<BND>(q[li].ix0, Wk), X1 = win_texel<BND>(q[li].ix1, Wk);
+            for (int t = 0; t < 4; ++t)
 #pragma unroll
-          for (int row = 0; row < 2; ++row) {
-            const int Y = win_texel<BND>(row == 0 ? q[li].iy0 : q[li].iy1, Hk);
-            const uint32_t off = ((uint32_t)Y * (uint32_t)Wk + (uint32_t)X0) * CT;
-#pragma unroll
-            for (int j = 0; j < 2 * CT; ++j)
-              st[lane * 2 * CT + j] = adds ? (double)v[row * 2 * CT + j] : 0.0;
-            __builtin_amdgcn_wave_barrier();  // (LDS is ordered within a wave)
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-#pragma unroll 1
-            for (int i = 0; i < 2 * CT; ++i) {
-              const int e = (i * 64 + lane) / (2 * CT), j = (i * 64 + lane) - e * 2 * CT;
-              const uint32_t eo = (uint32_t)__builtin_amdgcn_ds_bpermute(e << 2, (int)off);
-              const int ed = __builtin_amdgcn_ds_bpermute(e << 2, X1 - X0);
-              const float x = (float)st[i * 64 + lane];
-              if (x != 0.0f)
-                unsafeAtomicAdd(base + eo + (j < CT ? j : ed * CT + j - CT), x);
-            }
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+              for (int c = 0; c < CT; ++c) {
+                const float x = v[t * CT + c];
+                if (x != 0.0f) unsafeAtomicAdd(lv + ((t & 2) ? o1 : o0) + ((t & 1) ? dx : 0) + c, x);
+              }
           }
+          continue;
+        }
+        staged = true;
+#pragma unroll
+        for (int row = 0; row < 2; ++row) {
+          const uint64_t p = (uint64_t)(lv + (row == 0 ? o0 : o1));
+#pragma unroll
+          for (int j = 0; j < 2 * CT; ++j)
+            st[lane * 2 * CT + j] = adds ? (double)v[row * 2 * CT + j] : 0.0;
+          __builtin_amdgcn_wave_barrier();  // (LDS is ordered within a wave)
+          __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+#pragma unroll 1
+          for (int i = 0; i < 2 * CT; ++i) {
+            const int e = (i * 64 + lane) / (2 * CT), j = (i * 64 + lane) - e * 2 * CT;
+            const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute(e << 2, (int)(uint32_t)p);
+            const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_bpermute(e << 2, (int)(p >> 32));
+            const int ed = __builtin_amdgcn_ds_bpermute(e << 2, dx);
+            const float x = (float)st[i * 64 + lane];
+            if (x != 0.0f)
+              unsafeAtomicAdd((float*)(((uint64_t)hi << 32) | lo) + (j < CT ? j : ed + j - CT), x);
+          }
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         }
       }
+      if (staged) {  // zero again before the next barrier
 #pragma unroll
-      for (int j = 0; j < 2 * CT; ++j) st[lane * 2 * CT + j] = 0.0;  // before the next barrier
+        for (int j = 0; j < 2 * CT; ++j) st[lane * 2 * CT + j] = 0.0;
+      }
     }
   }
-  acc_flush(acc);
+  acc_flush_group(acc, s_acc);
 }
 
 // Texture.swift:156: level k = 2x2 mean of level k-1.
@@ -2043,6 +2106,7 @@ template <int MODE, int CT>
 __global__ void __launch_bounds__(256) k_cube_bwd(CubeArgs A, int Hi, int Wi, int ntx,
                                                   int total_tiles) {
   __shared__ CubeTable<CT> tab;
+  __shared__ FootAccLds<(CT > 0 ? CT : 1), 4> s_acc;
   FootAcc<(CT > 0 ? CT : 1)> acc0;
   acc_init(acc0);
   lds_table_clear(tab);
@@ -2059,7 +2123,7 @@ __global__ void __launch_bounds__(256) k_cube_bwd(CubeArgs A, int Hi, int Wi, in
     lds_table_flush(tab);
     __syncthreads();
   }
-  acc_flush(acc0);
+  acc_flush_group(acc0, s_acc);
 }
 
 }  // namespace dr
