@@ -1474,56 +1474,668 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
   acc_flush_group(acc, s_acc);
 }
 
-// Texture.swift:156: level k = 2x2 mean of level k-1.
-__global__ void __launch_bounds__(256) k_mip_down(const float* __restrict__ src,
-                                                  float* __restrict__ dst, int Nt, int h, int w,
-                                                  int C) {
-  const int h2 = h / 2, w2 = w / 2;
-  const int64_t total = (int64_t)Nt * h2 * w2 * C;
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= total) return;
-  const int c = (int)(i % C);
-  int64_t r = i / C;
-  const int x = (int)(r % w2);
-  r /= w2;
-  const int y = (int)(r % h2);
-  const int n = (int)(r / h2);
-  const float* s = src + (int64_t)n * h * w * C;
-  const float a = s[((int64_t)(2 * y) * w + 2 * x) * C + c];
-  const float b = s[((int64_t)(2 * y) * w + 2 * x + 1) * C + c];
-  const float d = s[((int64_t)(2 * y + 1) * w + 2 * x) * C + c];
-  const float e = s[((int64_t)(2 * y + 1) * w + 2 * x + 1) * C + c];
-  dst[i] = (((a + b) + d) + e) * 0.25f;
+// ---------------------------------------------------------------------------
+// More than four channels (feature textures).  The forward gives a thread
+// four channels of a pixel, consecutive threads consecutive channels, so
+// texel reads and output writes are whole cache lines; one thread per pixel
+// walking its channels read four bytes a lane at a stride of C floats
+// (2 x 768^2 x 16, trilinear: 286 -> 40 us).
+// ---------------------------------------------------------------------------
+
+// Four channels from p, the first nc of them in memory (nc = 4: one load
+// whatever p's alignment; the hardware takes 4-byte aligned vectors).
+typedef float dr_f4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ float4 ld_chunk(const float* __restrict__ p, int nc) {
+  if (nc == 4) {
+    const dr_f4u v = *reinterpret_cast<const dr_f4u*>(p);
+    return make_float4(v.x, v.y, v.z, v.w);
+  }
+  return make_float4(p[0], nc > 1 ? p[1] : 0.0f, nc > 2 ? p[2] : 0.0f, 0.0f);
+}
+__device__ __forceinline__ void st_chunk(float* __restrict__ p, float4 x, int nc) {
+  if (nc == 4) {
+    dr_f4u v = {x.x, x.y, x.z, x.w};
+    *reinterpret_cast<dr_f4u*>(p) = v;
+    return;
+  }
+  p[0] = x.x;
+  if (nc > 1) p[1] = x.y;
+  if (nc > 2) p[2] = x.z;
 }
 
-// Builds up to five levels at once: each workgroup reduces a 2^m x 2^m
-// block of level s through levels s+1..s+m in LDS (m <= 5; the sizes of
-// levels s..s+m-1 are even, so the blocks tile level s exactly).  Same 2x2
-// sums as k_mip_down, in the same order.
+// The bilinear sample of channels [c, c + nc) of one level, in tex_fwd_px's
+// operation order.
+__device__ __forceinline__ float4 sample_chunk(const float* __restrict__ lv, int Wk, int C,
+                                               const Bilin& b, int c, int nc) {
+  const int64_t r0 = (int64_t)b.iy0 * Wk, r1 = (int64_t)b.iy1 * Wk;
+  const float4 a = ld_chunk(lv + (r0 + b.ix0) * C + c, nc), d = ld_chunk(lv + (r0 + b.ix1) * C + c, nc);
+  const float4 e = ld_chunk(lv + (r1 + b.ix0) * C + c, nc), f = ld_chunk(lv + (r1 + b.ix1) * C + c, nc);
+  return make_float4(b.w00 * a.x + b.w10 * d.x + b.w01 * e.x + b.w11 * f.x,
+                     b.w00 * a.y + b.w10 * d.y + b.w01 * e.y + b.w11 * f.y,
+                     b.w00 * a.z + b.w10 * d.z + b.w01 * e.z + b.w11 * f.z,
+                     b.w00 * a.w + b.w10 * d.w + b.w01 * e.w + b.w11 * f.w);
+}
+
+template <int FILTER, int BND>
+__global__ void __launch_bounds__(256) k_tex_fwd_many(
+    const float* __restrict__ tex, const float* __restrict__ pyr, MipDesc md, int64_t tex_stride,
+    int Ht, int Wt, int C, const float* __restrict__ uv, const float* __restrict__ uv_da,
+    const float* __restrict__ bias_map, float scale_bias, int has_bias, int64_t, int Hi, int Wi,
+    float* __restrict__ out) {
+  const int ntx = (Wi + 15) >> 4, tiles = ntx * ((Hi + 15) >> 4);
+  const int b = (int)blockIdx.x, n = b / tiles, tile = b - n * tiles;
+  const int ty = tile / ntx, tx = tile - ty * ntx;
+  const int G = (C + 3) >> 2;  // chunks of four channels
+  const bool shared = tex_stride == 0;
+  for (int i = (int)threadIdx.x; i < 256 * G; i += 256) {
+    const int lp = i / G, c = (i - lp * G) * 4;  // tile pixel, first channel
+    const int ph = ty * 16 + (lp >> 4), pw = tx * 16 + (lp & 15);
+    if (ph >= Hi || pw >= Wi) continue;
+    const int64_t pix = ((int64_t)n * Hi + ph) * Wi + pw;
+    const int nc = min(4, C - c);
+    float4 o;
+    if (BND == DR_BOUNDARY_CUBE) {
+      Bilin bl;
+      const int face = cube_bilin(uv[pix * 3 + 0], uv[pix * 3 + 1], uv[pix * 3 + 2], Wt, Ht, bl);
+      o = sample_chunk(tex + n * tex_stride + (int64_t)face * Ht * Wt * C, Wt, C, bl, c, nc);
+    } else {
+      const float2 uvp = *reinterpret_cast<const float2*>(uv + pix * 2);
+      if (FILTER == DR_FILTER_NEAREST) {
+        float ox, oy;
+        const int ix = apply_boundary(f2i(floorf(uvp.x * (float)Wt)), Wt, BND, ox);
+        const int iy = apply_boundary(f2i(floorf(uvp.y * (float)Ht)), Ht, BND, oy);
+        const float mask = (1.0f - ox) * (1.0f - oy);
+        o = ld_chunk(tex + n * tex_stride + ((int64_t)iy * Wt + ix) * C + c, nc);
+        o = make_float4(o.x * mask, o.y * mask, o.z * mask, o.w * mask);
+      } else if (FILTER == DR_FILTER_LINEAR) {
+        o = sample_chunk(tex + n * tex_stride, Wt, C, bilin(uvp.x, uvp.y, Wt, Ht, BND), c, nc);
+      } else {
+        float4 da = *reinterpret_cast<const float4*>(uv_da + pix * 4);
+        const float s = bias_scale(bias_map, pix, scale_bias, has_bias != 0);
+        if (bias_map || has_bias) da = make_float4(da.x * s, da.y * s, da.z * s, da.w * s);
+        const Lod ld = mip_lod(da, Ht, Wt, md.L, FILTER == DR_FILTER_LINEAR_MIPMAP_LINEAR);
+        auto level = [&](int k) {
+          const int Hk = mip_h(md, k), Wk = mip_w(md, k);
+          const float* lv = k == 0 ? tex + n * tex_stride
+                                   : pyr + mip_off(md, k) + (shared ? 0 : (int64_t)n * Hk * Wk * C);
+          return sample_chunk(lv, Wk, C, bilin(uvp.x, uvp.y, Wk, Hk, BND), c, nc);
+        };
+        const float w0 = 1.0f - ld.frac, w1 = ld.frac;
+        o = level(ld.k0);
+        o = make_float4(w0 * o.x, w0 * o.y, w0 * o.z, w0 * o.w);
+        if (w1 != 0.0f) {  // (a zero-weight level is not read)
+          const float4 p = level(ld.k1);
+          o = make_float4(o.x + w1 * p.x, o.y + w1 * p.y, o.z + w1 * p.z, o.w + w1 * p.w);
+        }
+      }
+    }
+    st_chunk(out + pix * C + c, o, nc);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Windowed backward for more than four channels: k_tex_bwd_win's boxes and
+// pool, with the channels taken four at a time and as many of them in the
+// pool at once as the tile's boxes leave room for, so a window's flush writes
+// a texel's channels as one run of memory.  One footprint set-up serves all
+// channels, and d_uv and the LOD's gradient sum over them in registers.  The
+// general kernel's wave probes and one device atomic per tap and channel
+// took 3,453 us at 2 x 768^2 x 16, trilinear; this takes 180 (188 with the
+// direct way's cotangents loaded one pixel at a time; 264 at four waves per
+// SIMD, which spills 46 registers; 211 with two and a pool twice the size).
+// Cube maps: k is the face, one level each.
+// ---------------------------------------------------------------------------
+
+constexpr int kManyPool = 4096;  // doubles: 32 KiB (3072: 197 us, 5632: 204)
+constexpr int kManyC = 128;      // channels the empty pixels' sums have room for
+
+// The sum of an empty-pixel group (one uv, so one footprint and one set of
+// weights), kept in LDS per wave and channel until another footprint takes
+// its place (wave-uniform).
+struct ManyHot {
+  bool on;
+  int ux, uy;           // the uv's bits
+  float* base;          // the level
+  int ix0, ix1, iy0, iy1, Wk;
+  float w00, w10, w01, w11;
+};
+
+__device__ __forceinline__ void hot_flush(const ManyHot& h, int C, const double* s) {
+  for (int i = lane_id(); i < 4 * C; i += 64) {
+    const int t = i / C, c = i - t * C;
+    const float w = t == 0 ? h.w00 : t == 1 ? h.w10 : t == 2 ? h.w01 : h.w11;
+    const float v = (float)((double)w * s[c]);
+    if (v != 0.0f)
+      unsafeAtomicAdd(h.base + ((int64_t)((t & 2) ? h.iy1 : h.iy0) * h.Wk +
+                                ((t & 1) ? h.ix1 : h.ix0)) * C + c, v);
+  }
+}
+
+template <int FILTER, int BND>
+__global__ void __launch_bounds__(256, 3) k_tex_bwd_many(TexBwdArgs A, int total_tiles) {
+  __shared__ double win[kManyPool];  // channel-major: win[c * texels + texel]
+  __shared__ double s_hot[4][kManyC];
+  __shared__ __align__(16) int s_lmask[4];
+  __shared__ int2 s_lbox[4][kMaxLevels];
+  __shared__ uint64_t s_hbase[4];
+  __shared__ int2 s_hkey[4];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  for (int i = tid; i < kManyPool; i += 256) win[i] = 0.0;
+  for (int i = tid; i < 4 * kManyC; i += 256) (&s_hot[0][0])[i] = 0.0;
+  __syncthreads();
+  constexpr bool kCube = BND == DR_BOUNDARY_CUBE;
+  constexpr bool mip = FILTER == DR_FILTER_LINEAR_MIPMAP_LINEAR || FILTER == DR_FILTER_LINEAR_MIPMAP_NEAREST;
+  const MipDesc& md = A.md;
+  const int C = A.C;
+  // texels are read for the gradients of uv and the LOD only
+  const bool want = !kCube && FILTER != DR_FILTER_NEAREST && (A.d_uv || A.d_uv_da || A.d_bias);
+  const bool shared_tex = A.tex_stride == 0;
+  const int tiles = A.ntx * A.nty;
+  ManyHot hot;
+  hot.on = false;
+  hot.ux = hot.uy = hot.ix0 = hot.ix1 = hot.iy0 = hot.iy1 = hot.Wk = 0;
+  hot.base = nullptr;
+  hot.w00 = hot.w10 = hot.w01 = hot.w11 = 0.0f;
+  for (int bt = (int)blockIdx.x; bt < total_tiles; bt += (int)gridDim.x) {
+    const int n = bt / tiles, tile = bt - n * tiles;
+    const int ty = tile / A.ntx, tx = tile - ty * A.ntx;
+    const int pw = tx * 16 + (lane & 15), ph = ty * 16 + wave * 4 + (lane >> 4);
+    const bool valid = pw < A.Wi && ph < A.Hi;
+    const int64_t pix = ((int64_t)n * A.Hi + min(ph, A.Hi - 1)) * A.Wi + min(pw, A.Wi - 1);
+    const float* gp = A.d_out + pix * C;
+    auto level_w = [&](int k) { return kCube ? A.Wt : mip_w(md, k); };
+    auto level_h = [&](int k) { return kCube ? A.Ht : mip_h(md, k); };
+    // float offset of level (face) k within the image's texture or pyramid
+    auto level_ptr = [&](int k) -> const float* {
+      if (kCube) return A.tex + n * A.tex_stride + (int64_t)k * A.Ht * A.Wt * C;
+      return k == 0 ? A.tex + n * A.tex_stride
+                    : A.pyr + mip_off(md, k) + (shared_tex ? 0 : (int64_t)n * mip_h(md, k) * mip_w(md, k) * C);
+    };
+    auto dlevel_ptr = [&](int k) -> float* {
+      if (kCube) return A.d_tex + n * A.tex_stride + (int64_t)k * A.Ht * A.Wt * C;
+      return k == 0 ? A.d_tex + n * A.tex_stride
+                    : A.d_pyr + mip_off(md, k) + (shared_tex ? 0 : (int64_t)n * mip_h(md, k) * mip_w(md, k) * C);
+    };
+
+    // -- per pixel: LOD and footprints ------------------------------------------
+    TapSlot q[2];
+    float fx[2] = {0.0f, 0.0f}, fy[2] = {0.0f, 0.0f};
+    int tx1[2] = {0, 0}, ty1[2] = {0, 0};   // second column and row as texels
+    int tx0[2] = {0, 0}, ty0[2] = {0, 0};   // first
+    int mask[2] = {15, 15};                 // zero boundary: taps inside the image
+    float4 da_in = make_float4(0.f, 0.f, 0.f, 0.f), da = da_in;
+    float s = 1.0f;
+    const bool scaled = mip && (A.bias_map != nullptr || A.has_bias);
+    float2 uvp = make_float2(0.0f, 0.0f);
+    bool need1 = false;
+    q[0].k = q[1].k = 0;
+    q[0].scale = 1.0f;
+    q[1].scale = 0.0f;
+    Bilin cb;
+    if (kCube) {
+      const float* d = A.uv + pix * 3;
+      q[0].k = cube_bilin(d[0], d[1], d[2], A.Wt, A.Ht, cb);
+    } else {
+      uvp = ld_nt2(A.uv + pix * 2);
+    }
+    if (mip) {
+      da_in = ld_nt4(A.uv_da + pix * 4);
+      if (scaled) s = bias_scale(A.bias_map, pix, A.scale_bias, A.has_bias != 0);
+      da = scaled ? make_float4(da_in.x * s, da_in.y * s, da_in.z * s, da_in.w * s) : da_in;
+      const Lod ld = mip_lod(da, A.Ht, A.Wt, md.L, FILTER == DR_FILTER_LINEAR_MIPMAP_LINEAR);
+      q[0].k = ld.k0;
+      q[0].scale = 1.0f - ld.frac;
+      q[1].k = ld.k1;
+      q[1].scale = ld.frac;
+      need1 = ld.frac != 0.0f || (FILTER == DR_FILTER_LINEAR_MIPMAP_LINEAR && ld.k0 != 0);
+    }
+#pragma unroll
+    for (int li = 0; li < (mip ? 2 : 1); ++li) {
+      const int k = q[li].k, Hk = level_h(k), Wk = level_w(k);
+      Bilin b;
+      if (kCube) {
+        b = cb;
+      } else if (FILTER == DR_FILTER_NEAREST) {  // one tap (Texture.swift:576-605)
+        float ox, oy;
+        b.tx0 = f2i(floorf(uvp.x * (float)Wk));
+        b.ty0 = f2i(floorf(uvp.y * (float)Hk));
+        b.ix0 = b.ix1 = apply_boundary(b.tx0, Wk, BND, ox);
+        b.iy0 = b.iy1 = apply_boundary(b.ty0, Hk, BND, oy);
+        b.fx = b.fy = 0.0f;
+        b.w00 = b.m00 = b.m10 = b.m01 = b.m11 = (1.0f - ox) * (1.0f - oy);
+        b.w10 = b.w01 = b.w11 = 0.0f;
+      } else {
+        b = bilin(uvp.x, uvp.y, Wk, Hk, BND);
+      }
+      float w00 = b.w00, w10 = b.w10, w01 = b.w01, w11 = b.w11;
+      if (b.ix1 == b.ix0) { w00 += w10; w01 += w11; w10 = 0.0f; w11 = 0.0f; }
+      if (b.iy1 == b.iy0) { w00 += w01; w10 += w11; w01 = 0.0f; w11 = 0.0f; }
+      const bool on = valid && q[li].scale != 0.0f;
+      q[li].w00 = on ? w00 : 0.0f; q[li].w10 = on ? w10 : 0.0f;
+      q[li].w01 = on ? w01 : 0.0f; q[li].w11 = on ? w11 : 0.0f;
+      fx[li] = b.fx; fy[li] = b.fy;
+      tx0[li] = b.ix0; tx1[li] = b.ix1; ty0[li] = b.iy0; ty1[li] = b.iy1;
+      if (BND == DR_BOUNDARY_ZERO)
+        mask[li] = (b.m00 != 0.0f ? 1 : 0) | (b.m10 != 0.0f ? 2 : 0) | (b.m01 != 0.0f ? 4 : 0) |
+                   (b.m11 != 0.0f ? 8 : 0);
+      if (BND == DR_BOUNDARY_WRAP) {
+        q[li].ix0 = win_coord(b.tx0, b.ix0); q[li].ix1 = q[li].ix0 + 1;
+        q[li].iy0 = win_coord(b.ty0, b.iy0); q[li].iy1 = q[li].iy0 + 1;
+      } else {
+        q[li].ix0 = b.ix0; q[li].ix1 = b.ix1; q[li].iy0 = b.iy0; q[li].iy1 = b.iy1;
+      }
+    }
+    if (!mip) {
+      q[1].ix0 = q[1].ix1 = q[1].iy0 = q[1].iy1 = 0;
+      q[1].w00 = q[1].w10 = q[1].w01 = q[1].w11 = 0.0f;
+    }
+
+    // -- empty pixels (k_tex_bwd_win): lanes of one uv, summed per wave --------
+    bool use0 = q[0].w00 != 0.0f || q[0].w10 != 0.0f || q[0].w01 != 0.0f || q[0].w11 != 0.0f;
+    const bool use1 = q[1].w00 != 0.0f || q[1].w10 != 0.0f || q[1].w01 != 0.0f || q[1].w11 != 0.0f;
+    bool in_hot = false;  // slot 0's gradient is in the hot sum
+    if (!kCube) {
+      const int ux = __float_as_int(uvp.x), uy = __float_as_int(uvp.y);
+      const int lx = dpp_shift<0x111>(ux), ly = dpp_shift<0x111>(uy);
+      const int rx = dpp_shift<0x101>(ux), ry = dpp_shift<0x101>(uy);
+      const bool left = (lane & 15) != 0 && lx == ux && ly == uy;
+      const bool right = (lane & 15) != 15 && rx == ux && ry == uy;
+      const uint64_t cand = __ballot(use0 && ((uvp.x == 0.0f && uvp.y == 0.0f) || left || right));
+      if (cand != 0ull) {  // uniform; one group a wave and tile
+        const int leader = __ffsll((long long)cand) - 1;
+        const int lux = __builtin_amdgcn_readlane(ux, leader), luy = __builtin_amdgcn_readlane(uy, leader);
+        const int lk = __builtin_amdgcn_readlane(q[0].k, leader);
+        in_hot = use0 && ux == lux && uy == luy && q[0].k == lk;
+        float* base = dlevel_ptr(lk);
+        if (!(hot.on && hot.ux == lux && hot.uy == luy && hot.base == base)) {
+          if (hot.on) {
+            hot_flush(hot, C, s_hot[wave]);
+            for (int c = lane; c < C; c += 64) s_hot[wave][c] = 0.0;
+          }
+          hot.on = true;
+          hot.ux = lux;
+          hot.uy = luy;
+          hot.base = base;
+          hot.Wk = level_w(lk);
+          hot.ix0 = __builtin_amdgcn_readlane(tx0[0], leader);
+          hot.ix1 = __builtin_amdgcn_readlane(tx1[0], leader);
+          hot.iy0 = __builtin_amdgcn_readlane(ty0[0], leader);
+          hot.iy1 = __builtin_amdgcn_readlane(ty1[0], leader);
+          hot.w00 = leader_weight(q[0], leader, 0);
+          hot.w10 = leader_weight(q[0], leader, 1);
+          hot.w01 = leader_weight(q[0], leader, 2);
+          hot.w11 = leader_weight(q[0], leader, 3);
+        }
+        for (int c = 0; c < C; c += 4) {
+          const float4 g = in_hot ? ld_chunk(gp + c, min(4, C - c)) : make_float4(0.f, 0.f, 0.f, 0.f);
+          const float x[4] = {g.x * q[0].scale, g.y * q[0].scale, g.z * q[0].scale, g.w * q[0].scale};
+          const float z = wave_sum4(x);  // lane l: total of value l & 3
+          if (lane < 4 && c + lane < C) s_hot[wave][c + lane] += (double)z;
+        }
+        if (in_hot) use0 = false;
+      }
+    }
+
+    // -- boxes of the levels in use, and their windows (k_tex_bwd_win) -----------
+    {
+      const int lm = wave_or((use0 ? 1 << q[0].k : 0) | (use1 ? 1 << q[1].k : 0));
+#pragma unroll 1
+      for (int rem = lm; rem != 0; rem &= rem - 1) {
+        const int L = __builtin_ctz(rem);
+        int x0 = 32767, x1 = -32767, y0 = 32767, y1 = -32767;
+#pragma unroll
+        for (int li = 0; li < 2; ++li) {
+          const bool u = li == 0 ? use0 : use1;
+          if (!u || q[li].k != L) continue;
+          int a0, a1, b0, b1;
+          slot_box(q[li], a0, a1, b0, b1);
+          x0 = min(x0, a0); x1 = max(x1, a1); y0 = min(y0, b0); y1 = max(y1, b1);
+        }
+        const int px = wave_min_pk16(pack16(x0, -x1));
+        const int py = wave_min_pk16(pack16(y0, -y1));
+        if (lane == 0) s_lbox[wave][L] = make_int2(px, py);
+      }
+      if (lane == 0) s_lmask[wave] = lm;
+    }
+    __syncthreads();
+    const int4 wm = *reinterpret_cast<const int4*>(s_lmask);
+    const int lmask = __builtin_amdgcn_readfirstlane(wm.x | wm.y | wm.z | wm.w);
+    // lane L of each 16-lane row: level L's box, and (below) its place
+    int bx = 0, by = 0, bw = 0, bh = 0;
+    {
+      const int L = lane & 15;
+      int px = pack16(32767, 32767), py = px;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int mv = v == 0 ? wm.x : v == 1 ? wm.y : v == 2 ? wm.z : wm.w;
+        if ((mv >> L) & 1) {
+          const int2 b = s_lbox[v][L];
+          px = pk16_min(px, b.x);
+          py = pk16_min(py, b.y);
+        }
+      }
+      const int x0 = unpack16_lo(px), x1 = -unpack16_hi(px);
+      const int y0 = unpack16_lo(py), y1 = -unpack16_hi(py);
+      if (((lmask >> L) & 1) && x1 >= x0 && y1 >= y0) {
+        bx = x0; by = y0; bw = x1 - x0 + 1; bh = y1 - y0 + 1;
+      }
+    }
+    constexpr int kMaxTexels = kManyPool / 4;  // with four channels in the pool
+    const int64_t area64 = (int64_t)bw * bh;
+    const int fit = area64 <= kMaxTexels ? (int)area64 : 0;
+    int incl = fit;  // prefix sum of the fitting areas along the 16-lane row
+    {
+      int t = dpp_shift<0x111>(incl);
+      incl += t;
+      t = dpp_shift<0x112>(incl);
+      incl += t;
+      t = dpp_shift<0x114>(incl);
+      incl += t;
+      t = dpp_shift<0x118>(incl);
+      incl += t;
+    }
+    const bool usable = fit > 0 && incl <= kMaxTexels;
+    const int at = usable ? incl - fit : -1;  // first texel in the pool, -1: no window
+    // texels of the windows, and the channels that then fit (a multiple of 4)
+    const int texels = wave_max(usable ? incl : 0);
+    const int cap_c = texels > 0 ? min((kManyPool / texels) & ~3, (C + 3) & ~3) : (C + 3) & ~3;
+    // nowin: levels in use without a window
+    int nowin = 0;
+#pragma unroll 1
+    for (int rem = lmask; rem != 0; rem &= rem - 1) {
+      const int k = __builtin_ctz(rem);
+      if (__builtin_amdgcn_readlane(at, k) < 0) nowin |= 1 << k;
+    }
+
+    // a slot's tap cells in the pool (clamped into its box: a zero-weight
+    // tap outside it adds 0), -1 without a window, and its run
+    int o[2][4];
+    RowRun run[2];
+    int maxlen[2] = {0, 0};
+    bool adds[2] = {false, false};
+#pragma unroll
+    for (int li = 0; li < (mip ? 2 : 1); ++li) {
+      const bool u = li == 0 ? use0 : use1;
+      const int k = q[li].k;
+      const int wx = __builtin_amdgcn_ds_bpermute(k << 2, bx), wy = __builtin_amdgcn_ds_bpermute(k << 2, by);
+      const int ww = __builtin_amdgcn_ds_bpermute(k << 2, bw), wh = __builtin_amdgcn_ds_bpermute(k << 2, bh);
+      const int wa = __builtin_amdgcn_ds_bpermute(k << 2, at);
+      const int cx0 = min(max(q[li].ix0 - wx, 0), ww - 1), cx1 = min(max(q[li].ix1 - wx, 0), ww - 1);
+      const int r0 = wa + min(max(q[li].iy0 - wy, 0), wh - 1) * ww;
+      const int r1 = wa + min(max(q[li].iy1 - wy, 0), wh - 1) * ww;
+      o[li][0] = r0 + cx0; o[li][1] = r0 + cx1; o[li][2] = r1 + cx0; o[li][3] = r1 + cx1;
+      const uint64_t key = !u ? (0x7FFFull << 45) | (uint64_t)lane
+                              // (a border's merged column or row has the first coordinate twice)
+                              : ((uint64_t)k << 60) | ((uint64_t)(uint16_t)q[li].ix0 << 16) |
+                                    (uint16_t)q[li].iy0 |
+                                    ((uint64_t)(q[li].ix0 == q[li].ix1) << 32) |
+                                    ((uint64_t)(q[li].iy0 == q[li].iy1) << 33);
+      run[li] = row_run(key);
+      maxlen[li] = wave_max(run[li].li - run[li].s + 1);
+      adds[li] = u && run[li].tail && wa >= 0;
+    }
+
+    // -- channels: d_uv and the LOD samples, the windows' sums, their flush -----
+    float dfx_total = 0.0f, dfy_total = 0.0f, samp[2] = {0.0f, 0.0f};
+    const bool lod0 = FILTER != DR_FILTER_LINEAR_MIPMAP_LINEAR || (q[0].k == 0 && q[1].scale == 0.0f);
+    float dfx[2] = {0.0f, 0.0f}, dfy[2] = {0.0f, 0.0f};
+#pragma unroll 1
+    for (int c0 = 0; c0 < C; c0 += cap_c) {
+      const int c1 = min(C, c0 + cap_c);
+#pragma unroll 1
+      for (int c = c0; c < c1; c += 4) {
+        const int nc = min(4, C - c);
+        const float4 g4 = valid ? ld_chunk(gp + c, nc) : make_float4(0.f, 0.f, 0.f, 0.f);
+        const float g[4] = {g4.x, g4.y, g4.z, g4.w};
+#pragma unroll
+        for (int li = 0; li < (mip ? 2 : 1); ++li) {
+          const bool flat = BND != DR_BOUNDARY_ZERO && tx0[li] == tx1[li] && ty0[li] == ty1[li] && lod0;
+          if (want && valid && (li == 0 || need1) && !flat) {
+            const int k = q[li].k, Wk = level_w(k);
+            const float* lv = level_ptr(k) + c;
+            const uint32_t ra = (uint32_t)ty0[li] * (uint32_t)Wk, rb = (uint32_t)ty1[li] * (uint32_t)Wk;
+            const float4 A0 = ld_chunk(lv + (ra + (uint32_t)tx0[li]) * (uint32_t)C, nc);
+            const float4 A1 = ld_chunk(lv + (ra + (uint32_t)tx1[li]) * (uint32_t)C, nc);
+            const float4 A2 = ld_chunk(lv + (rb + (uint32_t)tx0[li]) * (uint32_t)C, nc);
+            const float4 A3 = ld_chunk(lv + (rb + (uint32_t)tx1[li]) * (uint32_t)C, nc);
+            const float a0[4] = {A0.x, A0.y, A0.z, A0.w}, a1[4] = {A1.x, A1.y, A1.z, A1.w};
+            const float a2[4] = {A2.x, A2.y, A2.z, A2.w}, a3[4] = {A3.x, A3.y, A3.z, A3.w};
+            const float u = fx[li], v = fy[li];
+            const float sc = mip ? q[li].scale : 1.0f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const float t00 = (mask[li] & 1) ? a0[j] : 0.0f, t10 = (mask[li] & 2) ? a1[j] : 0.0f;
+              const float t01 = (mask[li] & 4) ? a2[j] : 0.0f, t11 = (mask[li] & 8) ? a3[j] : 0.0f;
+              const float gc = g[j] * sc;
+              dfx[li] += gc * ((1.0f - v) * (t10 - t00) + v * (t11 - t01));
+              dfy[li] += gc * ((1.0f - u) * (t01 - t00) + u * (t11 - t10));
+              if (mip) {
+                const float sample = (1.0f - u) * (1.0f - v) * t00 + u * (1.0f - v) * t10 +
+                                     (1.0f - u) * v * t01 + u * v * t11;
+                samp[li] += sample * g[j];
+              }
+            }
+          }
+          const bool us = li == 0 ? use0 : use1;
+          if (__ballot(us) == 0ull) continue;
+          const float sc = mip ? q[li].scale : 1.0f;
+          const float wt[4] = {q[li].w00, q[li].w10, q[li].w01, q[li].w11};
+          float v[16];
+#pragma unroll
+          for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[t * 4 + j] = us ? wt[t] * (g[j] * sc) : 0.0f;
+          row_run_scan_n(run[li], v, maxlen[li]);
+          if (adds[li]) {
+            double* w = win + (c - c0) * texels;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              if (j < nc) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) atomicAdd(w + j * texels + o[li][t], (double)v[t * 4 + j]);
+              }
+            }
+          }
+        }
+      }
+      __syncthreads();
+      // consecutive lanes take consecutive channels of a texel
+      const int nch = c1 - c0;
+      const float inv = __builtin_amdgcn_rcpf((float)nch);
+#pragma unroll 1
+      for (int rem = lmask & ~nowin; rem != 0; rem &= rem - 1) {  // uniform
+        const int k = __builtin_ctz(rem);
+        const int W = __builtin_amdgcn_readlane(bw, k), H = __builtin_amdgcn_readlane(bh, k);
+        const int a0 = __builtin_amdgcn_readlane(at, k);
+        float* base = dlevel_ptr(k) + c0;
+        const int Wk = level_w(k), Hk = level_h(k);
+        const int X0 = win_texel<BND>(__builtin_amdgcn_readlane(bx, k), Wk);
+        const int Y0 = win_texel<BND>(__builtin_amdgcn_readlane(by, k), Hk);
+        const float invw = __builtin_amdgcn_rcpf((float)W);
+        for (int i = tid; i < W * H * nch; i += 256) {
+          // i < 2^13: the products with the reciprocals stay clear of integers
+          const int e = f2i(((float)i + 0.5f) * inv), ch = i - e * nch;
+          const int r = f2i(((float)e + 0.5f) * invw), x = e - r * W;
+          double* p = win + ch * texels + a0 + e;
+          const double v = *p;
+          if (v != 0.0) {
+            int X = X0 + x, Y = Y0 + r;
+            if (BND == DR_BOUNDARY_WRAP) {
+              X = wrap_up(X, Wk);
+              Y = wrap_up(Y, Hk);
+            }
+            unsafeAtomicAdd(base + ((int64_t)Y * Wk + X) * C + ch, (float)v);
+            *p = 0.0;
+          }
+        }
+      }
+      __syncthreads();
+    }
+
+    // -- levels without a window: a pixel at a time, lanes on (tap, channel):
+    //    a texel's channels in one request ------------------------------------
+    if (nowin != 0) {
+#pragma unroll
+      for (int li = 0; li < (mip ? 2 : 1); ++li) {
+        const int k = q[li].k;
+        const bool u = (li == 0 ? use0 : use1) && ((nowin >> k) & 1);
+        const float sc = mip ? q[li].scale : 1.0f;
+        // four pixels a step: their cotangents are loaded together
+        for (uint64_t m = __ballot(u); m != 0ull;) {
+          int e[4];
+          float w[4];
+          const float* ge[4];
+          float* p[4];
+          const int t = lane >> 4;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const bool on = m != 0ull;  // uniform; past the last one: its lane again, weight 0
+            e[r] = on ? __ffsll((long long)m) - 1 : e[r > 0 ? r - 1 : 0];
+            m &= m - 1;
+            const int kk = __builtin_amdgcn_readlane(k, e[r]), Wk = level_w(kk);
+            w[r] = on ? leader_weight(q[li], e[r], t) *
+                            __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sc), e[r]))
+                      : 0.0f;
+            const int X = (t & 1) ? __builtin_amdgcn_readlane(tx1[li], e[r]) : __builtin_amdgcn_readlane(tx0[li], e[r]);
+            const int Y = (t & 2) ? __builtin_amdgcn_readlane(ty1[li], e[r]) : __builtin_amdgcn_readlane(ty0[li], e[r]);
+            const int ph_e = ty * 16 + wave * 4 + (e[r] >> 4), pw_e = tx * 16 + (e[r] & 15);
+            ge[r] = A.d_out + (((int64_t)n * A.Hi + ph_e) * A.Wi + pw_e) * C;
+            p[r] = dlevel_ptr(kk) + ((int64_t)Y * Wk + X) * C;
+          }
+          for (int c = lane & 15; c < C; c += 16) {
+            float v[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = ge[r][c];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const float x = w[r] * v[r];
+              if (w[r] != 0.0f && x != 0.0f) unsafeAtomicAdd(p[r] + c, x);
+            }
+          }
+        }
+      }
+    }
+
+    // -- d_uv, d_uvDA, d_bias (Texture.swift:500-520, :979-1102) -----------------
+    if (kCube) {
+      if (A.d_uv && valid) {
+        A.d_uv[pix * 3 + 0] = 0.0f;
+        A.d_uv[pix * 3 + 1] = 0.0f;
+        A.d_uv[pix * 3 + 2] = 0.0f;
+      }
+      continue;
+    }
+    if (!valid) continue;
+#pragma unroll
+    for (int li = 0; li < (mip ? 2 : 1); ++li) {
+      dfx_total += dfx[li] * (float)level_w(q[li].k);
+      dfy_total += dfy[li] * (float)level_h(q[li].k);
+    }
+    if (A.d_uv) st_nt2(A.d_uv + pix * 2, make_float2(dfx_total, dfy_total));
+    if (!mip || (!A.d_uv_da && !A.d_bias)) continue;
+    const float sx = da.x * (float)A.Wt, sy = da.y * (float)A.Wt;
+    const float tx_ = da.z * (float)A.Ht, ty_ = da.w * (float)A.Ht;
+    const float Asq = sx * sx + tx_ * tx_;
+    const float Bsq = sy * sy + ty_ * ty_;
+    const float rho_sq = fmaxf(Asq, Bsq);
+    const float lod_raw = 0.5f * log2f(fmaxf(rho_sq, 1e-20f));
+    float4 d_eff = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (!(lod_raw <= 0.0f || lod_raw >= (float)(md.L - 1))) {
+      float d_lod;
+      if (FILTER == DR_FILTER_LINEAR_MIPMAP_LINEAR) {
+        d_lod = -samp[0] + samp[1];
+      } else {  // the trilinear surrogate's two levels
+        const int k0 = f2i(floorf(lod_raw));
+        const int k1 = min(k0 + 1, md.L - 1);
+        float s0 = 0.0f, s1 = 0.0f;
+        const Bilin b0 = bilin(uvp.x, uvp.y, mip_w(md, k0), mip_h(md, k0), BND);
+        const Bilin b1 = bilin(uvp.x, uvp.y, mip_w(md, k1), mip_h(md, k1), BND);
+        for (int c = 0; c < C; c += 4) {
+          const int nc = min(4, C - c);
+          const float4 g = ld_chunk(gp + c, nc);
+          const float4 a = sample_chunk(level_ptr(k0), mip_w(md, k0), C, b0, c, nc);
+          const float4 b = sample_chunk(level_ptr(k1), mip_w(md, k1), C, b1, c, nc);
+          s0 += a.x * g.x; s0 += a.y * g.y; s0 += a.z * g.z; s0 += a.w * g.w;
+          s1 += b.x * g.x; s1 += b.y * g.y; s1 += b.z * g.z; s1 += b.w * g.w;
+        }
+        d_lod = -s0 + s1;
+      }
+      const float ln2 = 0.6931471805599453f;
+      const float dlod_drho_sq = 1.0f / (2.0f * rho_sq * ln2);
+      const float A_is_max = (Asq >= Bsq) ? 1.0f : 0.0f;
+      const float B_is_max = 1.0f - A_is_max;
+      d_eff = make_float4(d_lod * dlod_drho_sq * A_is_max * 2.0f * sx * (float)A.Wt,
+                          d_lod * dlod_drho_sq * B_is_max * 2.0f * sy * (float)A.Wt,
+                          d_lod * dlod_drho_sq * A_is_max * 2.0f * tx_ * (float)A.Ht,
+                          d_lod * dlod_drho_sq * B_is_max * 2.0f * ty_ * (float)A.Ht);
+    }
+    if (A.d_uv_da) {
+      const float4 ov = scaled ? make_float4(d_eff.x * s, d_eff.y * s, d_eff.z * s, d_eff.w * s) : d_eff;
+      st_nt4(A.d_uv_da + pix * 4, ov);
+    }
+    if (A.d_bias && A.bias_map) {
+      const float gm = d_eff.x * da_in.x + d_eff.y * da_in.y + d_eff.z * da_in.z + d_eff.w * da_in.w;
+      A.d_bias[pix] = gm * s * 0.6931471805599453f;
+    }
+  }
+  // the waves' empty-pixel sums, those of one footprint together (one
+  // workgroup's atomics on a texel instead of four waves')
+  if (lane == 0) {
+    s_hbase[wave] = hot.on ? (uint64_t)hot.base : 0ull;
+    s_hkey[wave] = make_int2(hot.ux, hot.uy);
+  }
+  __syncthreads();
+  if (!hot.on) return;
+  auto same = [&](int w) {
+    return s_hbase[w] == s_hbase[wave] && s_hkey[w].x == s_hkey[wave].x && s_hkey[w].y == s_hkey[wave].y;
+  };
+  for (int w = 0; w < wave; ++w)
+    if (same(w)) return;  // an earlier wave writes this footprint
+  for (int w = wave + 1; w < 4; ++w)
+    if (same(w))
+      for (int c = lane; c < C; c += 64) s_hot[wave][c] += s_hot[w][c];
+  __builtin_amdgcn_wave_barrier();  // (LDS is ordered within a wave)
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  hot_flush(hot, C, s_hot[wave]);
+}
+
+// Texture.swift:156: level k = 2x2 mean of level k-1.  Builds up to five
+// levels at once: each workgroup reduces a 32 x 32 patch of level s, four
+// channels of it, through levels s+1..s+m in LDS (m <= 5; the sizes of
+// levels s..s+m-1 are even, so the patches' outputs do not straddle).  More
+// than four channels take a workgroup per four, neighbours in the grid (512^2 x
+// 16: nine single-level launches, 66 us; two of these, 29 us).
 constexpr int kMipMaxC = 4;
+constexpr int kMipPatchLog = 5, kMipPatch = 1 << kMipPatchLog;
 
 __global__ void __launch_bounds__(256) k_mip_block(const float* __restrict__ src,
                                                    float* __restrict__ pyr, MipDesc md, int s,
-                                                   int m, int Nt, int C) {
+                                                   int m, int C) {
   __shared__ float buf[2][256 * kMipMaxC];
-  const int bs = 1 << m;  // source block edge
   const int Ws = md.w[s];
-  const int nbx = Ws / bs;
-  const int bx = (int)blockIdx.x % nbx, by = (int)blockIdx.x / nbx;
-  const int n = (int)blockIdx.y;
-  const float* lvl = src + (int64_t)n * md.h[s] * Ws * C;
+  const int nbx = (Ws + kMipPatch - 1) / kMipPatch;
+  const int per_n = nbx * ((md.h[s] + kMipPatch - 1) / kMipPatch);
+  const int chunks = (C + kMipMaxC - 1) / kMipMaxC;
+  int blk = (int)blockIdx.x / chunks;
+  const int c0 = ((int)blockIdx.x - blk * chunks) * kMipMaxC, nc = min(kMipMaxC, C - c0);
+  const int n = blk / per_n;
+  blk -= n * per_n;
+  const int by = blk / nbx, bx = blk - by * nbx;
+  const float* lvl = src + (int64_t)n * md.h[s] * Ws * C + c0;
   int cur = 0;
   for (int j = 1; j <= m; ++j) {
-    const int e = bs >> j;  // output edge at this step
+    const int e = kMipPatch >> j;  // output edge at this step
     const int k = s + j;
-    const int Wk = md.w[k];
-    float* dst = pyr + md.off[k] + (int64_t)n * md.h[k] * Wk * C;
-    for (int t = threadIdx.x; t < e * e * C; t += blockDim.x) {
-      const int c = t % C, q = t / C;
-      const int x = q % e, y = q / e;
+    const int Wk = md.w[k], Hk = md.h[k];
+    float* dst = pyr + md.off[k] + (int64_t)n * Hk * Wk * C + c0;
+    for (int t = threadIdx.x; t < e * e * nc; t += blockDim.x) {
+      const int q = t / nc, c = t - q * nc;
+      const int y = q >> (kMipPatchLog - j), x = q & (e - 1);
+      const int ox = bx * e + x, oy = by * e + y;
+      if (ox >= Wk || oy >= Hk) continue;  // past the level's edge
       float a, b, d, f;
       if (j == 1) {
-        const int sx = bx * bs + 2 * x, sy = by * bs + 2 * y;
+        const int sx = 2 * ox, sy = 2 * oy;
         a = lvl[((int64_t)sy * Ws + sx) * C + c];
         b = lvl[((int64_t)sy * Ws + sx + 1) * C + c];
         d = lvl[((int64_t)(sy + 1) * Ws + sx) * C + c];
@@ -1531,14 +2143,13 @@ __global__ void __launch_bounds__(256) k_mip_block(const float* __restrict__ src
       } else {
         const int pe = 2 * e;
         const float* pb = buf[cur ^ 1];
-        a = pb[((2 * y) * pe + 2 * x) * C + c];
-        b = pb[((2 * y) * pe + 2 * x + 1) * C + c];
-        d = pb[((2 * y + 1) * pe + 2 * x) * C + c];
-        f = pb[((2 * y + 1) * pe + 2 * x + 1) * C + c];
+        a = pb[((2 * y) * pe + 2 * x) * nc + c];
+        b = pb[((2 * y) * pe + 2 * x + 1) * nc + c];
+        d = pb[((2 * y + 1) * pe + 2 * x) * nc + c];
+        f = pb[((2 * y + 1) * pe + 2 * x + 1) * nc + c];
       }
       const float v = (((a + b) + d) + f) * 0.25f;
-      buf[cur][(y * e + x) * C + c] = v;
-      const int ox = bx * e + x, oy = by * e + y;
+      buf[cur][(y * e + x) * nc + c] = v;
       dst[((int64_t)oy * Wk + ox) * C + c] = v;
     }
     __syncthreads();
@@ -1552,11 +2163,11 @@ __global__ void __launch_bounds__(256) k_mip_block_c4(const float* __restrict__ 
                                                       float* __restrict__ pyr, MipDesc md, int s,
                                                       int m) {
   __shared__ float4 buf[2][256];
-  const int bs = 1 << m;  // source block edge
   const int Ws = md.w[s];
-  const int nbx = Ws / bs;
-  const int bx = (int)blockIdx.x % nbx, by = (int)blockIdx.x / nbx;
-  const int n = (int)blockIdx.y;
+  const int nbx = (Ws + kMipPatch - 1) / kMipPatch;
+  const int per_n = nbx * ((md.h[s] + kMipPatch - 1) / kMipPatch);
+  const int n = (int)blockIdx.x / per_n, blk = (int)blockIdx.x - n * per_n;
+  const int by = blk / nbx, bx = blk - by * nbx;
   const float4* lvl = reinterpret_cast<const float4*>(src) + (int64_t)n * md.h[s] * Ws;
   auto mean4 = [](float4 a, float4 b, float4 d, float4 f) {
     return make_float4((((a.x + b.x) + d.x) + f.x) * 0.25f, (((a.y + b.y) + d.y) + f.y) * 0.25f,
@@ -1564,15 +2175,17 @@ __global__ void __launch_bounds__(256) k_mip_block_c4(const float* __restrict__ 
   };
   int cur = 0;
   for (int j = 1; j <= m; ++j) {
-    const int e = bs >> j;  // output edge at this step
+    const int e = kMipPatch >> j;  // output edge at this step
     const int k = s + j;
-    const int Wk = md.w[k];
-    float4* dst = reinterpret_cast<float4*>(pyr + md.off[k]) + (int64_t)n * md.h[k] * Wk;
+    const int Wk = md.w[k], Hk = md.h[k];
+    float4* dst = reinterpret_cast<float4*>(pyr + md.off[k]) + (int64_t)n * Hk * Wk;
     for (int t = threadIdx.x; t < e * e; t += blockDim.x) {
-      const int x = t % e, y = t / e;
+      const int y = t >> (kMipPatchLog - j), x = t & (e - 1);
+      const int ox = bx * e + x, oy = by * e + y;
+      if (ox >= Wk || oy >= Hk) continue;  // past the level's edge
       float4 v;
       if (j == 1) {
-        const int sx = bx * bs + 2 * x, sy = by * bs + 2 * y;
+        const int sx = 2 * ox, sy = 2 * oy;
         v = mean4(lvl[(int64_t)sy * Ws + sx], lvl[(int64_t)sy * Ws + sx + 1],
                   lvl[(int64_t)(sy + 1) * Ws + sx], lvl[(int64_t)(sy + 1) * Ws + sx + 1]);
       } else {
@@ -1582,7 +2195,7 @@ __global__ void __launch_bounds__(256) k_mip_block_c4(const float* __restrict__ 
                   pb[(2 * y + 1) * pe + 2 * x], pb[(2 * y + 1) * pe + 2 * x + 1]);
       }
       buf[cur][y * e + x] = v;
-      dst[(int64_t)(by * e + y) * Wk + bx * e + x] = v;
+      dst[(int64_t)oy * Wk + ox] = v;
     }
     __syncthreads();
     cur ^= 1;
@@ -1592,68 +2205,57 @@ __global__ void __launch_bounds__(256) k_mip_block_c4(const float* __restrict__ 
 // Backward of the pyramid (MLX autodiff of concatenate + mean): level k's
 // total cotangent is its own gradient plus 1/4 of level k+1's total,
 // accumulated from the coarsest level down; level 0's total is added to
-// d_tex (which already holds level 0's own gradient).
-__global__ void __launch_bounds__(256) k_mip_collapse(const float* __restrict__ d_pyr, MipDesc md,
-                                                      int C, int bpr, float* __restrict__ d_tex) {
-  // one thread per texel of level 0: block = 256 texels of one row
-  const int64_t row = (int64_t)blockIdx.x / bpr;  // n * H + y
-  const int x = (int)((int64_t)blockIdx.x - row * bpr) * 256 + (int)threadIdx.x;
-  if (x >= md.w[0] || md.L < 2) return;
-  const int y = (int)(row % md.h[0]);
-  const int n = (int)(row / md.h[0]);
-  const int kL = md.L - 1;
-  float* dt = d_tex + (row * md.w[0] + x) * C;
-  for (int c = 0; c < C; ++c) {
-    auto at = [&](int k) {
-      return d_pyr[md.off[k] + (((int64_t)n * md.h[k] + (y >> k)) * md.w[k] + (x >> k)) * C + c];
-    };
-    float acc = at(kL);
-    for (int k = kL - 1; k >= 1; --k) acc = at(k) + acc * 0.25f;
-    dt[c] = dt[c] + acc * 0.25f;
-  }
-}
+// d_tex (which already holds level 0's own gradient).  Two passes: level 1's
+// totals in place (each of its values walks its chain of ancestors), then
+// level 0 adds a quarter of its parent's total.  A workgroup takes 256
+// values, or vectors of V = 4 where C is a multiple of 4, of one row, so
+// consecutive threads read consecutive memory; one thread per texel walking
+// the whole chain for each of its channels took 71 us at 512^2 x 16, this
+// takes 16.
+template <int V>
+struct alignas(4 * V) VecF {
+  float v[V];
+};
 
-// The same collapse for C = 4 in two passes with texel vectors: level 1's
-// totals first, in place (one thread per level-1 texel walks its chain of
-// ancestors, the same sums in the same order), then level 0 adds a quarter
-// of its parent's total.
-__global__ void __launch_bounds__(256) k_mip_collapse1_c4(float* __restrict__ d_pyr, MipDesc md,
-                                                          int64_t n1) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n1) return;
+template <int V>
+__global__ void __launch_bounds__(256) k_mip_collapse1(float* __restrict__ d_pyr, MipDesc md,
+                                                       int G, int bpr) {
+  const int row = (int)blockIdx.x / bpr;  // n * H1 + y
+  const int i = ((int)blockIdx.x - row * bpr) * 256 + (int)threadIdx.x;  // value of the row
   const int W1 = md.w[1], H1 = md.h[1];
-  const int64_t r = i % ((int64_t)H1 * W1);
-  const int n = (int)(i / ((int64_t)H1 * W1));
-  const int y = (int)(r / W1), x = (int)(r - (int64_t)(r / W1) * W1);
-  const int kL = md.L - 1;
-  auto at = [&](int k) {
+  if (i >= W1 * G) return;
+  const int x = i / G, c = i - x * G;
+  const int n = row / H1, y = row - n * H1;
+  VecF<V>* d = reinterpret_cast<VecF<V>*>(d_pyr);
+  auto at = [&](int k) -> VecF<V>& {
     const int sh = k - 1;
-    return *reinterpret_cast<const float4*>(
-        d_pyr + md.off[k] + (((int64_t)n * md.h[k] + (y >> sh)) * md.w[k] + (x >> sh)) * 4);
+    return d[md.off[k] / V + (((int64_t)n * md.h[k] + (y >> sh)) * md.w[k] + (x >> sh)) * G + c];
   };
-  float4 acc = at(kL);
-  for (int k = kL - 1; k >= 1; --k) {
-    const float4 o = at(k);
-    acc = make_float4(o.x + acc.x * 0.25f, o.y + acc.y * 0.25f, o.z + acc.z * 0.25f,
-                      o.w + acc.w * 0.25f);
+  VecF<V> acc = at(md.L - 1);
+  for (int k = md.L - 2; k >= 1; --k) {
+    const VecF<V> o = at(k);
+#pragma unroll
+    for (int j = 0; j < V; ++j) acc.v[j] = o.v[j] + acc.v[j] * 0.25f;
   }
-  *reinterpret_cast<float4*>(d_pyr + md.off[1] + i * 4) = acc;
+  at(1) = acc;
 }
 
-__global__ void __launch_bounds__(256) k_mip_collapse0_c4(const float* __restrict__ d_pyr,
-                                                          MipDesc md, int64_t n0,
-                                                          float* __restrict__ d_tex) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n0) return;
+template <int V>
+__global__ void __launch_bounds__(256) k_mip_collapse0(const float* __restrict__ d_pyr, MipDesc md,
+                                                       int G, int bpr, float* __restrict__ d_tex) {
+  const int64_t row = (int64_t)blockIdx.x / bpr;  // n * H + y
+  const int i = ((int)blockIdx.x - (int)row * bpr) * 256 + (int)threadIdx.x;
   const int W = md.w[0], H = md.h[0];
-  const int64_t r = i % ((int64_t)H * W);
-  const int n = (int)(i / ((int64_t)H * W));
-  const int y = (int)(r / W), x = (int)(r - (int64_t)(r / W) * W);
-  const float4 t = *reinterpret_cast<const float4*>(
-      d_pyr + md.off[1] + (((int64_t)n * md.h[1] + (y >> 1)) * md.w[1] + (x >> 1)) * 4);
-  float4* dp = reinterpret_cast<float4*>(d_tex + i * 4);
-  const float4 d = *dp;
-  *dp = make_float4(d.x + t.x * 0.25f, d.y + t.y * 0.25f, d.z + t.z * 0.25f, d.w + t.w * 0.25f);
+  if (i >= W * G) return;
+  const int x = i / G, c = i - x * G;
+  const int n = (int)row / H, y = (int)row - n * H;
+  const VecF<V> t = reinterpret_cast<const VecF<V>*>(
+      d_pyr)[md.off[1] / V + (((int64_t)n * md.h[1] + (y >> 1)) * md.w[1] + (x >> 1)) * G + c];
+  VecF<V>* dp = reinterpret_cast<VecF<V>*>(d_tex) + row * W * G + i;
+  VecF<V> d = *dp;
+#pragma unroll
+  for (int j = 0; j < V; ++j) d.v[j] += t.v[j] * 0.25f;
+  *dp = d;
 }
 
 template <int FILTER, int CT, int BND, bool BIAS>
@@ -1690,6 +2292,33 @@ hipError_t launch_tex_bwd_win(const TexBwdArgs& args, int total_tiles, hipStream
   if (args.boundary == DR_BOUNDARY_WRAP)
     return launch_tex_bwd_win_b<FILTER, CT, DR_BOUNDARY_WRAP>(args, total_tiles, stream);
   return launch_tex_bwd_win_b<FILTER, CT, DR_BOUNDARY_ZERO>(args, total_tiles, stream);
+}
+
+template <int FILTER, int BND>
+hipError_t launch_tex_bwd_many(const TexBwdArgs& args, int total_tiles, hipStream_t stream) {
+  static int per_cu = 0;
+  if (per_cu == 0) {
+    int b = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k_tex_bwd_many<FILTER, BND>, 256, 0) !=
+            hipSuccess ||
+        b <= 0)
+      b = 2;
+    per_cu = b;
+  }
+  const int64_t resident = (int64_t)device_cu_count() * per_cu;
+  const unsigned grid = (unsigned)(total_tiles < resident ? total_tiles : resident);
+  hipLaunchKernelGGL((k_tex_bwd_many<FILTER, BND>), dim3(grid), dim3(256), 0, stream, args,
+                     total_tiles);
+  return hipGetLastError();
+}
+
+template <int FILTER>
+hipError_t launch_tex_bwd_many_b(const TexBwdArgs& args, int total_tiles, hipStream_t stream) {
+  if (args.boundary == DR_BOUNDARY_CLAMP)
+    return launch_tex_bwd_many<FILTER, DR_BOUNDARY_CLAMP>(args, total_tiles, stream);
+  if (args.boundary == DR_BOUNDARY_WRAP)
+    return launch_tex_bwd_many<FILTER, DR_BOUNDARY_WRAP>(args, total_tiles, stream);
+  return launch_tex_bwd_many<FILTER, DR_BOUNDARY_ZERO>(args, total_tiles, stream);
 }
 
 // Launches the persistent backward with as many workgroups as fit on the
@@ -2191,32 +2820,24 @@ extern "C" int dr_texture_build_mip(const float* tex, int Nt, int H, int W, int 
   int st = build_desc(H, W, C, Nt, L, md);
   if (st) return st;
   if (L > 1) DR_CHECK_ARG(pyramid != nullptr, "texture_build_mip: null pyramid");
-  if (C <= kMipMaxC) {
-    for (int sl = 0; sl < L - 1;) {
-      const int m = (L - 1 - sl) < 5 ? (L - 1 - sl) : 5;
-      const float* src = sl == 0 ? tex : pyramid + md.off[sl];
-      const int bs = 1 << m;
-      const dim3 grid((unsigned)((md.h[sl] / bs) * (md.w[sl] / bs)), (unsigned)Nt);
-      {
-        DR_TIMED("k_mip_block", stream);
-        if (C == 4 && (((uintptr_t)src | (uintptr_t)pyramid) & 15) == 0)
-          hipLaunchKernelGGL(k_mip_block_c4, grid, dim3(256), 0, stream, src, pyramid, md, sl, m);
-        else
-          hipLaunchKernelGGL(k_mip_block, grid, dim3(256), 0, stream, src, pyramid, md, sl, m, Nt,
-                             C);
-      }
-      DR_CHECK_LAUNCH();
-      sl += m;
+  for (int sl = 0; sl < L - 1;) {
+    const int m = (L - 1 - sl) < 5 ? (L - 1 - sl) : 5;
+    const float* src = sl == 0 ? tex : pyramid + md.off[sl];
+    const int64_t patches = (int64_t)((md.h[sl] + kMipPatch - 1) / kMipPatch) *
+                            ((md.w[sl] + kMipPatch - 1) / kMipPatch) * Nt;
+    const int64_t blocks = patches * ((C + kMipMaxC - 1) / kMipMaxC);
+    DR_CHECK_ARG(blocks < ((int64_t)1 << 31), "texture_build_mip: texture too large");
+    {
+      DR_TIMED("k_mip_block", stream);
+      if (C == 4 && (((uintptr_t)src | (uintptr_t)pyramid) & 15) == 0)
+        hipLaunchKernelGGL(k_mip_block_c4, dim3((unsigned)blocks), dim3(256), 0, stream, src,
+                           pyramid, md, sl, m);
+      else
+        hipLaunchKernelGGL(k_mip_block, dim3((unsigned)blocks), dim3(256), 0, stream, src, pyramid,
+                           md, sl, m, C);
     }
-    return DR_OK;
-  }
-  for (int k = 1; k < L; ++k) {
-    const float* src = k == 1 ? tex : pyramid + md.off[k - 1];
-    const int64_t n = (int64_t)Nt * md.h[k] * md.w[k] * C;
-    DR_TIMED("k_mip_down", stream);
-    hipLaunchKernelGGL(k_mip_down, dim3(grid_for(n, 256)), dim3(256), 0, stream, src,
-                       pyramid + md.off[k], Nt, md.h[k - 1], md.w[k - 1], C);
     DR_CHECK_LAUNCH();
+    sl += m;
   }
   return DR_OK;
 }
@@ -2248,7 +2869,7 @@ static int check_tex(const float* tex, const float* pyr, int Nt, int N, int Ht, 
       case 2: hipLaunchKernelGGL((KERNEL<F, BNDV, 2>), GRID, dim3(256), 0, stream, __VA_ARGS__); break; \
       case 3: hipLaunchKernelGGL((KERNEL<F, BNDV, 3>), GRID, dim3(256), 0, stream, __VA_ARGS__); break; \
       case 4: hipLaunchKernelGGL((KERNEL<F, BNDV, 4>), GRID, dim3(256), 0, stream, __VA_ARGS__); break; \
-      default: hipLaunchKernelGGL((KERNEL<F, BNDV, 0>), GRID, dim3(256), 0, stream, __VA_ARGS__); break; \
+      default: hipLaunchKernelGGL((k_tex_fwd_many<F, BNDV>), GRID, dim3(256), 0, stream, __VA_ARGS__); break; \
     }                                                                                         \
   } while (0)
 
@@ -2272,22 +2893,23 @@ static int check_tex(const float* tex, const float* pyr, int Nt, int N, int Ht, 
 static int mip_collapse(float* d_pyr, const MipDesc& md, int ntex, int Ht, int Wt, int C,
                         float* d_tex, hipStream_t stream) {
   DR_TIMED("k_mip_collapse", stream);
-  if (C == 4 && (((uintptr_t)d_pyr | (uintptr_t)d_tex) & 15) == 0) {
-    if (md.L >= 3) {
-      const int64_t n1 = (int64_t)ntex * md.h[1] * md.w[1];
-      hipLaunchKernelGGL(k_mip_collapse1_c4, dim3(grid_for(n1, 256)), dim3(256), 0, stream,
-                         d_pyr, md, n1);
-      DR_CHECK_LAUNCH();
-    }
-    const int64_t n0 = (int64_t)ntex * Ht * Wt;
-    hipLaunchKernelGGL(k_mip_collapse0_c4, dim3(grid_for(n0, 256)), dim3(256), 0, stream, d_pyr,
-                       md, n0, d_tex);
+  const bool vec = C % 4 == 0 && (((uintptr_t)d_pyr | (uintptr_t)d_tex) & 15) == 0;
+  const int G = vec ? C / 4 : C;  // values of a texel
+  if (md.L >= 3) {
+    const int bpr = (int)(((int64_t)md.w[1] * G + 255) / 256);
+    const dim3 grid((unsigned)((int64_t)ntex * md.h[1] * bpr));
+    if (vec)
+      hipLaunchKernelGGL(k_mip_collapse1<4>, grid, dim3(256), 0, stream, d_pyr, md, G, bpr);
+    else
+      hipLaunchKernelGGL(k_mip_collapse1<1>, grid, dim3(256), 0, stream, d_pyr, md, G, bpr);
     DR_CHECK_LAUNCH();
-    return DR_OK;
   }
-  const int bpr = (Wt + 255) / 256;
-  hipLaunchKernelGGL(k_mip_collapse, dim3((unsigned)((int64_t)ntex * Ht * bpr)), dim3(256), 0,
-                     stream, d_pyr, md, C, bpr, d_tex);
+  const int bpr = (int)(((int64_t)Wt * G + 255) / 256);
+  const dim3 grid((unsigned)((int64_t)ntex * Ht * bpr));
+  if (vec)
+    hipLaunchKernelGGL(k_mip_collapse0<4>, grid, dim3(256), 0, stream, d_pyr, md, G, bpr, d_tex);
+  else
+    hipLaunchKernelGGL(k_mip_collapse0<1>, grid, dim3(256), 0, stream, d_pyr, md, G, bpr, d_tex);
   DR_CHECK_LAUNCH();
   return DR_OK;
 }
@@ -2552,7 +3174,21 @@ static int texture_bwd(const float* tex, const float* pyramid, int Nt, int Ht, i
   }
     const bool windowed = !cube && filter != DR_FILTER_NEAREST && C >= 1 && C <= 4 &&
                           Wt <= 32767 && Ht <= 32767;  // window boxes use 16-bit texel coordinates
-    if (windowed && filter == DR_FILTER_LINEAR) DR_TW(DR_FILTER_LINEAR)
+    // more channels: while the empty pixels' sums have room, texel
+    // coordinates fit 16 bits and a level's floats 32
+    const bool many = C > 4 && C <= kManyC && Wt <= 32767 && Ht <= 32767 &&
+                      (uint64_t)Ht * Wt * C < (1ull << 32);
+    if (many && cube)
+      e = launch_tex_bwd_many<DR_FILTER_LINEAR, DR_BOUNDARY_CUBE>(args, (int)total_tiles, stream);
+    else if (many && filter == DR_FILTER_NEAREST)
+      e = launch_tex_bwd_many_b<DR_FILTER_NEAREST>(args, (int)total_tiles, stream);
+    else if (many && filter == DR_FILTER_LINEAR)
+      e = launch_tex_bwd_many_b<DR_FILTER_LINEAR>(args, (int)total_tiles, stream);
+    else if (many && filter == DR_FILTER_LINEAR_MIPMAP_NEAREST)
+      e = launch_tex_bwd_many_b<DR_FILTER_LINEAR_MIPMAP_NEAREST>(args, (int)total_tiles, stream);
+    else if (many)
+      e = launch_tex_bwd_many_b<DR_FILTER_LINEAR_MIPMAP_LINEAR>(args, (int)total_tiles, stream);
+    else if (windowed && filter == DR_FILTER_LINEAR) DR_TW(DR_FILTER_LINEAR)
     else if (windowed && filter == DR_FILTER_LINEAR_MIPMAP_NEAREST) DR_TW(DR_FILTER_LINEAR_MIPMAP_NEAREST)
     else if (windowed) DR_TW(DR_FILTER_LINEAR_MIPMAP_LINEAR)
     else if (cube) DR_TB_C(DR_FILTER_LINEAR, true)

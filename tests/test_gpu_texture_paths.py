@@ -1,7 +1,9 @@
 """texture's backward paths on smooth uv fields (what a rendered surface
 gives), against the CPU oracle, at the sizes where a path changes: wrap
 windows across the texture's border and repeats; boxes that fill the LDS
-pool, take it in bands, or are written to memory directly."""
+pool, take it in bands, or are written to memory directly; more than four
+channels (chunks of four, remainders, one pool pass or several, the channel
+limit); pyramids of sizes that are no multiple of a patch."""
 import numpy as np
 import pytest
 
@@ -27,12 +29,14 @@ def smooth_uv(rng, N, Hi, Wi, scale, offset, background):
     return uv.astype(np.float32), da.astype(np.float32)
 
 
-def check(rng, tex, uv, da, filt, bnd, rtol=1e-4):
+def check(rng, tex, uv, da, filt, bnd, rtol=1e-4, bias=None):
     from diffrast import DiffRast
     mip = "mipmap" in filt
     t, u = dev(tex).requires_grad_(True), dev(uv).requires_grad_(True)
     d = dev(da).requires_grad_(True) if mip else None
     kw = dict(filterMode=filt, boundaryMode=bnd)
+    if bias is not None:
+        kw["mipLevelBias"] = bias
     out = DiffRast.texture(t, u, uvDA=d, **kw)
     ref = O.texture(tex, uv, uvDA=da if mip else None, **kw)
     assert_fwd_close(host(out), ref)
@@ -77,3 +81,52 @@ def test_minified_boxes(texels, bnd, filt, C):
         da *= 1e-3
     tex = rng.random((1, Ht, Wt, C)).astype(np.float32)
     check(rng, tex, uv, da, filt, bnd)
+
+
+# channels: the first past the four-channel kernels, whole chunks, a pool
+# filled exactly and in several passes, the limit of the empty pixels' sums
+# and one beyond (the general kernel)
+@pytest.mark.parametrize("C", [5, 8, 16, 23, 128, 129])
+@pytest.mark.parametrize("filt,bnd", [("nearest", "wrap"), ("linear", "wrap"), ("linear", "zero"),
+                                      ("linear-mipmap-linear", "clamp"),
+                                      ("linear-mipmap-nearest", "wrap")])
+@pytest.mark.parametrize("Nt,texels", [(1, 0.7), (2, 6.0)])
+def test_many_channels(C, filt, bnd, Nt, texels):
+    torch_dev()
+    rng = np.random.default_rng(C * 10 + Nt)
+    Hi, Wi, Ht, Wt = 35, 38, 64, 96
+    uv, da = smooth_uv(rng, 2, Hi, Wi, texels * Wi / Wt / 1.5, 0.3, (0.0, 0.0))
+    if "mipmap" in filt:
+        da *= 0.6  # off whole LODs (a switch)
+    tex = rng.random((Nt, Ht, Wt, C)).astype(np.float32)
+    check(rng, tex, uv, da, filt, bnd, bias=0.3 if "mipmap" in filt else None)
+
+
+@pytest.mark.parametrize("C", [6, 9])
+def test_many_channels_cube(C):
+    torch_dev()
+    from diffrast import DiffRast
+    rng = np.random.default_rng(C)
+    tex = rng.random((1, 6, 24, 24, C)).astype(np.float32)
+    y, x = np.meshgrid(np.linspace(-2, 2, 33), np.linspace(-2, 2, 40), indexing="ij")
+    dirs = np.stack([np.stack([x, y, np.full_like(x, z)], -1) for z in (0.7, -1.1)])
+    dirs = dirs.astype(np.float32)  # smooth, across the faces' edges
+    t, u = dev(tex).requires_grad_(True), dev(dirs).requires_grad_(True)
+    out = DiffRast.texture(t, u, boundaryMode="cube")
+    np.testing.assert_array_equal(host(out), O.texture(tex, dirs, boundaryMode="cube"))
+    g = rng.normal(size=out.shape).astype(np.float32)
+    out.backward(dev(g))
+    assert_grad_close(host(t.grad), O.texture_vjp(tex, dirs, g, boundaryMode="cube")[0], "d_tex")
+    assert not host(u.grad).any()
+
+
+@pytest.mark.parametrize("H,W", [(2, 2), (34, 66), (100, 40), (96, 32)])
+@pytest.mark.parametrize("C", [3, 4, 6])
+def test_pyramid_sizes(H, W, C):
+    torch_dev()
+    from diffrast import DiffRast
+    tex = np.random.default_rng(C).random((2, H, W, C)).astype(np.float32)
+    got, ref = DiffRast.textureConstructMip(dev(tex)), O.textureConstructMip(tex)
+    assert len(got) == len(ref)
+    for a, b in zip(got, ref):
+        np.testing.assert_array_equal(host(a), b)
