@@ -126,6 +126,20 @@ __device__ __forceinline__ Bilin bilin(float u, float v, int Wk, int Hk, int mod
   return b;
 }
 
+// The nearest texel as a one-tap footprint (Texture.swift:555-571).
+__device__ __forceinline__ Bilin nearest_tap(float u, float v, int Wk, int Hk, int mode) {
+  Bilin b;
+  float ox, oy;
+  b.tx0 = f2i(floorf(u * (float)Wk));
+  b.ty0 = f2i(floorf(v * (float)Hk));
+  b.ix0 = b.ix1 = apply_boundary(b.tx0, Wk, mode, ox);
+  b.iy0 = b.iy1 = apply_boundary(b.ty0, Hk, mode, oy);
+  b.fx = b.fy = 0.0f;
+  b.w00 = b.m00 = b.m10 = b.m01 = b.m11 = (1.0f - ox) * (1.0f - oy);
+  b.w10 = b.w01 = b.w11 = 0.0f;
+  return b;
+}
+
 // Texture.swift:616-672: cube face + clamped bilinear footprint.
 __device__ __forceinline__ int cube_bilin(float x, float y, float z, int Wt, int Ht, Bilin& b) {
   const float ax = fabsf(x), ay = fabsf(y), az = fabsf(z);
@@ -228,6 +242,7 @@ __device__ __forceinline__ void tex_fwd_px(
     int64_t tex_stride, int Ht, int Wt, int C_, const float* __restrict__ uv,
     const float* __restrict__ uv_da, const float* __restrict__ bias_map, float scale_bias,
     int has_bias, int boundary, int64_t P, int n, float* __restrict__ out, int64_t pix) {
+  static_assert(CT >= 1 && CT <= kMaxC, "more channels: k_tex_fwd_many");
   if (pix >= P) return;
   const int C = dimC<CT>(C_);
   float* o = out + pix * C;
@@ -260,24 +275,14 @@ __device__ __forceinline__ void tex_fwd_px(
   if (FILTER == DR_FILTER_LINEAR) {  // Texture.swift:359-403
     const Bilin b = bilin(uvp.x, uvp.y, Wt, Ht, boundary);
     const float* tb = tex + n * tex_stride;
-    if (CT > 0) {
-      float t00[kMaxC], t10[kMaxC], t01[kMaxC], t11[kMaxC];
-      load_texel<CT>(tb + ((int64_t)b.iy0 * Wt + b.ix0) * C, C, t00);
-      load_texel<CT>(tb + ((int64_t)b.iy0 * Wt + b.ix1) * C, C, t10);
-      load_texel<CT>(tb + ((int64_t)b.iy1 * Wt + b.ix0) * C, C, t01);
-      load_texel<CT>(tb + ((int64_t)b.iy1 * Wt + b.ix1) * C, C, t11);
+    float t00[kMaxC], t10[kMaxC], t01[kMaxC], t11[kMaxC];
+    load_texel<CT>(tb + ((int64_t)b.iy0 * Wt + b.ix0) * C, C, t00);
+    load_texel<CT>(tb + ((int64_t)b.iy0 * Wt + b.ix1) * C, C, t10);
+    load_texel<CT>(tb + ((int64_t)b.iy1 * Wt + b.ix0) * C, C, t01);
+    load_texel<CT>(tb + ((int64_t)b.iy1 * Wt + b.ix1) * C, C, t11);
 #pragma unroll
-      for (int c = 0; c < (CT > 0 ? CT : 1); ++c)
-        o[c] = b.w00 * t00[c] + b.w10 * t10[c] + b.w01 * t01[c] + b.w11 * t11[c];
-    } else {
-      for (int c = 0; c < C; ++c) {
-        const float t00 = tb[((int64_t)b.iy0 * Wt + b.ix0) * C + c];
-        const float t10 = tb[((int64_t)b.iy0 * Wt + b.ix1) * C + c];
-        const float t01 = tb[((int64_t)b.iy1 * Wt + b.ix0) * C + c];
-        const float t11 = tb[((int64_t)b.iy1 * Wt + b.ix1) * C + c];
-        o[c] = b.w00 * t00 + b.w10 * t10 + b.w01 * t01 + b.w11 * t11;
-      }
-    }
+    for (int c = 0; c < CT; ++c)
+      o[c] = b.w00 * t00[c] + b.w10 * t10[c] + b.w01 * t01[c] + b.w11 * t11[c];
     return;
   }
   // Mip filters (Texture.swift:795-863).
@@ -286,54 +291,35 @@ __device__ __forceinline__ void tex_fwd_px(
   if (bias_map || has_bias) da = make_float4(da.x * s, da.y * s, da.z * s, da.w * s);
   const Lod ld = mip_lod(da, Ht, Wt, md.L, FILTER == DR_FILTER_LINEAR_MIPMAP_LINEAR);
   const bool shared = tex_stride == 0;
-  if constexpr (CT > 0) {  // texels as vectors, the sum in registers
-    float acc[CT];
+  // texels as vectors, the sum in registers
+  float acc[CT];
 #pragma unroll
-    for (int li = 0; li < 2; ++li) {
-      // a zero weight adds +0 to every channel: the second level is not read
-      // (the result differs only for non-finite texels, where 0 * inf is NaN)
-      if (li == 1 && ld.frac == 0.0f) break;
-      const int k = li == 0 ? ld.k0 : ld.k1;
-      const int Hk = mip_h(md, k), Wk = mip_w(md, k);
-      const float* lv = k == 0 ? tex + n * tex_stride
-                               : pyr + mip_off(md, k) + (shared ? 0 : (int64_t)n * Hk * Wk * C);
-      const Bilin b = bilin(uvp.x, uvp.y, Wk, Hk, boundary);
-      const float wgt = li == 0 ? (1.0f - ld.frac) : ld.frac;
-      float t00[kMaxC], t10[kMaxC], t01[kMaxC], t11[kMaxC];
-      load_texel<CT>(lv + ((int64_t)b.iy0 * Wk + b.ix0) * C, C, t00);
-      load_texel<CT>(lv + ((int64_t)b.iy0 * Wk + b.ix1) * C, C, t10);
-      load_texel<CT>(lv + ((int64_t)b.iy1 * Wk + b.ix0) * C, C, t01);
-      load_texel<CT>(lv + ((int64_t)b.iy1 * Wk + b.ix1) * C, C, t11);
-#pragma unroll
-      for (int c = 0; c < CT; ++c) {
-        const float sample = b.w00 * t00[c] + b.w10 * t10[c] + b.w01 * t01[c] + b.w11 * t11[c];
-        acc[c] = li == 0 ? wgt * sample : acc[c] + wgt * sample;  // two roundings, as :855 / :858
-      }
-    }
-    if constexpr (CT == 4) {
-      *reinterpret_cast<float4*>(o) = make_float4(acc[0], acc[1], acc[2], acc[3]);
-    } else {
-#pragma unroll
-      for (int c = 0; c < CT; ++c) o[c] = acc[c];
-    }
-    return;
-  }
   for (int li = 0; li < 2; ++li) {
+    // a zero weight adds +0 to every channel: the second level is not read
+    // (the result differs only for non-finite texels, where 0 * inf is NaN)
+    if (li == 1 && ld.frac == 0.0f) break;
     const int k = li == 0 ? ld.k0 : ld.k1;
     const int Hk = mip_h(md, k), Wk = mip_w(md, k);
     const float* lv = k == 0 ? tex + n * tex_stride
                              : pyr + mip_off(md, k) + (shared ? 0 : (int64_t)n * Hk * Wk * C);
     const Bilin b = bilin(uvp.x, uvp.y, Wk, Hk, boundary);
     const float wgt = li == 0 ? (1.0f - ld.frac) : ld.frac;
-    for (int c = 0; c < C; ++c) {
-      const float t00 = lv[((int64_t)b.iy0 * Wk + b.ix0) * C + c];
-      const float t10 = lv[((int64_t)b.iy0 * Wk + b.ix1) * C + c];
-      const float t01 = lv[((int64_t)b.iy1 * Wk + b.ix0) * C + c];
-      const float t11 = lv[((int64_t)b.iy1 * Wk + b.ix1) * C + c];
-      const float sample = b.w00 * t00 + b.w10 * t10 + b.w01 * t01 + b.w11 * t11;
-      if (li == 0) o[c] = wgt * sample;  // two roundings, as :855 / :858
-      else o[c] = o[c] + wgt * sample;
+    float t00[kMaxC], t10[kMaxC], t01[kMaxC], t11[kMaxC];
+    load_texel<CT>(lv + ((int64_t)b.iy0 * Wk + b.ix0) * C, C, t00);
+    load_texel<CT>(lv + ((int64_t)b.iy0 * Wk + b.ix1) * C, C, t10);
+    load_texel<CT>(lv + ((int64_t)b.iy1 * Wk + b.ix0) * C, C, t01);
+    load_texel<CT>(lv + ((int64_t)b.iy1 * Wk + b.ix1) * C, C, t11);
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+      const float sample = b.w00 * t00[c] + b.w10 * t10[c] + b.w01 * t01[c] + b.w11 * t11[c];
+      acc[c] = li == 0 ? wgt * sample : acc[c] + wgt * sample;  // two roundings, as :855 / :858
     }
+  }
+  if constexpr (CT == 4) {
+    *reinterpret_cast<float4*>(o) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+  } else {
+#pragma unroll
+    for (int c = 0; c < CT; ++c) o[c] = acc[c];
   }
 }
 
@@ -812,8 +798,8 @@ __global__ void __launch_bounds__(256) k_tex_bwd(TexBwdArgs A, int total_tiles) 
 }
 
 // ---------------------------------------------------------------------------
-// Windowed backward for the sampled filters (linear, linear-mipmap-*), C in
-// 1..4.  Per 16x16 pixel tile the texel bounding box of the footprints on
+// Windowed backward, C in 1..4: every 2D filter, and bilinear cube maps (a
+// face in the place of a level).  Per 16x16 pixel tile the texel bounding box of the footprints on
 // each level in use is taken, and contributions are summed into dense fp64
 // LDS windows over those boxes (direct indexing, no hashing; the windows
 // share one pool).  The windows are written out row by row, so consecutive
@@ -823,7 +809,9 @@ __global__ void __launch_bounds__(256) k_tex_bwd(TexBwdArgs A, int total_tiles) 
 // memory a texel row at a time.  Before, such taps went through a small LDS
 // hash table and mostly from there to one device atomic per value (bilinear,
 // 4 x 1000^2 x 3 at 1-3 texels a pixel: 960 us, now 189; at 8 x 1024^2
-// trilinear with 1.3% of them, no change: 238 us).
+// trilinear with 1.3% of them, no change: 238 us).  Cube maps and the nearest
+// filter took the 512-entry hash table for all taps (cube, 4 x 800^2 x 3:
+// 94 us, now 49; nearest, 4 x 800 x 700 x 4: 86, now 49).
 // ---------------------------------------------------------------------------
 
 constexpr int kWinWaves = 4;                  // waves per workgroup; a tile is 16 x (4 * kWinWaves) pixels
@@ -837,7 +825,8 @@ constexpr int kWinThreads = 64 * kWinWaves;
 // backward 338 -> 289 us against 768, before the bands).
 template <int FILTER, int CT>
 constexpr int win_texels() {
-  return FILTER == DR_FILTER_LINEAR && CT < 4 ? 1008 : 232 * kWinWaves;
+  return (FILTER == DR_FILTER_LINEAR || FILTER == DR_FILTER_NEAREST) && CT < 4 ? 1008
+                                                                              : 232 * kWinWaves;
 }
 
 // Most bands of a box larger than the pool (bilinear): 289 -> 218 us at the
@@ -923,6 +912,9 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
 
   const MipDesc& md = A.md;
   const bool mip = FILTER == DR_FILTER_LINEAR_MIPMAP_LINEAR || FILTER == DR_FILTER_LINEAR_MIPMAP_NEAREST;
+  constexpr bool kCube = BND == DR_BOUNDARY_CUBE;
+  constexpr bool kSameUv = BND == DR_BOUNDARY_WRAP || FILTER == DR_FILTER_NEAREST;
+  constexpr bool kOneLevel = kCube || FILTER == DR_FILTER_NEAREST || FILTER == DR_FILTER_LINEAR;
   const bool shared_tex = A.tex_stride == 0;
   const int wave = tid >> 6, lane = tid & 63;
   const int tiles = A.ntx * A.nty;
@@ -953,11 +945,15 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
     const int ph = ty * (4 * kWinWaves) + wave * 4 + (lane >> 4);
     const bool valid = pw < A.Wi && ph < A.Hi;
     const int64_t pix = ((int64_t)n * A.Hi + min(ph, A.Hi - 1)) * A.Wi + min(pw, A.Wi - 1);
+    // cube maps: k is the face, one level each
+    auto level_w = [&](int k) { return kOneLevel ? A.Wt : mip_w(md, k); };
+    auto level_h = [&](int k) { return kOneLevel ? A.Ht : mip_h(md, k); };
     auto level_ptr = [&](int k) -> const float* {
       return k == 0 ? A.tex + n * A.tex_stride
                     : A.pyr + mip_off(md, k) + (shared_tex ? 0 : (int64_t)n * mip_h(md, k) * mip_w(md, k) * CT);
     };
     auto dlevel_ptr = [&](int k) -> float* {
+      if (kCube) return A.d_tex + n * A.tex_stride + (int64_t)k * A.Ht * A.Wt * CT;
       return k == 0 ? A.d_tex + n * A.tex_stride
                     : A.d_pyr + mip_off(md, k) + (shared_tex ? 0 : (int64_t)n * mip_h(md, k) * mip_w(md, k) * CT);
     };
@@ -972,7 +968,15 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
     }
 #pragma unroll
     for (int c = 0; c < CT; ++c) g[c] = valid ? g[c] : 0.0f;
-    const float2 uvp = ld_nt2(A.uv + pix * 2);
+    float2 uvp = make_float2(0.0f, 0.0f);
+    Bilin cb;
+    int face = 0;
+    if (kCube) {
+      const float* d = A.uv + pix * 3;
+      face = cube_bilin(d[0], d[1], d[2], A.Wt, A.Ht, cb);
+    } else {
+      uvp = ld_nt2(A.uv + pix * 2);
+    }
     TapSlot q[2];
     float4 da_in = make_float4(0.f, 0.f, 0.f, 0.f), da = da_in;
     float s = 1.0f;
@@ -998,7 +1002,7 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
       need1 = ld.frac != 0.0f || (FILTER == DR_FILTER_LINEAR_MIPMAP_LINEAR && ld.k0 != 0);
       lod0 = FILTER != DR_FILTER_LINEAR_MIPMAP_LINEAR || (ld.k0 == 0 && ld.frac == 0.0f);
     } else {
-      q[0].k = 0;
+      q[0].k = face;
       q[0].scale = 1.0f;
       q[1].k = 0;
       q[1].scale = 0.0f;
@@ -1013,8 +1017,10 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
         q[1].w00 = q[1].w10 = q[1].w01 = q[1].w11 = 0.0f;
         continue;
       }
-      const int k = q[li].k, Hk = mip_h(md, k), Wk = mip_w(md, k);
-      const Bilin b = bilin(uvp.x, uvp.y, Wk, Hk, BND);
+      const int k = q[li].k, Hk = level_h(k), Wk = level_w(k);
+      const Bilin b = kCube ? cb
+                      : FILTER == DR_FILTER_NEAREST ? nearest_tap(uvp.x, uvp.y, Wk, Hk, BND)
+                                                    : bilin(uvp.x, uvp.y, Wk, Hk, BND);
       float w00 = b.w00, w10 = b.w10, w01 = b.w01, w11 = b.w11;
       if (b.ix1 == b.ix0) { w00 += w10; w01 += w11; w10 = 0.0f; w11 = 0.0f; }
       if (b.iy1 == b.iy0) { w00 += w01; w10 += w11; w01 = 0.0f; w11 = 0.0f; }
@@ -1031,15 +1037,22 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
       // background pixel) has zero texel differences: its uv gradient is
       // zero and, at LOD 0, its sample is not needed.
       const bool flat = BND != DR_BOUNDARY_ZERO && b.ix0 == b.ix1 && b.iy0 == b.iy1 && lod0;
-      if (valid && (li == 0 || need1) && !flat) {
+      if (!kCube && FILTER != DR_FILTER_NEAREST && valid && (li == 0 || need1) && !flat) {
         float dfx, dfy;
         duv_level<uint32_t>(level_ptr(k), Wk, CT, b, g, mip ? q[li].scale : 1.0f, dfx, dfy, samp[li]);
         dfx_total += dfx * (float)Wk;
         dfy_total += dfy * (float)Hk;
       }
     }
-    if (valid && A.d_uv)
-      st_nt2(A.d_uv + pix * 2, make_float2(dfx_total, dfy_total));
+    if (valid && A.d_uv) {  // (cube and nearest: zero, Texture.swift:196-198, :234)
+      if (kCube) {
+        A.d_uv[pix * 3 + 0] = 0.0f;
+        A.d_uv[pix * 3 + 1] = 0.0f;
+        A.d_uv[pix * 3 + 2] = 0.0f;
+      } else {
+        st_nt2(A.d_uv + pix * 2, make_float2(dfx_total, dfy_total));
+      }
+    }
     if (mip && valid && (A.d_uv_da || A.d_bias)) {  // Texture.swift:1011-1102
       const float sx = da.x * (float)A.Wt, sy = da.y * (float)A.Wt;
       const float tx_ = da.z * (float)A.Ht, ty_ = da.w * (float)A.Ht;
@@ -1086,7 +1099,7 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
     bool hot = false;
     {
       const bool on0 = q[0].w00 != 0.0f || q[0].w10 != 0.0f || q[0].w01 != 0.0f || q[0].w11 != 0.0f;
-      const int Wk = mip_w(md, q[0].k);
+      const int Wk = level_w(q[0].k);
       const uint64_t key = ((uint64_t)q[0].k << 48) | (uint64_t)((int64_t)q[0].iy0 * Wk + q[0].ix0);
       const uint32_t key2 = ((uint32_t)(q[0].ix1 - q[0].ix0) << 16) ^ (uint32_t)(q[0].iy1 - q[0].iy0);
       // flat footprints only (all the weight on one texel: every background
@@ -1102,8 +1115,9 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
       // of weights, so the group's cotangents are summed and then weighted
       // (4 x 1000^2 x 3, bilinear, 55% of the pixels empty: 960 -> 92 us with
       // the windows' unwrapped coordinates).
+      // The nearest filter's footprints are all one texel: grouped by uv too.
       bool flat;
-      if (BND == DR_BOUNDARY_WRAP) {
+      if (kSameUv) {
         const int ux = __float_as_int(uvp.x), uy = __float_as_int(uvp.y);
         // (every lane executes the shifts)
         const int lx = dpp_shift<0x111>(ux), ly = dpp_shift<0x111>(uy);
@@ -1122,7 +1136,7 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
                               (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)key, leader);
         const uint32_t lkey2 = (uint32_t)__builtin_amdgcn_readlane((int)key2, leader);
         bool same;
-        if (BND == DR_BOUNDARY_WRAP)
+        if (kSameUv)
           same = flat && !hot && q[0].k == __builtin_amdgcn_readlane(q[0].k, leader) &&
                  __float_as_int(uvp.x) == __builtin_amdgcn_readlane(__float_as_int(uvp.x), leader) &&
                  __float_as_int(uvp.y) == __builtin_amdgcn_readlane(__float_as_int(uvp.y), leader);
@@ -1132,9 +1146,9 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
         pending &= ~members;
         const int lk = __builtin_amdgcn_readlane(q[0].k, leader);
         float* base = dlevel_ptr(lk);
-        const int lW = mip_w(md, lk);
+        const int lW = level_w(lk);
         float* lp[4];
-        const int lH = mip_h(md, lk);
+        const int lH = level_h(lk);
         const int lix0 = win_texel<BND>(__builtin_amdgcn_readlane(q[0].ix0, leader), lW);
         const int lix1 = win_texel<BND>(__builtin_amdgcn_readlane(q[0].ix1, leader), lW);
         const int liy0 = win_texel<BND>(__builtin_amdgcn_readlane(q[0].iy0, leader), lH);
@@ -1158,11 +1172,11 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
           const float gc = g[c < CT ? c : 0] * q[0].scale;
-          x[c] = (c < CT && same) ? (BND == DR_BOUNDARY_WRAP ? gc : q[0].w00 * gc) : 0.0f;
+          x[c] = (c < CT && same) ? (kSameUv ? gc : q[0].w00 * gc) : 0.0f;
         }
         const float z = wave_sum4(x);  // lane l: total of value l & 3
         const float zc = __shfl(z, (lane >> 2) & 3, kWave);
-        if (BND == DR_BOUNDARY_WRAP) {  // lane 4c + t: channel c, tap t
+        if (kSameUv) {  // lane 4c + t: channel c, tap t
           const float wt = leader_weight(q[0], leader, lane & 3);
           if (lane < 4 * CT) acc.v += wt * zc;
         } else {
@@ -1310,7 +1324,7 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
     // at `at` in the pool, added to the level and cleared.
     auto flush_window = [&](int k, int x0, int y0, int bw, int bh, int at) {
       float* base = dlevel_ptr(k);
-      const int Wk = mip_w(md, k), Hk = mip_h(md, k);
+      const int Wk = level_w(k), Hk = level_h(k);
       // (wrap mode: the first texel reduced into the texture; a window's
       // later columns and rows wrap from there)
       const int bx0 = win_texel<BND>(x0, Wk), by0 = win_texel<BND>(y0, Hk);
@@ -1360,7 +1374,7 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
     //    few texels a pixel) goes through it in bands of whole rows: a band's
     //    rows share cache-line requests, where the direct way below costs two
     //    requests a pixel whatever the box
-    if (!mip && nowin != 0) {  // uniform: level 0 alone is in use
+    if (!mip && !kCube && nowin != 0) {  // uniform: level 0 alone is in use
       int px = pack16(32767, 32767), py = px;
 #pragma unroll
       for (int w = 0; w < kWinWaves; ++w) {
@@ -1423,7 +1437,7 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
         if (__ballot(u) == 0) continue;
         float v[4 * CT];
         const bool adds = run_totals(li, u, v);
-        const int Wk = mip_w(md, k), Hk = mip_h(md, k);
+        const int Wk = level_w(k), Hk = level_h(k);
         const int X0 = win_texel<BND>(q[li].ix0, Wk), X1 = win_texel<BND>(q[li].ix1, Wk);
         const int Y0 = win_texel<BND>(q[li].iy0, Hk), Y1 = win_texel<BND>(q[li].iy1, Hk);
         float* const lv = dlevel_ptr(k);
@@ -1692,21 +1706,9 @@ __global__ void __launch_bounds__(256, 3) k_tex_bwd_many(TexBwdArgs A, int total
 #pragma unroll
     for (int li = 0; li < (mip ? 2 : 1); ++li) {
       const int k = q[li].k, Hk = level_h(k), Wk = level_w(k);
-      Bilin b;
-      if (kCube) {
-        b = cb;
-      } else if (FILTER == DR_FILTER_NEAREST) {  // one tap (Texture.swift:576-605)
-        float ox, oy;
-        b.tx0 = f2i(floorf(uvp.x * (float)Wk));
-        b.ty0 = f2i(floorf(uvp.y * (float)Hk));
-        b.ix0 = b.ix1 = apply_boundary(b.tx0, Wk, BND, ox);
-        b.iy0 = b.iy1 = apply_boundary(b.ty0, Hk, BND, oy);
-        b.fx = b.fy = 0.0f;
-        b.w00 = b.m00 = b.m10 = b.m01 = b.m11 = (1.0f - ox) * (1.0f - oy);
-        b.w10 = b.w01 = b.w11 = 0.0f;
-      } else {
-        b = bilin(uvp.x, uvp.y, Wk, Hk, BND);
-      }
+      const Bilin b = kCube ? cb
+                      : FILTER == DR_FILTER_NEAREST ? nearest_tap(uvp.x, uvp.y, Wk, Hk, BND)
+                                                    : bilin(uvp.x, uvp.y, Wk, Hk, BND);
       float w00 = b.w00, w10 = b.w10, w01 = b.w01, w11 = b.w11;
       if (b.ix1 == b.ix0) { w00 += w10; w01 += w11; w10 = 0.0f; w11 = 0.0f; }
       if (b.iy1 == b.iy0) { w00 += w01; w10 += w11; w01 = 0.0f; w11 = 0.0f; }
@@ -2278,8 +2280,10 @@ hipError_t launch_tex_bwd_win_bb(const TexBwdArgs& args, int total_tiles, hipStr
 
 template <int FILTER, int CT, int BND>
 hipError_t launch_tex_bwd_win_b(const TexBwdArgs& args, int total_tiles, hipStream_t stream) {
-  if (args.bias_map || args.has_bias)
-    return launch_tex_bwd_win_bb<FILTER, CT, BND, true>(args, total_tiles, stream);
+  if constexpr (FILTER == DR_FILTER_LINEAR_MIPMAP_NEAREST || FILTER == DR_FILTER_LINEAR_MIPMAP_LINEAR) {
+    if (args.bias_map || args.has_bias)
+      return launch_tex_bwd_win_bb<FILTER, CT, BND, true>(args, total_tiles, stream);
+  }
   return launch_tex_bwd_win_bb<FILTER, CT, BND, false>(args, total_tiles, stream);
 }
 
@@ -3172,8 +3176,7 @@ static int texture_bwd(const float* tex, const float* pyramid, int Nt, int Ht, i
     case 3: e = launch_tex_bwd_win<F, 3>(wargs, wtiles, stream); break; \
     default: e = launch_tex_bwd_win<F, 4>(wargs, wtiles, stream); break; \
   }
-    const bool windowed = !cube && filter != DR_FILTER_NEAREST && C >= 1 && C <= 4 &&
-                          Wt <= 32767 && Ht <= 32767;  // window boxes use 16-bit texel coordinates
+    const bool windowed = C <= 4 && Wt <= 32767 && Ht <= 32767;  // window boxes use 16-bit texel coordinates
     // more channels: while the empty pixels' sums have room, texel
     // coordinates fit 16 bits and a level's floats 32
     const bool many = C > 4 && C <= kManyC && Wt <= 32767 && Ht <= 32767 &&
@@ -3188,6 +3191,14 @@ static int texture_bwd(const float* tex, const float* pyramid, int Nt, int Ht, i
       e = launch_tex_bwd_many_b<DR_FILTER_LINEAR_MIPMAP_NEAREST>(args, (int)total_tiles, stream);
     else if (many)
       e = launch_tex_bwd_many_b<DR_FILTER_LINEAR_MIPMAP_LINEAR>(args, (int)total_tiles, stream);
+    else if (windowed && cube)
+      switch (C) {
+        case 1: e = launch_tex_bwd_win_bb<DR_FILTER_LINEAR, 1, DR_BOUNDARY_CUBE, false>(wargs, wtiles, stream); break;
+        case 2: e = launch_tex_bwd_win_bb<DR_FILTER_LINEAR, 2, DR_BOUNDARY_CUBE, false>(wargs, wtiles, stream); break;
+        case 3: e = launch_tex_bwd_win_bb<DR_FILTER_LINEAR, 3, DR_BOUNDARY_CUBE, false>(wargs, wtiles, stream); break;
+        default: e = launch_tex_bwd_win_bb<DR_FILTER_LINEAR, 4, DR_BOUNDARY_CUBE, false>(wargs, wtiles, stream); break;
+      }
+    else if (windowed && filter == DR_FILTER_NEAREST) DR_TW(DR_FILTER_NEAREST)
     else if (windowed && filter == DR_FILTER_LINEAR) DR_TW(DR_FILTER_LINEAR)
     else if (windowed && filter == DR_FILTER_LINEAR_MIPMAP_NEAREST) DR_TW(DR_FILTER_LINEAR_MIPMAP_NEAREST)
     else if (windowed) DR_TW(DR_FILTER_LINEAR_MIPMAP_LINEAR)

@@ -56,7 +56,8 @@ def check(rng, tex, uv, da, filt, bnd, rtol=1e-4, bias=None):
 @pytest.mark.parametrize("Ht,Wt", [(1, 1), (1, 7), (5, 3), (40, 72), (512, 256)])
 @pytest.mark.parametrize("offset,background", [(0.0, (0.0, 0.0)), (-3.5, (0.3, 0.7)),
                                                (40000.0, (0.0, 0.0))])
-@pytest.mark.parametrize("filt,C", [("linear", 1), ("linear", 3), ("linear-mipmap-linear", 4)])
+@pytest.mark.parametrize("filt,C", [("linear", 1), ("linear", 3), ("linear-mipmap-linear", 4),
+                                    ("nearest", 2)])
 def test_wrap_windows(Ht, Wt, offset, background, filt, C):
     torch_dev()
     rng = np.random.default_rng(Ht * 1000 + Wt + C)
@@ -69,7 +70,7 @@ def test_wrap_windows(Ht, Wt, offset, background, filt, C):
 # over several bands (2 to 4) to the direct way (12); C = 4 has a smaller pool
 @pytest.mark.parametrize("texels", [0.5, 2.0, 3.0, 4.0, 12.0])
 @pytest.mark.parametrize("bnd", ["wrap", "clamp", "zero"])
-@pytest.mark.parametrize("filt,C", [("linear", 1), ("linear", 3), ("linear", 4),
+@pytest.mark.parametrize("filt,C", [("linear", 1), ("linear", 3), ("linear", 4), ("nearest", 3),
                                     ("linear-mipmap-linear", 2)])
 def test_minified_boxes(texels, bnd, filt, C):
     torch_dev()
@@ -102,8 +103,8 @@ def test_many_channels(C, filt, bnd, Nt, texels):
     check(rng, tex, uv, da, filt, bnd, bias=0.3 if "mipmap" in filt else None)
 
 
-@pytest.mark.parametrize("C", [6, 9])
-def test_many_channels_cube(C):
+@pytest.mark.parametrize("C", [1, 3, 4, 6, 9])
+def test_smooth_cube(C):
     torch_dev()
     from diffrast import DiffRast
     rng = np.random.default_rng(C)
