@@ -250,6 +250,26 @@ __device__ __forceinline__ void st_nt2(float* p, float2 v) {
   __builtin_nontemporal_store(x, reinterpret_cast<dr_f2v*>(p));
 }
 
+// Four values from p, the first nc of them in memory (nc = 4: one load
+// whatever p's alignment; the hardware takes 4-byte aligned vectors).
+typedef float dr_f4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ float4 ld_chunk(const float* __restrict__ p, int nc) {
+  if (nc == 4) {
+    const dr_f4u v = *reinterpret_cast<const dr_f4u*>(p);
+    return make_float4(v.x, v.y, v.z, v.w);
+  }
+  return make_float4(p[0], nc > 1 ? p[1] : 0.0f, nc > 2 ? p[2] : 0.0f, 0.0f);
+}
+__device__ __forceinline__ void st_chunk(float* __restrict__ p, float4 x, int nc) {
+  if (nc == 4) {
+    dr_f4u v = {x.x, x.y, x.z, x.w};
+    *reinterpret_cast<dr_f4u*>(p) = v;
+    return;
+  }
+  p[0] = x.x;
+  if (nc > 1) p[1] = x.y;
+  if (nc > 2) p[2] = x.z;
+}
 
 // Wave-uniform values: keep them in scalar registers.
 __device__ __forceinline__ float uni(float x) {

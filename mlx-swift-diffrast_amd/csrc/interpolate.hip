@@ -23,11 +23,6 @@ namespace dr {
 // 6.3M x 3, backward 5.50 -> 4.79 ms.
 constexpr int64_t kXcdL2Bytes = 4 << 20;
 
-// Compile-time attribute / derivative counts for the common shapes; 0 means
-// "given at run time".
-template <int AT>
-__device__ __forceinline__ int dimA(int A) { return AT > 0 ? AT : A; }
-
 // Stores n consecutive floats; two or four at a time when the count and the
 // (16-byte aligned) buffers allow.
 template <int NC>
@@ -68,14 +63,12 @@ constexpr int interp_strip() {
 template <int AT, int KT>
 __global__ void __launch_bounds__(256) k_interp_fwd(
     const float* __restrict__ attr, int64_t attr_stride, const float* __restrict__ rast,
-    const float* __restrict__ rast_db, const int32_t* __restrict__ tri,
-    const int32_t* __restrict__ diff_idx, int K_, int H, int W, int ntx, int nty, int V, int T,
-    int A_, float* __restrict__ out, float* __restrict__ out_da, int xcd) {
+    const float* __restrict__ rast_db, const int32_t* __restrict__ tri, int H, int W, int ntx,
+    int nty, int V, int T, float* __restrict__ out, float* __restrict__ out_da, int xcd) {
   constexpr int PX = interp_pix<AT>();
-  constexpr int NA = AT > 0 ? AT : 8;       // register slots for attributes
-  constexpr int NK = KT > 0 ? 2 * KT : 8;   // and for derivative outputs
-  const int A = dimA<AT>(A_);
-  const int K = KT > 0 ? KT : K_;
+  static_assert(AT > 0, "other shapes: k_interp_fwd_any");
+  constexpr int NA = AT;                    // register slots for attributes
+  constexpr int NK = KT > 0 ? 2 * KT : 1;   // and for derivative outputs
   const int tiles = ntx * nty;
   const int b = xcd ? xcd_remap((int)blockIdx.x, (int)gridDim.x) : (int)blockIdx.x;
   const int img = b / tiles;
@@ -136,41 +129,6 @@ __global__ void __launch_bounds__(256) k_interp_fwd(
       iv[q][0] = iv[q][1] = iv[q][2] = 0;
     }
   }
-  if (AT == 0 || KT == 0 && K > 0) {  // any shape: element by element
-#pragma unroll
-    for (int q = 0; q < PX; ++q) {
-      const int64_t pix = pixq[q];
-      if (!in[q]) continue;
-      float* o = out + pix * A;
-      float* od = K > 0 ? out_da + pix * 2 * K : nullptr;
-      if (t[q] < 0) {
-        for (int a = 0; a < A; ++a) o[a] = 0.0f;
-        for (int k = 0; k < 2 * K; ++k) od[k] = 0.0f;
-        continue;
-      }
-      const float* a0p = at + (int64_t)iv[q][0] * A;
-      const float* a1p = at + (int64_t)iv[q][1] * A;
-      const float* a2p = at + (int64_t)iv[q][2] * A;
-      const float u = r[q].x, v = r[q].y;
-      const float bw = 1.0f - u - v;
-      for (int a = 0; a < A; ++a) o[a] = bw * a0p[a] + u * a1p[a] + v * a2p[a];
-      if (K > 0) {
-        const float4 db = *reinterpret_cast<const float4*>(rast_db + pix * 4);
-        for (int k = 0; k < K; ++k) {
-          const int a = diff_idx ? diff_idx[k] : k;
-          if ((unsigned)a >= (unsigned)A) {  // not an attribute: zero derivatives
-            od[2 * k + 0] = od[2 * k + 1] = 0.0f;
-            continue;
-          }
-          const float d01 = a1p[a] - a0p[a];
-          const float d02 = a2p[a] - a0p[a];
-          od[2 * k + 0] = d01 * db.x + d02 * db.z;
-          od[2 * k + 1] = d01 * db.y + d02 * db.w;
-        }
-      }
-    }
-    return;
-  }
   // compile-time shape (identity diff_idx when KT > 0)
   bool rows = false;
 #pragma unroll
@@ -223,6 +181,74 @@ __global__ void __launch_bounds__(256) k_interp_fwd(
   }
 }
 
+// Any other shape: attributes in chunks of four, a thread per (pixel, chunk)
+// with consecutive threads on consecutive chunks, so a vertex row's reads and
+// a pixel's writes are runs of memory; the derivatives of a pixel's K chosen
+// attributes (diff_idx, or all) go to its threads in turn.  One thread per
+// pixel walking its attributes one by one read and wrote four bytes a lane
+// at a stride of A floats (4 x 720 x 1280, A = 8, K = 2: 126 us, now
+// 70).
+__global__ void __launch_bounds__(256) k_interp_fwd_any(
+    const float* __restrict__ attr, int64_t attr_stride, const float* __restrict__ rast,
+    const float* __restrict__ rast_db, const int32_t* __restrict__ tri,
+    const int32_t* __restrict__ diff_idx, int K, int H, int W, int ntx, int nty, int V, int T,
+    int A, float* __restrict__ out, float* __restrict__ out_da, int xcd) {
+  const int tiles = ntx * nty;
+  const int b = xcd ? xcd_remap((int)blockIdx.x, (int)gridDim.x) : (int)blockIdx.x;
+  const int img = b / tiles;
+  const int tile = b - img * tiles;
+  const int ty = tile / ntx, tx = tile - ty * ntx;
+  const int G = (A + 3) >> 2;
+  const float* at = attr + (int64_t)img * attr_stride;
+  for (int i = (int)threadIdx.x; i < 256 * G; i += 256) {
+    const int lp = i / G, g = i - lp * G, a = g * 4;
+    const int pw = tx * 16 + (lp & 15), ph = ty * 16 + (lp >> 4);
+    if (pw >= W || ph >= H) continue;
+    const int64_t pix = ((int64_t)img * H + ph) * W + pw;
+    const int na = min(4, A - a);
+    const float4 r = *reinterpret_cast<const float4*>(rast + pix * 4);
+    int t = f2i(r.w) - 1;
+    int i0 = 0, i1 = 0, i2 = 0;
+    if ((unsigned)t < (unsigned)T) {
+      i0 = tri[t * 3 + 0];
+      i1 = tri[t * 3 + 1];
+      i2 = tri[t * 3 + 2];
+    } else {
+      t = -1;  // not a triangle of this mesh: empty
+    }
+    float* o = out + pix * A + a;
+    if (t < 0 || !verts_ok(i0, i1, i2, V)) {
+      st_chunk(o, make_float4(0.f, 0.f, 0.f, 0.f), na);
+      for (int k = g; k < K; k += G) {
+        out_da[pix * 2 * K + 2 * k + 0] = 0.0f;
+        out_da[pix * 2 * K + 2 * k + 1] = 0.0f;
+      }
+      continue;
+    }
+    const float* r0 = at + (int64_t)i0 * A;
+    const float* r1 = at + (int64_t)i1 * A;
+    const float* r2 = at + (int64_t)i2 * A;
+    const float4 x = ld_chunk(r0 + a, na), y = ld_chunk(r1 + a, na), z = ld_chunk(r2 + a, na);
+    const float u = r.x, v = r.y;
+    const float bw = 1.0f - u - v;
+    st_chunk(o, make_float4(bw * x.x + u * y.x + v * z.x, bw * x.y + u * y.y + v * z.y,
+                            bw * x.z + u * y.z + v * z.z, bw * x.w + u * y.w + v * z.w), na);
+    if (g >= K) continue;
+    const float4 db = *reinterpret_cast<const float4*>(rast_db + pix * 4);
+    for (int k = g; k < K; k += G) {
+      const int q = diff_idx ? diff_idx[k] : k;
+      float2 d = make_float2(0.0f, 0.0f);  // not an attribute: zero derivatives
+      if ((unsigned)q < (unsigned)A) {
+        const float a0 = r0[q];
+        const float d01 = r1[q] - a0, d02 = r2[q] - a0;
+        d = make_float2(d01 * db.x + d02 * db.z, d01 * db.y + d02 * db.w);
+      }
+      out_da[pix * 2 * K + 2 * k + 0] = d.x;
+      out_da[pix * 2 * K + 2 * k + 1] = d.y;
+    }
+  }
+}
+
 // Fused backward.  Pixels are walked in 16x16 tiles, a 16x4 strip per wave;
 // runs of one triangle along a pixel row are summed before their d_attr
 // terms meet the LDS table.
@@ -230,11 +256,11 @@ template <int AT, int KT>
 __global__ void __launch_bounds__(256) k_interp_bwd(
     const float* __restrict__ attr, int64_t attr_stride, const float* __restrict__ rast,
     const float* __restrict__ rast_db, const int32_t* __restrict__ tri,
-    const int32_t* __restrict__ diff_idx, int K_, const float* __restrict__ d_out,
-    const float* __restrict__ d_out_da, int N, int H, int W, int ntx, int nty, int V, int T,
-    int A_, float* __restrict__ d_attr, int64_t d_attr_stride, int ncopy, int64_t copy_stride,
-    float* __restrict__ d_rast, float* __restrict__ d_rast_db, int xcd) {
-  __shared__ LdsTableU<(AT > 0 ? AT : 1), 256> tab;  // d_attr rows (or elements) touched by this tile
+    const float* __restrict__ d_out, const float* __restrict__ d_out_da, int H, int W, int ntx,
+    int nty, int V, int T, float* __restrict__ d_attr, int64_t d_attr_stride, int ncopy,
+    int64_t copy_stride, float* __restrict__ d_rast, float* __restrict__ d_rast_db, int xcd) {
+  static_assert(AT > 0, "other shapes: k_interp_bwd_any");
+  __shared__ LdsTableU<AT, 256> tab;  // d_attr rows touched by this tile
   __shared__ int s_any[4];  // per wave: a covered pixel
   const int tiles = ntx * nty;
   const int b = xcd ? xcd_remap((int)blockIdx.x, (int)gridDim.x) : (int)blockIdx.x;
@@ -258,7 +284,7 @@ __global__ void __launch_bounds__(256) k_interp_bwd(
   if (!(s_any[0] | s_any[1] | s_any[2] | s_any[3])) {  // uniform: an empty tile
     if (inside) {
       *reinterpret_cast<float4*>(d_rast + pix * 4) = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (K_ > 0 && d_rast_db)
+      if (KT > 0 && d_rast_db)
         *reinterpret_cast<float4*>(d_rast_db + pix * 4) = make_float4(0.f, 0.f, 0.f, 0.f);
     }
     return;
@@ -272,161 +298,266 @@ __global__ void __launch_bounds__(256) k_interp_bwd(
   float* da = d_attr + (ncopy ? (int64_t)(b % ncopy) * copy_stride : 0) + (int64_t)n * d_attr_stride;
   int i0 = 0, i1 = 0, i2 = 0;
 
-  if constexpr (AT > 0) {
-    // Compile-time shape (identity diff_idx when KT > 0): every input of the
-    // pixel is loaded once, the cotangents and rast_db together with the
-    // triangle's vertex ids, then the three attribute rows.
-    constexpr int NK = KT > 0 ? KT : 1;
-    float gv[AT], gdv[2 * NK], a0[AT], a1[AT], a2[AT];
-    float4 db = make_float4(0.f, 0.f, 0.f, 0.f);
+  // Compile-time shape (identity diff_idx when KT > 0): every input of the
+  // pixel is loaded once, the cotangents and rast_db together with the
+  // triangle's vertex ids, then the three attribute rows.
+  constexpr int NK = KT > 0 ? KT : 1;
+  float gv[AT], gdv[2 * NK], a0[AT], a1[AT], a2[AT];
+  float4 db = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-    for (int a = 0; a < AT; ++a) gv[a] = a0[a] = a1[a] = a2[a] = 0.0f;
+  for (int a = 0; a < AT; ++a) gv[a] = a0[a] = a1[a] = a2[a] = 0.0f;
 #pragma unroll
-    for (int k = 0; k < 2 * NK; ++k) gdv[k] = 0.0f;
-    if (valid) {
-      i0 = tri[t * 3 + 0];
-      i1 = tri[t * 3 + 1];
-      i2 = tri[t * 3 + 2];
+  for (int k = 0; k < 2 * NK; ++k) gdv[k] = 0.0f;
+  if (valid) {
+    i0 = tri[t * 3 + 0];
+    i1 = tri[t * 3 + 1];
+    i2 = tri[t * 3 + 2];
 #pragma unroll
-      for (int a = 0; a < AT; ++a) gv[a] = d_out[pix * AT + a];
-      if constexpr (KT > 0) {
+    for (int a = 0; a < AT; ++a) gv[a] = d_out[pix * AT + a];
+    if constexpr (KT > 0) {
 #pragma unroll
-        for (int k = 0; k < 2 * KT; ++k) gdv[k] = d_out_da[pix * 2 * KT + k];
-        db = *reinterpret_cast<const float4*>(rast_db + pix * 4);
-      }
-      valid = verts_ok(i0, i1, i2, V);  // pixels of foreign ids are empty
+      for (int k = 0; k < 2 * KT; ++k) gdv[k] = d_out_da[pix * 2 * KT + k];
+      db = *reinterpret_cast<const float4*>(rast_db + pix * 4);
     }
-    if (valid) {
+    valid = verts_ok(i0, i1, i2, V);  // pixels of foreign ids are empty
+  }
+  if (valid) {
 #pragma unroll
-      for (int a = 0; a < AT; ++a) {
-        a0[a] = at[(int64_t)i0 * AT + a];
-        a1[a] = at[(int64_t)i1 * AT + a];
-        a2[a] = at[(int64_t)i2 * AT + a];
-      }
+    for (int a = 0; a < AT; ++a) {
+      a0[a] = at[(int64_t)i0 * AT + a];
+      a1[a] = at[(int64_t)i1 * AT + a];
+      a2[a] = at[(int64_t)i2 * AT + a];
     }
-    // d_rast (Interpolate.swift:327-367) and d_rast_db (:370-417).
-    float du = 0.0f, dv = 0.0f;
-    float d_udx = 0.0f, d_udy = 0.0f, d_vdx = 0.0f, d_vdy = 0.0f;
-    if (valid) {
+  }
+  // d_rast (Interpolate.swift:327-367) and d_rast_db (:370-417).
+  float du = 0.0f, dv = 0.0f;
+  float d_udx = 0.0f, d_udy = 0.0f, d_vdx = 0.0f, d_vdy = 0.0f;
+  if (valid) {
 #pragma unroll
-      for (int a = 0; a < AT; ++a) {
-        du += (a1[a] - a0[a]) * gv[a];
-        dv += (a2[a] - a0[a]) * gv[a];
-      }
+    for (int a = 0; a < AT; ++a) {
+      du += (a1[a] - a0[a]) * gv[a];
+      dv += (a2[a] - a0[a]) * gv[a];
+    }
 #pragma unroll
-      for (int k = 0; k < (KT > 0 ? KT : 0); ++k) {
-        const float d01 = a1[k] - a0[k], d02 = a2[k] - a0[k];
-        const float gx = gdv[2 * k + 0], gy = gdv[2 * k + 1];
-        d_udx += d01 * gx;
-        d_udy += d01 * gy;
-        d_vdx += d02 * gx;
-        d_vdy += d02 * gy;
-      }
+    for (int k = 0; k < (KT > 0 ? KT : 0); ++k) {
+      const float d01 = a1[k] - a0[k], d02 = a2[k] - a0[k];
+      const float gx = gdv[2 * k + 0], gy = gdv[2 * k + 1];
+      d_udx += d01 * gx;
+      d_udy += d01 * gy;
+      d_vdx += d02 * gx;
+      d_vdy += d02 * gy;
     }
-    if (inside) {
-      *reinterpret_cast<float4*>(d_rast + pix * 4) = make_float4(du, dv, 0.0f, 0.0f);
-      if (KT > 0 && d_rast_db)
-        *reinterpret_cast<float4*>(d_rast_db + pix * 4) = make_float4(d_udx, d_udy, d_vdx, d_vdy);
-    }
-    // d_attr (Interpolate.swift:231-264, :269-324), summed per vertex row in
-    // LDS before the global atomics.
-    float rv[3 * AT];  // rows of i0, i1, i2
+  }
+  if (inside) {
+    *reinterpret_cast<float4*>(d_rast + pix * 4) = make_float4(du, dv, 0.0f, 0.0f);
+    if (KT > 0 && d_rast_db)
+      *reinterpret_cast<float4*>(d_rast_db + pix * 4) = make_float4(d_udx, d_udy, d_vdx, d_vdy);
+  }
+  // d_attr (Interpolate.swift:231-264, :269-324), summed per vertex row in
+  // LDS before the global atomics.
+  float rv[3 * AT];  // rows of i0, i1, i2
 #pragma unroll
-    for (int q = 0; q < 3 * AT; ++q) rv[q] = 0.0f;
-    if (valid) {
+  for (int q = 0; q < 3 * AT; ++q) rv[q] = 0.0f;
+  if (valid) {
 #pragma unroll
-      for (int a = 0; a < AT; ++a) {
-        rv[a] = bw * gv[a];
-        rv[AT + a] = u * gv[a];
-        rv[2 * AT + a] = v * gv[a];
-      }
+    for (int a = 0; a < AT; ++a) {
+      rv[a] = bw * gv[a];
+      rv[AT + a] = u * gv[a];
+      rv[2 * AT + a] = v * gv[a];
+    }
 #pragma unroll
-      for (int k = 0; k < (KT > 0 ? KT : 0); ++k) {
-        const float gx = gdv[2 * k + 0], gy = gdv[2 * k + 1];
-        const float u_term = gx * db.x + gy * db.y;
-        const float v_term = gx * db.z + gy * db.w;
-        rv[k] += -u_term - v_term;
-        rv[AT + k] += u_term;
-        rv[2 * AT + k] += v_term;
-      }
+    for (int k = 0; k < (KT > 0 ? KT : 0); ++k) {
+      const float gx = gdv[2 * k + 0], gy = gdv[2 * k + 1];
+      const float u_term = gx * db.x + gy * db.y;
+      const float v_term = gx * db.z + gy * db.w;
+      rv[k] += -u_term - v_term;
+      rv[AT + k] += u_term;
+      rv[2 * AT + k] += v_term;
     }
-    // Runs of same-triangle lanes along a pixel row add into the same rows:
-    // sum each run first, its last lane adds the total.
-    const bool tail = row_run_sum(valid ? (uint64_t)t : (1ull << 63) | (uint64_t)lane, rv);
-    if (valid && tail) {
-      lds_table_add(tab, da + (int64_t)i0 * AT, &rv[0]);
-      lds_table_add(tab, da + (int64_t)i1 * AT, &rv[AT]);
-      lds_table_add(tab, da + (int64_t)i2 * AT, &rv[2 * AT]);
-    }
-  } else {
-    // Any shape: element by element.
-    const int A = A_;
-    const int K = K_;
-    if (valid) {
-      i0 = tri[t * 3 + 0];
-      i1 = tri[t * 3 + 1];
-      i2 = tri[t * 3 + 2];
-      valid = verts_ok(i0, i1, i2, V);  // pixels of foreign ids are empty
-    }
-    const float* g = d_out + pix * A;
-    float4 db = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (K > 0 && valid) db = *reinterpret_cast<const float4*>(rast_db + pix * 4);
-    float du = 0.0f, dv = 0.0f;
-    if (valid) {
-      for (int a = 0; a < A; ++a) {
-        const float a0 = at[(int64_t)i0 * A + a], a1 = at[(int64_t)i1 * A + a],
-                    a2 = at[(int64_t)i2 * A + a];
-        du += (a1 - a0) * g[a];
-        dv += (a2 - a0) * g[a];
-      }
-    }
-    float d_udx = 0.0f, d_udy = 0.0f, d_vdx = 0.0f, d_vdy = 0.0f;
-    if (K > 0 && valid) {
-      const float* gd = d_out_da + pix * 2 * K;
-      for (int k = 0; k < K; ++k) {
-        const int a = diff_idx ? diff_idx[k] : k;
-        if ((unsigned)a >= (unsigned)A) continue;  // not an attribute
-        const float a0 = at[(int64_t)i0 * A + a], a1 = at[(int64_t)i1 * A + a],
-                    a2 = at[(int64_t)i2 * A + a];
-        const float d01 = a1 - a0, d02 = a2 - a0;
-        const float gx = gd[2 * k + 0], gy = gd[2 * k + 1];
-        d_udx += d01 * gx;
-        d_udy += d01 * gy;
-        d_vdx += d02 * gx;
-        d_vdy += d02 * gy;
-      }
-    }
-    if (inside) {
-      *reinterpret_cast<float4*>(d_rast + pix * 4) = make_float4(du, dv, 0.0f, 0.0f);
-      if (K > 0 && d_rast_db)
-        *reinterpret_cast<float4*>(d_rast_db + pix * 4) = make_float4(d_udx, d_udy, d_vdx, d_vdy);
-    }
-    if (valid) {
-      for (int a = 0; a < A; ++a) {
-        const float ga = g[a];
-        const float v0[1] = {bw * ga}, v1[1] = {u * ga}, v2[1] = {v * ga};
-        lds_table_add(tab, da + (int64_t)i0 * A + a, v0);
-        lds_table_add(tab, da + (int64_t)i1 * A + a, v1);
-        lds_table_add(tab, da + (int64_t)i2 * A + a, v2);
-      }
-      if (K > 0) {
-        const float* gd = d_out_da + pix * 2 * K;
-        for (int k = 0; k < K; ++k) {
-          const int a = diff_idx ? diff_idx[k] : k;
-          if ((unsigned)a >= (unsigned)A) continue;  // not an attribute
-          const float gx = gd[2 * k + 0], gy = gd[2 * k + 1];
-          const float u_term = gx * db.x + gy * db.y;
-          const float v_term = gx * db.z + gy * db.w;
-          const float v0[1] = {-u_term - v_term}, v1[1] = {u_term}, v2[1] = {v_term};
-          lds_table_add(tab, da + (int64_t)i0 * A + a, v0);
-          lds_table_add(tab, da + (int64_t)i1 * A + a, v1);
-          lds_table_add(tab, da + (int64_t)i2 * A + a, v2);
-        }
-      }
-    }
+  }
+  // Runs of same-triangle lanes along a pixel row add into the same rows:
+  // sum each run first, its last lane adds the total.
+  const bool tail = row_run_sum(valid ? (uint64_t)t : (1ull << 63) | (uint64_t)lane, rv);
+  if (valid && tail) {
+    lds_table_add(tab, da + (int64_t)i0 * AT, &rv[0]);
+    lds_table_add(tab, da + (int64_t)i1 * AT, &rv[AT]);
+    lds_table_add(tab, da + (int64_t)i2 * AT, &rv[2 * AT]);
   }
   __syncthreads();
   lds_table_flush_last(tab);  // the taken rows only
+}
+
+// The backward of any other shape, on the same tiles.  A lane finds its three
+// vertices' entries in the tile's table of d_attr rows once; the attributes
+// then go through the entries' sums four at a time (run sums along the pixel
+// row, LDS adds, one row-run of device atomics per entry, clear), while d_rast
+// and d_rast_db sum over them in registers.  Element by element, each
+// attribute of each vertex searched a table of 256 single values by itself
+// and, once that was full, became a device atomic (4 x 720 x 1280, A = 8,
+// K = 2: 320 us, now 95).
+constexpr int kAnyRows = 256;   // table entries: vertex rows of a tile
+constexpr int kAnyChunk = 4;
+constexpr int kAnyNone = 0xffff;  // no entry: the row goes to memory
+
+__global__ void __launch_bounds__(256) k_interp_bwd_any(
+    const float* __restrict__ attr, int64_t attr_stride, const float* __restrict__ rast,
+    const float* __restrict__ rast_db, const int32_t* __restrict__ tri,
+    const int32_t* __restrict__ diff_idx, int K, const float* __restrict__ d_out,
+    const float* __restrict__ d_out_da, int H, int W, int ntx, int nty, int V, int T, int A,
+    float* __restrict__ d_attr, int64_t d_attr_stride, int ncopy, int64_t copy_stride,
+    float* __restrict__ d_rast, float* __restrict__ d_rast_db, int xcd) {
+  __shared__ int s_row[kAnyRows];                   // vertex of an entry, -1 = free
+  __shared__ double s_sum[kAnyChunk][kAnyRows];     // component-major (LdsTable)
+  __shared__ uint16_t s_used[kAnyRows];
+  __shared__ int s_n;
+  __shared__ int s_any[4];  // per wave: a covered pixel
+  const int tiles = ntx * nty;
+  const int b = xcd ? xcd_remap((int)blockIdx.x, (int)gridDim.x) : (int)blockIdx.x;
+  const int n = b / tiles;
+  const int tile = b - n * tiles;
+  const int ty = tile / ntx, tx = tile - ty * ntx;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int pw = tx * 16 + (lane & 15), ph = ty * 16 + wave * 4 + (lane >> 4);
+  const bool inside = pw < W && ph < H;
+  const int64_t pix = ((int64_t)n * H + min(ph, H - 1)) * W + min(pw, W - 1);
+  const float4 r = *reinterpret_cast<const float4*>(rast + pix * 4);
+  const int t = f2i(r.w) - 1;
+  bool valid = inside && t >= 0 && t < T;
+  {
+    const uint64_t any = __ballot(valid);
+    if (lane == 0) s_any[wave] = any != 0ull;
+  }
+  s_row[tid] = -1;
+#pragma unroll
+  for (int j = 0; j < kAnyChunk; ++j) s_sum[j][tid] = 0.0;
+  static_assert(kAnyRows == 256, "one entry per thread");
+  if (tid == 0) s_n = 0;
+  __syncthreads();
+  if (!(s_any[0] | s_any[1] | s_any[2] | s_any[3])) {  // uniform: an empty tile
+    if (inside) {
+      *reinterpret_cast<float4*>(d_rast + pix * 4) = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (K > 0 && d_rast_db)
+        *reinterpret_cast<float4*>(d_rast_db + pix * 4) = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    return;
+  }
+  const float u = r.x, v = r.y;
+  const float bw = 1.0f - u - v;
+  const float* at = attr + (int64_t)n * attr_stride;
+  float* da = d_attr + (ncopy ? (int64_t)(b % ncopy) * copy_stride : 0) + (int64_t)n * d_attr_stride;
+  int vi[3] = {0, 0, 0};
+  float4 db = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (valid) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j) vi[j] = tri[t * 3 + j];
+    if (K > 0) db = *reinterpret_cast<const float4*>(rast_db + pix * 4);
+    valid = verts_ok(vi[0], vi[1], vi[2], V);  // pixels of foreign ids are empty
+  }
+  // runs of one triangle along a pixel row; the run's last lane adds its sums
+  const RowRun run = row_run(valid ? (uint64_t)t : (1ull << 63) | (uint64_t)lane);
+  const int maxlen = wave_max(run.li - run.s + 1);
+  const bool tail = valid && run.tail;
+  int slot[3] = {kAnyNone, kAnyNone, kAnyNone};
+  if (tail) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      uint32_t h = ((uint32_t)vi[j] * 0x9E3779B1u) >> 24;
+#pragma unroll 1
+      for (int probe = 0; probe < kLdsProbes; ++probe) {
+        int cur = s_row[h];
+        if (cur == -1) {
+          cur = atomicCAS(&s_row[h], -1, vi[j]);
+          if (cur == -1) s_used[atomicAdd(&s_n, 1)] = (uint16_t)h;  // taken here
+        }
+        if (cur == -1 || cur == vi[j]) {
+          slot[j] = (int)h;
+          break;
+        }
+        h = (h + 1) & (kAnyRows - 1);
+      }
+    }
+  }
+  float du = 0.0f, dv = 0.0f;
+  float d_udx = 0.0f, d_udy = 0.0f, d_vdx = 0.0f, d_vdy = 0.0f;
+  const float* g = d_out + pix * A;
+  const float* gd = K > 0 ? d_out_da + pix * 2 * K : nullptr;
+  const int64_t o0 = (int64_t)vi[0] * A, o1 = (int64_t)vi[1] * A, o2 = (int64_t)vi[2] * A;
+#pragma unroll 1
+  for (int c = 0; c < A; c += kAnyChunk) {
+    const int nc = min(kAnyChunk, A - c);
+    float rv[3 * kAnyChunk];
+#pragma unroll
+    for (int j = 0; j < 3 * kAnyChunk; ++j) rv[j] = 0.0f;
+    if (valid) {
+      const float4 g4 = ld_chunk(g + c, nc);
+      const float4 x = ld_chunk(at + o0 + c, nc), y = ld_chunk(at + o1 + c, nc),
+                   z = ld_chunk(at + o2 + c, nc);
+      const float ga[4] = {g4.x, g4.y, g4.z, g4.w};
+      const float d01[4] = {y.x - x.x, y.y - x.y, y.z - x.z, y.w - x.w};
+      const float d02[4] = {z.x - x.x, z.y - x.y, z.z - x.z, z.w - x.w};
+#pragma unroll
+      for (int j = 0; j < kAnyChunk; ++j) {
+        du += d01[j] * ga[j];
+        dv += d02[j] * ga[j];
+        rv[j] = bw * ga[j];
+        rv[kAnyChunk + j] = u * ga[j];
+        rv[2 * kAnyChunk + j] = v * ga[j];
+      }
+      // derivative outputs of this chunk's attributes (indices are uniform)
+#pragma unroll 1
+      for (int k = diff_idx ? 0 : c; k < (diff_idx ? K : min(K, c + nc)); ++k) {
+        const int q = (diff_idx ? diff_idx[k] : k) - c;
+        if ((unsigned)q >= (unsigned)nc) continue;  // another chunk's, or no attribute
+        const float gx = gd[2 * k + 0], gy = gd[2 * k + 1];
+        const float u_term = gx * db.x + gy * db.y;
+        const float v_term = gx * db.z + gy * db.w;
+#pragma unroll
+        for (int j = 0; j < kAnyChunk; ++j) {
+          if (j != q) continue;
+          d_udx += d01[j] * gx;
+          d_udy += d01[j] * gy;
+          d_vdx += d02[j] * gx;
+          d_vdy += d02[j] * gy;
+          rv[j] += -u_term - v_term;
+          rv[kAnyChunk + j] += u_term;
+          rv[2 * kAnyChunk + j] += v_term;
+        }
+      }
+    }
+    row_run_scan_n(run, rv, maxlen);
+    if (tail) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+#pragma unroll
+        for (int j = 0; j < kAnyChunk; ++j) {
+          const float x = rv[i * kAnyChunk + j];
+          if (j >= nc || x == 0.0f) continue;
+          if (slot[i] != kAnyNone)
+            atomicAdd(&s_sum[j][slot[i]], (double)x);
+          else
+            unsafeAtomicAdd(da + (int64_t)vi[i] * A + c + j, x);
+        }
+      }
+    }
+    __syncthreads();
+    // the taken entries' sums of this chunk, consecutive lanes on
+    // consecutive attributes of a row
+    const int m = s_n * kAnyChunk;
+    for (int i = tid; i < m; i += 256) {
+      const int e = s_used[i >> 2], j = i & 3;
+      const double x = s_sum[j][e];
+      if (x != 0.0) {
+        unsafeAtomicAdd(da + (int64_t)s_row[e] * A + c + j, (float)x);
+        s_sum[j][e] = 0.0;
+      }
+    }
+    if (c + kAnyChunk < A) __syncthreads();  // cleared before the next chunk adds
+  }
+  if (inside) {
+    *reinterpret_cast<float4*>(d_rast + pix * 4) = make_float4(du, dv, 0.0f, 0.0f);
+    if (K > 0 && d_rast_db)
+      *reinterpret_cast<float4*>(d_rast_db + pix * 4) = make_float4(d_udx, d_udy, d_vdx, d_vdy);
+  }
 }
 
 // d_attr[i] = (accumulate ? d_attr[i] : 0) + the sum of the 256 copies'
@@ -452,15 +583,25 @@ __global__ void __launch_bounds__(256) k_sum_copies(float* __restrict__ copies, 
 
 using namespace dr;
 
+// The shapes with a kernel of their own: those whose attributes and
+// derivatives fit registers whole and are the common ones (a mask, uv, uv
+// with derivatives, a direction or colour, a direction with derivatives,
+// RGBA, normal + colour).  The others take the chunked kernels, which are
+// slower where both apply (4 x 720 x 1280, A = 1: forward 21 against 18 us).
+static bool interp_shape(int A, int K, bool diff_idx) {
+  if (K == 0) return A <= 4 || A == 6;
+  return !diff_idx && K == A && (A == 2 || A == 3);
+}
+
 #define DR_INTERP_DISPATCH(KERNEL, GRID, ...)                                              \
   do {                                                                                     \
-    if (A == 2 && K == 0) hipLaunchKernelGGL((KERNEL<2, 0>), GRID, dim3(256), 0, stream, __VA_ARGS__); \
-    else if (A == 2 && K == 2 && !diff_idx) hipLaunchKernelGGL((KERNEL<2, 2>), GRID, dim3(256), 0, stream, __VA_ARGS__); \
+    if (A == 1) hipLaunchKernelGGL((KERNEL<1, 0>), GRID, dim3(256), 0, stream, __VA_ARGS__); \
+    else if (A == 2 && K == 0) hipLaunchKernelGGL((KERNEL<2, 0>), GRID, dim3(256), 0, stream, __VA_ARGS__); \
+    else if (A == 2) hipLaunchKernelGGL((KERNEL<2, 2>), GRID, dim3(256), 0, stream, __VA_ARGS__); \
     else if (A == 3 && K == 0) hipLaunchKernelGGL((KERNEL<3, 0>), GRID, dim3(256), 0, stream, __VA_ARGS__); \
-    else if (A == 3 && K == 3 && !diff_idx) hipLaunchKernelGGL((KERNEL<3, 3>), GRID, dim3(256), 0, stream, __VA_ARGS__); \
-    else if (A == 4 && K == 0) hipLaunchKernelGGL((KERNEL<4, 0>), GRID, dim3(256), 0, stream, __VA_ARGS__); \
-    else if (A == 6 && K == 0) hipLaunchKernelGGL((KERNEL<6, 0>), GRID, dim3(256), 0, stream, __VA_ARGS__); \
-    else hipLaunchKernelGGL((KERNEL<0, 0>), GRID, dim3(256), 0, stream, __VA_ARGS__);      \
+    else if (A == 3) hipLaunchKernelGGL((KERNEL<3, 3>), GRID, dim3(256), 0, stream, __VA_ARGS__); \
+    else if (A == 4) hipLaunchKernelGGL((KERNEL<4, 0>), GRID, dim3(256), 0, stream, __VA_ARGS__); \
+    else hipLaunchKernelGGL((KERNEL<6, 0>), GRID, dim3(256), 0, stream, __VA_ARGS__);      \
   } while (0)
 
 static int check_interp(const float* attr, const float* rast, const int32_t* tri,
@@ -489,23 +630,22 @@ extern "C" int dr_interpolate_fwd(const float* attr, int64_t attr_batch_stride,
   DR_TIMED("k_interp_fwd", stream);
   // the compile-time shapes store with 8/16-byte vector writes
   const bool aligned = (((uintptr_t)out | (uintptr_t)(out_da ? out_da : out)) & 15) == 0;
-  // the dispatched kernel's pixels per thread (DR_INTERP_DISPATCH's choice)
-  const int px = aligned && A == 6 && K == 0 ? interp_pix<6>() : interp_pix<0>();
-  // and its strip width: the shapes of DR_INTERP_DISPATCH with an even A
-  const bool even = aligned && (A == 2 || A == 4 || A == 6) &&
-                    ((A == 2 && (K == 0 || (K == 2 && !diff_idx))) || (A != 2 && K == 0));
-  const int sw = even ? interp_strip<2>() : interp_strip<0>(), sh = 256 / sw;
+  const bool shape = aligned && interp_shape(A, K, diff_idx != nullptr);
+  // the kernel's tile: strips interp_strip wide, interp_pix pixels a thread;
+  // the general one's is 16 x 16
+  const int px = shape ? interp_pix<2>() : 1;
+  const int sw = !shape || A % 2 == 0 ? interp_strip<2>() : interp_strip<3>(), sh = 256 / sw;
   const int ntx = (W + sw - 1) / sw, nty = (H + sh * px - 1) / (sh * px);
   const int64_t nblk = (int64_t)N * ntx * nty;
   DR_CHECK_ARG(nblk < ((int64_t)1 << 31), "interpolate: too many pixels");
   const dim3 grid((unsigned)nblk);
   const int xcd = (int64_t)V * A * (int64_t)sizeof(float) > kXcdL2Bytes;
-  if (!aligned)
-    hipLaunchKernelGGL((k_interp_fwd<0, 0>), grid, dim3(256), 0, stream, attr, attr_batch_stride,
-                       rast, rast_db, tri, diff_idx, K, H, W, ntx, nty, V, T, A, out, out_da, xcd);
+  if (shape)
+    DR_INTERP_DISPATCH(k_interp_fwd, grid, attr, attr_batch_stride, rast, rast_db, tri, H, W, ntx,
+                       nty, V, T, out, out_da, xcd);
   else
-    DR_INTERP_DISPATCH(k_interp_fwd, grid, attr, attr_batch_stride, rast, rast_db, tri, diff_idx,
-                       K, H, W, ntx, nty, V, T, A, out, out_da, xcd);
+    hipLaunchKernelGGL(k_interp_fwd_any, grid, dim3(256), 0, stream, attr, attr_batch_stride, rast,
+                       rast_db, tri, diff_idx, K, H, W, ntx, nty, V, T, A, out, out_da, xcd);
   DR_CHECK_LAUNCH();
   return DR_OK;
 }
@@ -553,9 +693,15 @@ extern "C" int dr_interpolate_bwd(const float* attr, int64_t attr_batch_stride,
   const int xcd = (int64_t)V * A * (int64_t)sizeof(float) > kXcdL2Bytes;
   {
     DR_TIMED("k_interp_bwd", stream);
-    DR_INTERP_DISPATCH(k_interp_bwd, grid, attr, attr_batch_stride, rast, rast_db, tri, diff_idx,
-                       K, d_out, d_out_da, N, H, W, ntx, nty, V, T, A, target,
-                       d_attr_batch_stride, copy ? kCopies : 0, nattr, d_rast, d_rast_db, xcd);
+    if (interp_shape(A, K, diff_idx != nullptr))
+      DR_INTERP_DISPATCH(k_interp_bwd, grid, attr, attr_batch_stride, rast, rast_db, tri, d_out,
+                         d_out_da, H, W, ntx, nty, V, T, target, d_attr_batch_stride,
+                         copy ? kCopies : 0, nattr, d_rast, d_rast_db, xcd);
+    else
+      hipLaunchKernelGGL(k_interp_bwd_any, grid, dim3(256), 0, stream, attr, attr_batch_stride,
+                         rast, rast_db, tri, diff_idx, K, d_out, d_out_da, H, W, ntx, nty, V, T, A,
+                         target, d_attr_batch_stride, copy ? kCopies : 0, nattr, d_rast, d_rast_db,
+                         xcd);
   }
   DR_CHECK_LAUNCH();
   if (copy) {

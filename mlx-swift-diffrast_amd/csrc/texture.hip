@@ -1496,27 +1496,6 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
 // (2 x 768^2 x 16, trilinear: 286 -> 40 us).
 // ---------------------------------------------------------------------------
 
-// Four channels from p, the first nc of them in memory (nc = 4: one load
-// whatever p's alignment; the hardware takes 4-byte aligned vectors).
-typedef float dr_f4u __attribute__((ext_vector_type(4), aligned(4)));
-__device__ __forceinline__ float4 ld_chunk(const float* __restrict__ p, int nc) {
-  if (nc == 4) {
-    const dr_f4u v = *reinterpret_cast<const dr_f4u*>(p);
-    return make_float4(v.x, v.y, v.z, v.w);
-  }
-  return make_float4(p[0], nc > 1 ? p[1] : 0.0f, nc > 2 ? p[2] : 0.0f, 0.0f);
-}
-__device__ __forceinline__ void st_chunk(float* __restrict__ p, float4 x, int nc) {
-  if (nc == 4) {
-    dr_f4u v = {x.x, x.y, x.z, x.w};
-    *reinterpret_cast<dr_f4u*>(p) = v;
-    return;
-  }
-  p[0] = x.x;
-  if (nc > 1) p[1] = x.y;
-  if (nc > 2) p[2] = x.z;
-}
-
 // The bilinear sample of channels [c, c + nc) of one level, in tex_fwd_px's
 // operation order.
 __device__ __forceinline__ float4 sample_chunk(const float* __restrict__ lv, int Wk, int C,
