@@ -244,6 +244,21 @@ int dr_interpolate_bwd(const float* attr, int64_t attr_batch_stride, const float
                        int V, int T, int A, float* d_attr, int64_t d_attr_batch_stride,
                        float* d_rast, float* d_rast_db, unsigned flags, dr_stream_t stream);
 
+/* The two calls with the K derivative indices in host memory (read before
+ * the call returns; K in 1..DR_INTERPOLATE_HOST_IDX): they travel with the
+ * launch, so the caller makes no device copy of them.  Results as above. */
+#define DR_INTERPOLATE_HOST_IDX 32
+int dr_interpolate_fwd_idx(const float* attr, int64_t attr_batch_stride, const float* rast,
+                           const float* rast_db, const int32_t* tri,
+                           const int32_t* diff_idx_host, int K, int N, int H, int W, int V, int T,
+                           int A, float* out, float* out_da, dr_stream_t stream);
+int dr_interpolate_bwd_idx(const float* attr, int64_t attr_batch_stride, const float* rast,
+                           const float* rast_db, const int32_t* tri,
+                           const int32_t* diff_idx_host, int K, const float* d_out,
+                           const float* d_out_da, int N, int H, int W, int V, int T, int A,
+                           float* d_attr, int64_t d_attr_batch_stride, float* d_rast,
+                           float* d_rast_db, unsigned flags, dr_stream_t stream);
+
 /* ---- texture --------------------------------------------------------- */
 
 /* textureConstructMip (Texture.swift:144-161): number of levels (level 0

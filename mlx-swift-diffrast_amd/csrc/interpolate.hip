@@ -181,6 +181,18 @@ __global__ void __launch_bounds__(256) k_interp_fwd(
   }
 }
 
+// Which attributes the K derivative pairs are of: all of them in order, K
+// indices in device memory, or K indices in the launch's own arguments (a
+// caller that has them on the host then makes no device copy, which waits
+// for the stream: 4 x 720 x 1280, A = 8, K = 2: 187 -> 169 us a pass).
+struct DiffIdx {
+  const int32_t* dev;
+  int by_value;
+  int32_t v[DR_INTERPOLATE_HOST_IDX];
+  __device__ __forceinline__ int operator()(int k) const { return dev ? dev[k] : by_value ? v[k] : k; }
+  __device__ __forceinline__ bool listed() const { return dev != nullptr || by_value; }
+};
+
 // Any other shape: attributes in chunks of four, a thread per (pixel, chunk)
 // with consecutive threads on consecutive chunks, so a vertex row's reads and
 // a pixel's writes are runs of memory; the derivatives of a pixel's K chosen
@@ -191,8 +203,8 @@ __global__ void __launch_bounds__(256) k_interp_fwd(
 __global__ void __launch_bounds__(256) k_interp_fwd_any(
     const float* __restrict__ attr, int64_t attr_stride, const float* __restrict__ rast,
     const float* __restrict__ rast_db, const int32_t* __restrict__ tri,
-    const int32_t* __restrict__ diff_idx, int K, int H, int W, int ntx, int nty, int V, int T,
-    int A, float* __restrict__ out, float* __restrict__ out_da, int xcd) {
+    DiffIdx diff, int K, int H, int W, int ntx, int nty, int V, int T, int A,
+    float* __restrict__ out, float* __restrict__ out_da, int xcd) {
   const int tiles = ntx * nty;
   const int b = xcd ? xcd_remap((int)blockIdx.x, (int)gridDim.x) : (int)blockIdx.x;
   const int img = b / tiles;
@@ -236,7 +248,7 @@ __global__ void __launch_bounds__(256) k_interp_fwd_any(
     if (g >= K) continue;
     const float4 db = *reinterpret_cast<const float4*>(rast_db + pix * 4);
     for (int k = g; k < K; k += G) {
-      const int q = diff_idx ? diff_idx[k] : k;
+      const int q = diff(k);
       float2 d = make_float2(0.0f, 0.0f);  // not an attribute: zero derivatives
       if ((unsigned)q < (unsigned)A) {
         const float a0 = r0[q];
@@ -402,7 +414,7 @@ constexpr int kAnyNone = 0xffff;  // no entry: the row goes to memory
 __global__ void __launch_bounds__(256) k_interp_bwd_any(
     const float* __restrict__ attr, int64_t attr_stride, const float* __restrict__ rast,
     const float* __restrict__ rast_db, const int32_t* __restrict__ tri,
-    const int32_t* __restrict__ diff_idx, int K, const float* __restrict__ d_out,
+    DiffIdx diff, int K, const float* __restrict__ d_out,
     const float* __restrict__ d_out_da, int H, int W, int ntx, int nty, int V, int T, int A,
     float* __restrict__ d_attr, int64_t d_attr_stride, int ncopy, int64_t copy_stride,
     float* __restrict__ d_rast, float* __restrict__ d_rast_db, int xcd) {
@@ -505,8 +517,8 @@ __global__ void __launch_bounds__(256) k_interp_bwd_any(
       }
       // derivative outputs of this chunk's attributes (indices are uniform)
 #pragma unroll 1
-      for (int k = diff_idx ? 0 : c; k < (diff_idx ? K : min(K, c + nc)); ++k) {
-        const int q = (diff_idx ? diff_idx[k] : k) - c;
+      for (int k = diff.listed() ? 0 : c; k < (diff.listed() ? K : min(K, c + nc)); ++k) {
+        const int q = diff(k) - c;
         if ((unsigned)q >= (unsigned)nc) continue;  // another chunk's, or no attribute
         const float gx = gd[2 * k + 0], gy = gd[2 * k + 1];
         const float u_term = gx * db.x + gy * db.y;
@@ -606,7 +618,7 @@ static bool interp_shape(int A, int K, bool diff_idx) {
 
 static int check_interp(const float* attr, const float* rast, const int32_t* tri,
                         const float* rast_db, int K, int N, int H, int W, int V, int T, int A,
-                        int64_t attr_stride, const int32_t* diff_idx) {
+                        int64_t attr_stride, const DiffIdx& diff) {
   DR_CHECK_ARG(N >= 1 && H >= 1 && W >= 1 && V >= 0 && T >= 0 && A >= 1 && K >= 0,
                "interpolate: bad sizes");
   DR_CHECK_ARG(attr && rast && tri, "interpolate: null tensor");
@@ -614,23 +626,32 @@ static int check_interp(const float* attr, const float* rast, const int32_t* tri
   DR_CHECK_ARG(attr_stride == 0 || attr_stride == (int64_t)V * A,
                "interpolate: attr_batch_stride must be 0 or V*A");
   DR_CHECK_ARG(K == 0 || rast_db, "interpolate: rastDB is required when diffAttrs is set");
-  DR_CHECK_ARG(K == 0 || diff_idx || K == A, "interpolate: diff_idx NULL needs K == A");
+  DR_CHECK_ARG(K == 0 || diff.dev || diff.by_value || K == A, "interpolate: diff_idx NULL needs K == A");
   return DR_OK;
 }
 
-extern "C" int dr_interpolate_fwd(const float* attr, int64_t attr_batch_stride,
-                                  const float* rast, const float* rast_db, const int32_t* tri,
-                                  const int32_t* diff_idx, int K, int N, int H, int W, int V,
-                                  int T, int A, float* out, float* out_da, dr_stream_t stream_) {
-  hipStream_t stream = (hipStream_t)stream_;
+// K indices on the host, by value (K in [1, DR_INTERPOLATE_HOST_IDX]).
+static int host_idx(const int32_t* idx, int K, DiffIdx& diff) {
+  DR_CHECK_ARG(idx && K >= 1 && K <= DR_INTERPOLATE_HOST_IDX,
+               "interpolate: 1 to 32 derivative indices can be given on the host");
+  diff.dev = nullptr;
+  diff.by_value = 1;
+  for (int k = 0; k < K; ++k) diff.v[k] = idx[k];
+  return DR_OK;
+}
+
+static int interp_fwd(const float* attr, int64_t attr_batch_stride, const float* rast,
+                      const float* rast_db, const int32_t* tri, const DiffIdx& diff, int K, int N,
+                      int H, int W, int V, int T, int A, float* out, float* out_da,
+                      hipStream_t stream) {
   (void)hipGetLastError();
-  int st = check_interp(attr, rast, tri, rast_db, K, N, H, W, V, T, A, attr_batch_stride, diff_idx);
+  int st = check_interp(attr, rast, tri, rast_db, K, N, H, W, V, T, A, attr_batch_stride, diff);
   if (st) return st;
   DR_CHECK_ARG(out && (K == 0 || out_da), "interpolate: null output");
   DR_TIMED("k_interp_fwd", stream);
   // the compile-time shapes store with 8/16-byte vector writes
   const bool aligned = (((uintptr_t)out | (uintptr_t)(out_da ? out_da : out)) & 15) == 0;
-  const bool shape = aligned && interp_shape(A, K, diff_idx != nullptr);
+  const bool shape = aligned && interp_shape(A, K, diff.dev || diff.by_value);
   // the kernel's tile: strips interp_strip wide, interp_pix pixels a thread;
   // the general one's is 16 x 16
   const int px = shape ? interp_pix<2>() : 1;
@@ -645,21 +666,18 @@ extern "C" int dr_interpolate_fwd(const float* attr, int64_t attr_batch_stride,
                        nty, V, T, out, out_da, xcd);
   else
     hipLaunchKernelGGL(k_interp_fwd_any, grid, dim3(256), 0, stream, attr, attr_batch_stride, rast,
-                       rast_db, tri, diff_idx, K, H, W, ntx, nty, V, T, A, out, out_da, xcd);
+                       rast_db, tri, diff, K, H, W, ntx, nty, V, T, A, out, out_da, xcd);
   DR_CHECK_LAUNCH();
   return DR_OK;
 }
 
-extern "C" int dr_interpolate_bwd(const float* attr, int64_t attr_batch_stride,
-                                  const float* rast, const float* rast_db, const int32_t* tri,
-                                  const int32_t* diff_idx, int K, const float* d_out,
-                                  const float* d_out_da, int N, int H, int W, int V, int T,
-                                  int A, float* d_attr, int64_t d_attr_batch_stride,
-                                  float* d_rast, float* d_rast_db, unsigned flags,
-                                  dr_stream_t stream_) {
-  hipStream_t stream = (hipStream_t)stream_;
+static int interp_bwd(const float* attr, int64_t attr_batch_stride, const float* rast,
+                      const float* rast_db, const int32_t* tri, const DiffIdx& diff, int K,
+                      const float* d_out, const float* d_out_da, int N, int H, int W, int V, int T,
+                      int A, float* d_attr, int64_t d_attr_batch_stride, float* d_rast,
+                      float* d_rast_db, unsigned flags, hipStream_t stream) {
   (void)hipGetLastError();
-  int st = check_interp(attr, rast, tri, rast_db, K, N, H, W, V, T, A, attr_batch_stride, diff_idx);
+  int st = check_interp(attr, rast, tri, rast_db, K, N, H, W, V, T, A, attr_batch_stride, diff);
   if (st) return st;
   DR_CHECK_ARG(d_out && d_attr && d_rast && (K == 0 || d_out_da), "interpolate_bwd: null tensor");
   DR_CHECK_ARG(d_attr_batch_stride == 0 || d_attr_batch_stride == (int64_t)V * A,
@@ -693,13 +711,13 @@ extern "C" int dr_interpolate_bwd(const float* attr, int64_t attr_batch_stride,
   const int xcd = (int64_t)V * A * (int64_t)sizeof(float) > kXcdL2Bytes;
   {
     DR_TIMED("k_interp_bwd", stream);
-    if (interp_shape(A, K, diff_idx != nullptr))
+    if (interp_shape(A, K, diff.dev || diff.by_value))
       DR_INTERP_DISPATCH(k_interp_bwd, grid, attr, attr_batch_stride, rast, rast_db, tri, d_out,
                          d_out_da, H, W, ntx, nty, V, T, target, d_attr_batch_stride,
                          copy ? kCopies : 0, nattr, d_rast, d_rast_db, xcd);
     else
       hipLaunchKernelGGL(k_interp_bwd_any, grid, dim3(256), 0, stream, attr, attr_batch_stride,
-                         rast, rast_db, tri, diff_idx, K, d_out, d_out_da, H, W, ntx, nty, V, T, A,
+                         rast, rast_db, tri, diff, K, d_out, d_out_da, H, W, ntx, nty, V, T, A,
                          target, d_attr_batch_stride, copy ? kCopies : 0, nattr, d_rast, d_rast_db,
                          xcd);
   }
@@ -716,4 +734,51 @@ extern "C" int dr_interpolate_bwd(const float* attr, int64_t attr_batch_stride,
     if (sc && sc->copy_buf == target) sc->copy_zero = nattr * kCopies;
   }
   return DR_OK;
+}
+
+extern "C" int dr_interpolate_fwd(const float* attr, int64_t attr_batch_stride,
+                                  const float* rast, const float* rast_db, const int32_t* tri,
+                                  const int32_t* diff_idx, int K, int N, int H, int W, int V,
+                                  int T, int A, float* out, float* out_da, dr_stream_t stream) {
+  return interp_fwd(attr, attr_batch_stride, rast, rast_db, tri, DiffIdx{diff_idx, 0, {}}, K, N, H,
+                    W, V, T, A, out, out_da, (hipStream_t)stream);
+}
+
+extern "C" int dr_interpolate_bwd(const float* attr, int64_t attr_batch_stride,
+                                  const float* rast, const float* rast_db, const int32_t* tri,
+                                  const int32_t* diff_idx, int K, const float* d_out,
+                                  const float* d_out_da, int N, int H, int W, int V, int T,
+                                  int A, float* d_attr, int64_t d_attr_batch_stride,
+                                  float* d_rast, float* d_rast_db, unsigned flags,
+                                  dr_stream_t stream) {
+  return interp_bwd(attr, attr_batch_stride, rast, rast_db, tri, DiffIdx{diff_idx, 0, {}}, K, d_out,
+                    d_out_da, N, H, W, V, T, A, d_attr, d_attr_batch_stride, d_rast, d_rast_db,
+                    flags, (hipStream_t)stream);
+}
+
+extern "C" int dr_interpolate_fwd_idx(const float* attr, int64_t attr_batch_stride,
+                                      const float* rast, const float* rast_db, const int32_t* tri,
+                                      const int32_t* diff_idx_host, int K, int N, int H, int W,
+                                      int V, int T, int A, float* out, float* out_da,
+                                      dr_stream_t stream) {
+  DiffIdx diff{};
+  const int st = host_idx(diff_idx_host, K, diff);
+  if (st) return st;
+  return interp_fwd(attr, attr_batch_stride, rast, rast_db, tri, diff, K, N, H, W, V, T, A, out,
+                    out_da, (hipStream_t)stream);
+}
+
+extern "C" int dr_interpolate_bwd_idx(const float* attr, int64_t attr_batch_stride,
+                                      const float* rast, const float* rast_db, const int32_t* tri,
+                                      const int32_t* diff_idx_host, int K, const float* d_out,
+                                      const float* d_out_da, int N, int H, int W, int V, int T,
+                                      int A, float* d_attr, int64_t d_attr_batch_stride,
+                                      float* d_rast, float* d_rast_db, unsigned flags,
+                                      dr_stream_t stream) {
+  DiffIdx diff{};
+  const int st = host_idx(diff_idx_host, K, diff);
+  if (st) return st;
+  return interp_bwd(attr, attr_batch_stride, rast, rast_db, tri, diff, K, d_out, d_out_da, N, H, W,
+                    V, T, A, d_attr, d_attr_batch_stride, d_rast, d_rast_db, flags,
+                    (hipStream_t)stream);
 }

@@ -36,6 +36,10 @@ SIGNATURES = {
                            _i),
     "dr_interpolate_bwd": ([_p, _i64, _p, _p, _p, _p, _i, _p, _p, _i, _i, _i, _i, _i, _i, _p, _i64,
                             _p, _p, _u, _p], _i),
+    "dr_interpolate_fwd_idx": ([_p, _i64, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _p, _p, _p],
+                               _i),
+    "dr_interpolate_bwd_idx": ([_p, _i64, _p, _p, _p, _p, _i, _p, _p, _i, _i, _i, _i, _i, _i, _p,
+                                _i64, _p, _p, _u, _p], _i),
     "dr_texture_mip_levels": ([_i, _i, _i, _p, _p], _i),
     "dr_texture_mip_size": ([_i, _i, _i, _i, _i], _i64),
     "dr_texture_build_mip": ([_p, _i, _i, _i, _i, _i, _p, _p], _i),
@@ -61,6 +65,7 @@ DR_ACCUMULATE = 1
 DR_CUBE_DIR_GRAD = 2
 DR_RASTERIZE_BWD_REUSE = 4
 DR_TEXTURE_BWD_NOALLOC_FLOATS = 8 * 1024 * 1024
+DR_INTERPOLATE_HOST_IDX = 32
 ABI_VERSION = 1
 
 _lib = None

@@ -187,27 +187,35 @@ class _RasterizeFn(torch.autograd.Function):
 # ---------------------------------------------------------------------------
 
 class _InterpolateFn(torch.autograd.Function):
+    # diff_idx: None (all attributes), a host array of at most
+    # DR_INTERPOLATE_HOST_IDX indices (passed with the launch), or a device
+    # tensor of more
     @staticmethod
     def forward(ctx, attr, rast, rast_db, tri, diff_idx, K, shared):
         lib = _lib.load()
+        on_host = isinstance(diff_idx, ctypes.Array)
+        fwd = lib.dr_interpolate_fwd_idx if on_host else lib.dr_interpolate_fwd
         N, H, W, _ = rast.shape
         V, A = attr.shape[-2], attr.shape[-1]
         stride = 0 if shared else V * A
         out = torch.empty((N, H, W, A), device=rast.device, dtype=torch.float32)
         out_da = torch.empty((N, H, W, 2 * K), device=rast.device, dtype=torch.float32)
-        _lib.check(lib.dr_interpolate_fwd(
+        _lib.check(fwd(
             _ptr(attr), stride, _ptr(rast), _ptr(rast_db) if K else None, _ptr(tri),
-            _ptr(diff_idx), K, N, H, W, V, tri.shape[0], A, _ptr(out), _ptr(out_da) if K else None,
+            diff_idx if on_host else _ptr(diff_idx), K, N, H, W, V, tri.shape[0], A, _ptr(out), _ptr(out_da) if K else None,
             _stream()))
-        ctx.save_for_backward(attr, rast, rast_db if K else None, tri, diff_idx)
-        ctx.meta = (K, shared)
+        ctx.save_for_backward(attr, rast, rast_db if K else None, tri,
+                              None if on_host else diff_idx)
+        ctx.meta = (K, shared, diff_idx if on_host else None)
         return out, out_da
 
     @staticmethod
     def backward(ctx, d_out, d_out_da):
         lib = _lib.load()
         attr, rast, rast_db, tri, diff_idx = ctx.saved_tensors
-        K, shared = ctx.meta
+        K, shared, host_idx = ctx.meta
+        on_host = host_idx is not None
+        bwd = lib.dr_interpolate_bwd_idx if on_host else lib.dr_interpolate_bwd
         N, H, W, _ = rast.shape
         V, A = attr.shape[-2], attr.shape[-1]
         stride = 0 if shared else V * A
@@ -219,8 +227,9 @@ class _InterpolateFn(torch.autograd.Function):
         d_attr = _grad_buf(attr)
         d_rast = _grad_buf(rast)
         d_rast_db = _grad_buf(rast) if K else None
-        _lib.check(lib.dr_interpolate_bwd(
-            _ptr(attr), stride, _ptr(rast), _ptr(rast_db), _ptr(tri), _ptr(diff_idx), K,
+        _lib.check(bwd(
+            _ptr(attr), stride, _ptr(rast), _ptr(rast_db), _ptr(tri),
+            host_idx if on_host else _ptr(diff_idx), K,
             _ptr(d_out), _ptr(d_out_da) if K else None, N, H, W, V, tri.shape[0], A, _ptr(d_attr),
             stride,
             _ptr(d_rast), _ptr(d_rast_db), 0, _stream()))
@@ -544,7 +553,10 @@ class DiffRast:
             if any(i < 0 or i >= A for i in diffAttrs.idx):
                 raise ValueError(f"interpolate: diffAttrs.indices values must be in [0, A) (A={A})")
             K = len(diffAttrs.idx)
-            didx = torch.tensor(diffAttrs.idx, dtype=torch.int32, device=rast.device)
+            if K <= _lib.DR_INTERPOLATE_HOST_IDX:
+                didx = (ctypes.c_int32 * K)(*diffAttrs.idx)
+            else:
+                didx = torch.tensor(diffAttrs.idx, dtype=torch.int32, device=rast.device)
         return _InterpolateFn.apply(attrf, rastf, rastDB.to(torch.float32).contiguous(), tri32,
                                     didx, K, shared)
 

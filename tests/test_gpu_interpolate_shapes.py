@@ -1,6 +1,7 @@
 """interpolate for any attribute count and any set of derivatives, against
 the CPU oracle: chunks of four attributes with every remainder, derivative
-indices out of order, repeated, and spread over chunks; tiles with more
+indices out of order, repeated, and spread over chunks, as many as travel with
+the launch (32) and more; tiles with more
 vertex rows than the backward's table holds."""
 import numpy as np
 import pytest
@@ -14,7 +15,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("A,diff", [(1, None), (1, "all"), (4, "all"), (4, [3]), (5, None),
                                     (5, [0, 1]), (6, "all"), (7, [6, 0, 6]), (8, [0, 1]),
-                                    (9, [8, 4, 3, 0]), (16, "all"), (17, None), (33, [32, 1])])
+                                    (9, [8, 4, 3, 0]), (16, "all"), (17, None), (33, [32, 1]),
+                                    (40, list(range(32))), (40, list(range(39, 5, -1)))])
 @pytest.mark.parametrize("shared", [True, False])
 @pytest.mark.parametrize("level,H,W", [(2, 50, 41), (6, 33, 64)])  # level 6: ~8 triangles a pixel
 def test_any_shape(A, diff, shared, level, H, W):
