@@ -1,7 +1,9 @@
-"""ctypes binding of libdiffrast_mi355x.so (the C ABI in include/diffrast_mi355x.h).
+"""Binding of libdiffrast_mi355x.so (the C ABI in include/diffrast_mi355x.h):
+ctypes for single calls, and `_torch_ops.so`, the compiled autograd nodes of
+the differentiable ops over the same library.
 
-There is no fallback: if the library is missing or cannot be loaded, every
-op raises.
+There is no fallback: if either is missing or cannot be loaded, every op
+raises.
 """
 from __future__ import annotations
 
@@ -69,6 +71,7 @@ DR_INTERPOLATE_HOST_IDX = 32
 ABI_VERSION = 1
 
 _lib = None
+_ops = None
 
 
 def load():
@@ -88,6 +91,23 @@ def load():
         raise RuntimeError("diffrast: ABI version mismatch")
     _lib = lib
     return lib
+
+
+def ops():
+    """The compiled autograd nodes (csrc/torch_ops.cpp) over the library;
+    raises if they are missing."""
+    global _ops
+    if _ops is not None:
+        return _ops
+    load()
+    try:
+        from . import _torch_ops
+    except ImportError as e:
+        raise RuntimeError(f"diffrast: _torch_ops.so is not built for this torch "
+                           f"(run `make -C mlx-swift-diffrast_amd`): {e}") from e
+    _torch_ops.load(LIB_PATH)
+    _ops = _torch_ops
+    return _ops
 
 
 def check(rc: int) -> None:

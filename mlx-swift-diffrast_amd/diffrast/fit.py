@@ -39,34 +39,10 @@ def _stream():
 # loss
 # ---------------------------------------------------------------------------
 
-class _MSEFn(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, out, target):
-        lib = _lib.load()
-        loss = torch.empty((), device=out.device, dtype=torch.float32)
-        d_out = torch.empty_like(out) if ctx.needs_input_grad[0] else None
-        _lib.check(lib.dr_mse_loss(_ptr(out), _ptr(target), out.numel(), _ptr(loss),
-                                   _ptr(d_out), _stream()))
-        ctx.save_for_backward(d_out)
-        return loss
-
-    @staticmethod
-    def backward(ctx, g):
-        (d_out,) = ctx.saved_tensors
-        return d_out * g, None
-
-
 def mse_loss(out: torch.Tensor, target: torch.Tensor) -> torch.Tensor:
     """Mean of (out - target)^2 over every element (ColorFitExample/main.swift:62-66).
     Differentiable in `out`; the gradient is formed by the same kernel."""
-    if tuple(out.shape) != tuple(target.shape):
-        raise ValueError(f"mse_loss: shapes differ ({list(out.shape)} vs {list(target.shape)})")
-    if not out.is_cuda or not target.is_cuda:
-        raise ValueError("mse_loss: tensors must be on a ROCm device")
-    if out.numel() == 0:
-        raise ValueError("mse_loss: empty tensors")
-    return _MSEFn.apply(out.to(torch.float32).contiguous(),
-                        target.detach().to(torch.float32).contiguous())
+    return _lib.ops().mse_loss(out, target)
 
 
 # ---------------------------------------------------------------------------

@@ -1,0 +1,114 @@
+"""The ops as autograd nodes: what a Python autograd function over the same
+calls did with hooks on saved tensors, in-place changes, transforms, partial
+and missing cotangents, and other threads and streams."""
+import threading
+
+import numpy as np
+import pytest
+
+import scenes
+from parity import dev, host, torch_dev
+
+pytestmark = pytest.mark.gpu
+
+
+def scene():
+    sc = scenes.textured_icosphere(N=2, H=40, W=36, level=2, tex_size=16)
+    return dev(sc["pos"]), dev(sc["tri"]), dev(sc["uv"]), dev(sc["tex"])
+
+
+def chain(pos, tri, uv, tex):
+    from diffrast import DiffRast
+    rast, db = DiffRast.rasterize(pos, tri, (40, 36))
+    a, da = DiffRast.interpolate(uv, rast, tri, rastDB=db, diffAttrs=[0, 1])
+    col = DiffRast.texture(tex, a, uvDA=da, filterMode="linear-mipmap-linear", boundaryMode="clamp")
+    return DiffRast.antialias(col, rast, pos, tri)
+
+
+def test_saved_tensor_hooks_are_called():
+    torch = torch_dev()
+    pos, tri, uv, tex = scene()
+    pos.requires_grad_(True)
+    ref = torch.autograd.grad(chain(pos, tri, uv, tex).square().sum(), pos)[0]
+    seen = [0, 0]
+
+    def pack(t):
+        seen[0] += 1
+        return t.cpu()
+
+    def unpack(t):
+        seen[1] += 1
+        return t.cuda()
+    with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+        out = chain(pos, tri, uv, tex).square().sum()
+    got = torch.autograd.grad(out, pos)[0]
+    assert seen[0] >= 15 and seen[1] >= 15
+    np.testing.assert_allclose(host(got), host(ref), rtol=1e-5, atol=1e-5 * float(ref.abs().max()))
+
+
+def test_in_place_change_is_refused():
+    torch = torch_dev()
+    pos, tri, uv, tex = scene()
+    uv2 = uv.requires_grad_(True).clone()
+    out = chain(pos, tri, uv2, tex)
+    uv2.add_(1.0)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        out.sum().backward()
+
+
+def test_transforms_are_refused():
+    torch = torch_dev()
+    from diffrast import DiffRast
+    pos, tri, uv, tex = scene()
+    with pytest.raises(Exception):
+        torch.func.vmap(lambda t: DiffRast.rasterize(t, tri, (8, 8))[0])(pos[None])
+    with pytest.raises(Exception):
+        torch.func.jvp(lambda t: DiffRast.rasterize(t, tri, (8, 8))[0], (pos,), (pos,))
+
+
+def test_partial_cotangents():
+    """Only one of an op's outputs used; a leaf that gets no gradient."""
+    torch = torch_dev()
+    from diffrast import DiffRast
+    pos, tri, uv, tex = scene()
+    pos.requires_grad_(True), uv.requires_grad_(True)
+    rast, db = DiffRast.rasterize(pos, tri, (40, 36))
+    g = torch.randn_like(rast)
+    one = torch.autograd.grad(rast, pos, g, retain_graph=True)[0]
+    both = torch.autograd.grad([rast, db], pos, [g, torch.zeros_like(db)], retain_graph=True)[0]
+    np.testing.assert_array_equal(host(one), host(both))
+    only_db = torch.autograd.grad(db, pos, torch.ones_like(db), retain_graph=True)[0]
+    assert torch.isfinite(only_db).all()
+    a, da = DiffRast.interpolate(uv, rast.detach(), tri, rastDB=db.detach(), diffAttrs="all")
+    da_only = torch.autograd.grad(da, uv, torch.ones_like(da), retain_graph=True)[0]
+    ref = torch.autograd.grad([a, da], uv, [torch.zeros_like(a), torch.ones_like(da)])[0]
+    np.testing.assert_allclose(host(da_only), host(ref), rtol=1e-5, atol=1e-4)
+
+
+def test_threads_and_streams():
+    """Each thread on its own stream, forward and backward, repeatedly: the
+    results of one thread alone."""
+    torch = torch_dev()
+    pos, tri, uv, tex = scene()
+
+    def step(p):
+        p = p.detach().clone().requires_grad_(True)
+        return torch.autograd.grad(chain(p, tri, uv, tex).square().sum(), p)[0]
+    inputs = [pos * (1 + 0.01 * i) for i in range(3)]
+    refs = [host(step(p)) for p in inputs]
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(i):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for _ in range(5):
+                    got = host(step(inputs[i]))
+                    np.testing.assert_allclose(got, refs[i], rtol=1e-4,
+                                               atol=1e-4 * np.abs(refs[i]).max())
+        except Exception as e:  # reported by the main thread
+            bad.append(e)
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(3)]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    assert not bad, bad[0]
