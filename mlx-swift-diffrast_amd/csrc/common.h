@@ -660,25 +660,8 @@ __device__ __forceinline__ void lds_table_add(LdsTableU<NV, CAP>& u, D* dst, con
     if (v[j] != 0.0f) unsafeAtomicAdd(dst + j, (D)v[j]);
 }
 
-// Writes the taken entries out (call after a barrier) and leaves the table
-// cleared; the caller's next barrier orders the reset count before new adds.
-template <int NV, int CAP, typename D = float>
-__device__ __forceinline__ void lds_table_flush(LdsTableU<NV, CAP>& u) {
-  auto& t = u.t;
-  const int m = u.n;
-  for (int i = threadIdx.x; i < m * NV; i += blockDim.x) {
-    const int e = u.slot[i / NV], j = i - (i / NV) * NV;
-    const double v = t.val[j][e];
-    if (v != 0.0) unsafeAtomicAdd((D*)t.key[e] + j, (D)v);
-    t.val[j][e] = 0.0;
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < m; i += blockDim.x) t.key[u.slot[i]] = kEmptyKey;
-  if (threadIdx.x == 0) u.n = 0;
-}
-
-// The same for the last use of a table in a workgroup that ends after it:
-// no barrier and no reset.
+// Writes the taken entries out (call after a barrier), for the last use of a
+// table in a workgroup that ends after it: no barrier and no reset.
 template <int NV, int CAP, typename D = float>
 __device__ __forceinline__ void lds_table_flush_last(LdsTableU<NV, CAP>& u) {
   auto& t = u.t;
