@@ -30,3 +30,33 @@ def test_tile_counts(tiles):
     rr, rdb = O.rasterize(pos, tri, (H, W), max_per_tile=0)
     np.testing.assert_array_equal(host(r), rr)
     np.testing.assert_array_equal(host(db), rdb)
+
+
+def test_large_image_under_capture():
+    """More than 64 KiB of LDS counters inside a HIP graph: every replay, with
+    eager work between them, gives the eager result."""
+    torch = torch_dev()
+    from diffrast import DiffRast
+    rng = np.random.default_rng(3)
+    H, W, T = 2080, 2081, 900
+    xyz = np.repeat(rng.uniform(-1, 1, size=(1, T, 3)), 3, axis=1) + \
+        rng.uniform(-0.05, 0.05, size=(1, 3 * T, 3))
+    pos = dev(np.concatenate([xyz, np.ones((1, 3 * T, 1))], 2).astype(np.float32))
+    tri = dev(np.arange(3 * T, dtype=np.int32).reshape(T, 3))
+    other = dev((xyz * 0.5).astype(np.float32))
+    other = torch.cat([other, torch.ones_like(other[..., :1])], -1).contiguous()
+    ref = host(DiffRast.rasterize(pos, tri, (H, W))[0])
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        for _ in range(2):
+            DiffRast.rasterize(pos, tri, (H, W))
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            out, _ = DiffRast.rasterize(pos, tri, (H, W))
+        for _ in range(3):
+            out.zero_()
+            DiffRast.rasterize(other, tri, (H, W))
+            g.replay()
+            torch.cuda.synchronize()
+            np.testing.assert_array_equal(host(out), ref)
