@@ -5,17 +5,17 @@
 // Small calls are bound by the host: one triangle at 256^2, rasterize ->
 // interpolate -> MSE and back, is nine launches of a few microseconds each,
 // and the same nodes as Python autograd functions over ctypes calls took
-// 112 to 173 us a pass, depending on the host (these: 70 to 93; one view of
-// the textured chain at 512^2: 235 to 355, now 144 to 204).  Each op's semantics (checks, messages,
-// reuse rules) are those of diffrast/ops.py's documentation.
+// 112 to 173 us a pass, depending on the host (these: 70 to 98; one view of
+// the textured chain at 512^2: 235 to 355, now 144 to 208).  Each op's
+// semantics (checks, messages, reuse rules) are those of diffrast/ops.py's
+// documentation.
 #include <dlfcn.h>
 
-#include <c10/core/DeviceGuard.h>
-#include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/extension.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <string>
