@@ -16,6 +16,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "window_box.h"
 
 namespace dr {
 
@@ -961,17 +962,6 @@ __device__ __forceinline__ void slot_box(const TapSlot& q, int& x0, int& x1, int
 }
 
 
-// The wrap mode's window coordinates are the texel coordinates before the
-// wrap (reduced to texels when the window is written out), so a footprint
-// across the texture's border, and a tiled texture's pixels on both sides of
-// a repeat, stay neighbours: with wrapped coordinates their box spans the
-// texture, no window holds it, and the tile's taps all went to the hash
-// table and to device atomics.  Coordinates too far out for the packed
-// 16-bit boxes are taken wrapped, which is the same texel.
-constexpr int kWinCoordMax = 32000;
-__device__ __forceinline__ int win_coord(int t, int wrapped) {
-  return (unsigned)t + kWinCoordMax <= 2u * kWinCoordMax ? t : wrapped;
-}
 // The texel of window coordinate t.
 template <int BND>
 __device__ __forceinline__ int win_texel(int t, int size) {
@@ -1322,9 +1312,8 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
     // its slots' windows from the lanes of their levels.
     const int4 wm = *reinterpret_cast<const int4*>(s_lmask);
     const int lmask = __builtin_amdgcn_readfirstlane(wm.x | wm.y | wm.z | wm.w);
-    // (x0 | y0 << 16) and (width | height << 10 | (pool offset + 1) << 20),
-    // offset + 1 = 0 for no window (a box in the pool has at most 768 texels,
-    // so each of its sides and its offset fit in 10 bits)
+    // (x0 | y0 << 16) and win_pack's word (a box in the pool has at most
+    // kWinTexels texels, so each of its sides and its offset fit in 10 bits)
     int wxy, wsz;
     {
       const int L = lane & 15;
@@ -1341,8 +1330,7 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
       const int x0 = unpack16_lo(px), x1 = -unpack16_hi(px);
       const int y0 = unpack16_lo(py), y1 = -unpack16_hi(py);
       const bool present = L < kMaxLevels && ((lmask >> L) & 1) && x1 >= x0 && y1 >= y0;
-      const int area = present ? (x1 - x0 + 1) * (y1 - y0 + 1) : 0;
-      const int fit = area <= kWinTexels ? area : 0;
+      const int fit = present ? win_fit(x1 - x0 + 1, y1 - y0 + 1, kWinTexels) : 0;
       // inclusive prefix sum of the fitting areas along the row
       int incl = fit;
       int t = dpp_shift<0x111>(incl);
@@ -1353,10 +1341,10 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
       incl += t;
       t = dpp_shift<0x118>(incl);
       incl += t;
-      const bool usable = present && area == fit && incl <= kWinTexels;
+      const bool usable = fit > 0 && incl <= kWinTexels;
       static_assert(kWinTexels < 1024, "window sides and offsets are 10-bit fields");
       wxy = pack16(x0, y0);
-      wsz = usable ? (x1 - x0 + 1) | ((y1 - y0 + 1) << 10) | ((incl - fit + 1) << 20) : 0;
+      wsz = usable ? win_pack(x1 - x0 + 1, y1 - y0 + 1, incl - fit) : 0;
     }
 
     // -- accumulate: runs of one footprint along a pixel row are summed
@@ -1407,7 +1395,7 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
         // the image for the zero boundary) may lie outside it, and its
         // coordinates are clamped into the box, where it adds 0.
         const int wx = unpack16_lo(sxy), wy = unpack16_hi(sxy);
-        const int ww = ssz & 0x3ff, wh = (ssz >> 10) & 0x3ff, sbase = (ssz >> 20) - 1;
+        const int ww = win_w(ssz), wh = win_h(ssz), sbase = win_at(ssz);
         const int cx0 = min(max(q[li].ix0 - wx, 0), ww - 1);
         const int cx1 = min(max(q[li].ix1 - wx, 0), ww - 1);
         const int r0 = sbase + min(max(q[li].iy0 - wy, 0), wh - 1) * ww;
@@ -1470,8 +1458,7 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
         continue;
       }
       const int xy = __builtin_amdgcn_readlane(wxy, k);
-      flush_window(k, unpack16_lo(xy), unpack16_hi(xy), sz & 0x3ff, (sz >> 10) & 0x3ff,
-                   (sz >> 20) - 1);
+      flush_window(k, unpack16_lo(xy), unpack16_hi(xy), win_w(sz), win_h(sz), win_at(sz));
     }
     // -- bilinear: a box larger than the pool (a texture minified by up to a
     //    few texels a pixel) goes through it in bands of whole rows: a band's
@@ -1491,7 +1478,7 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
       py = __builtin_amdgcn_readfirstlane(py);
       const int x0 = unpack16_lo(px), y0 = unpack16_lo(py);
       const int bw = -unpack16_hi(px) - x0 + 1, bh = -unpack16_hi(py) - y0 + 1;
-      const int rows = bw <= kWinTexels ? kWinTexels / bw : 0;
+      const int rows = win_rows(bw, kWinTexels);
       if (rows * kWinBands >= bh) {  // (rows 0: too wide)
         float v[4 * CT];
         const bool adds = run_totals(0, use0, v);
@@ -1905,8 +1892,7 @@ __global__ void __launch_bounds__(256, 3) k_tex_bwd_many(TexBwdArgs A, int total
       }
     }
     constexpr int kMaxTexels = kManyPool / 4;  // with four channels in the pool
-    const int64_t area64 = (int64_t)bw * bh;
-    const int fit = area64 <= kMaxTexels ? (int)area64 : 0;
+    const int fit = win_fit(bw, bh, kMaxTexels);  // (no box: 0)
     int incl = fit;  // prefix sum of the fitting areas along the 16-lane row
     {
       int t = dpp_shift<0x111>(incl);

@@ -1,0 +1,44 @@
+// Integer arithmetic of the texture backward's LDS windows (k_tex_bwd_win,
+// k_tex_bwd_many in texture.hip), shared with a host-side check over every
+// box size the window coordinates allow (tests/texture_windows.cpp).
+#pragma once
+
+#ifdef __HIPCC__
+#define DR_WB_FN __host__ __device__ __attribute__((always_inline)) inline
+#else
+#define DR_WB_FN inline
+#endif
+
+namespace dr {
+
+// The wrap mode's window coordinates are the texel coordinates before the
+// wrap (reduced to texels when the window is written out), so a footprint
+// across the texture's border, and a tiled texture's pixels on both sides of
+// a repeat, stay neighbours: with wrapped coordinates their box spans the
+// texture and no window holds it.  Coordinates too far out for the packed
+// 16-bit boxes are taken wrapped, which is the same texel.
+constexpr int kWinCoordMax = 32000;
+DR_WB_FN int win_coord(int t, int wrapped) {
+  return (unsigned)t + kWinCoordMax <= 2u * kWinCoordMax ? t : wrapped;
+}
+
+// Texels of a w x h box (0 x 0: no box) when a pool of `cap` texels holds it,
+// else 0.  A side of wrap coordinates is at most 32767 + kWinCoordMax + 1 =
+// 64768, so the product of two does not fit 32 bits: the sides are held to
+// the pool first.
+DR_WB_FN int win_fit(int w, int h, int cap) {
+  if (w > cap || h > cap) return 0;
+  return w * h <= cap ? w * h : 0;
+}
+
+// A window's width, height and place in the pool (all below 1024, at >= 0)
+// in one word; 0 is no window.
+DR_WB_FN int win_pack(int w, int h, int at) { return w | (h << 10) | ((at + 1) << 20); }
+DR_WB_FN int win_w(int p) { return p & 0x3ff; }
+DR_WB_FN int win_h(int p) { return (p >> 10) & 0x3ff; }
+DR_WB_FN int win_at(int p) { return (p >> 20) - 1; }
+
+// Whole rows of a box w texels wide that the pool holds (0: too wide).
+DR_WB_FN int win_rows(int w, int cap) { return w <= cap ? cap / w : 0; }
+
+}  // namespace dr

@@ -131,3 +131,20 @@ def test_pyramid_sizes(H, W, C):
     assert len(got) == len(ref)
     for a, b in zip(got, ref):
         np.testing.assert_array_equal(host(a), b)
+
+
+# scattered uv over a tiled texture: a tile's box is up to 49,152 texels on a
+# side, more than 2^31 of them together
+@pytest.mark.parametrize("filt,C", [("linear", 1), ("linear", 3), ("linear", 4), ("linear", 6),
+                                    ("nearest", 1), ("nearest", 3), ("nearest", 6),
+                                    ("linear-mipmap-linear", 3), ("linear-mipmap-linear", 4),
+                                    ("linear-mipmap-nearest", 4), ("linear-mipmap-linear", 6)])
+def test_scattered_wrap(filt, C):
+    torch_dev()
+    rng = np.random.default_rng(C)
+    S = 2048
+    uv = rng.uniform(-12.0, 12.0, size=(2, 17, 33, 2)).astype(np.float32)
+    uv[:, :8] *= np.float32(0.01)  # and a part whose boxes fit
+    da = rng.uniform(0.9, 1.1, size=(2, 17, 33, 4)).astype(np.float32) * np.float32(1.1 / S)
+    tex = rng.random((1, S, S, C)).astype(np.float32)
+    check(rng, tex, uv, da, filt, "wrap")
