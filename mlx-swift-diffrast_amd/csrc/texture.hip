@@ -944,24 +944,6 @@ constexpr int kWinBands = 4;
 // lane).
 constexpr int kWinFewRuns = 12;
 
-struct TapSlot {
-  int k;         // level
-  float scale;   // (1 - frac) or frac; 0 = unused
-  int ix0, ix1, iy0, iy1;
-  float w00, w10, w01, w11;
-};
-
-__device__ __forceinline__ void slot_box(const TapSlot& q, int& x0, int& x1, int& y0, int& y1) {
-  const bool c0 = q.w00 != 0.0f || q.w01 != 0.0f, c1 = q.w10 != 0.0f || q.w11 != 0.0f;
-  const bool r0 = q.w00 != 0.0f || q.w10 != 0.0f, r1 = q.w01 != 0.0f || q.w11 != 0.0f;
-  x0 = 0x7fffffff; x1 = -1; y0 = 0x7fffffff; y1 = -1;
-  if (c0) { x0 = min(x0, q.ix0); x1 = max(x1, q.ix0); }
-  if (c1) { x0 = min(x0, q.ix1); x1 = max(x1, q.ix1); }
-  if (r0) { y0 = min(y0, q.iy0); y1 = max(y1, q.iy0); }
-  if (r1) { y0 = min(y0, q.iy1); y1 = max(y1, q.iy1); }
-}
-
-
 // The texel of window coordinate t.
 template <int BND>
 __device__ __forceinline__ int win_texel(int t, int size) {

@@ -1,8 +1,9 @@
 // Host-side check of the texture backward's window arithmetic
 // (window_box.h) over every side a box of window coordinates can have: the
 // area that is taken for a window against the exact product, the packed
-// word against its fields, and the bands' rows against the pool.  Prints the
-// number of boxes; exits 1 on the first violation.
+// word against its fields, the bands' rows against the pool, and a
+// footprint's box against its taps.  Prints the number of boxes; exits 1 on
+// the first violation.
 #include <cstdint>
 #include <cstdio>
 #include <random>
@@ -61,6 +62,32 @@ int main() {
       if (c < -kWinCoordMax || c + 1 > 32767 || ((c % size) + size) % size != wrapped)
         return fail("coordinate", (int)t, size, 0);
     }
+  // a footprint's box is that of its taps with a nonzero weight, on either
+  // side of the origin
+  std::uniform_int_distribution<int> coord(-kWinCoordMax, 32766), bits(0, 15), far(0, 3);
+  for (int i = 0; i < 1000000; ++i) {
+    const int span = far(rng) ? 20 : kWinCoordMax;  // mostly around the origin
+    TapSlot q{};
+    q.ix0 = coord(rng) % span; q.ix1 = bits(rng) ? q.ix0 + 1 : coord(rng) % span;
+    q.iy0 = coord(rng) % span; q.iy1 = bits(rng) ? q.iy0 + 1 : coord(rng) % span;
+    const int m = bits(rng);
+    q.w00 = m & 1 ? 0.25f : 0.0f; q.w10 = m & 2 ? 0.25f : 0.0f;
+    q.w01 = m & 4 ? 0.25f : 0.0f; q.w11 = m & 8 ? -0.25f : 0.0f;
+    int x0, x1, y0, y1;
+    slot_box(q, x0, x1, y0, y1);
+    if (m == 0) {
+      if (x1 >= x0 || y1 >= y0) return fail("box of nothing", q.ix0, q.iy0, 0);
+      continue;
+    }
+    int a0 = 1 << 30, a1 = -(1 << 30), b0 = 1 << 30, b1 = -(1 << 30);
+    for (int t = 0; t < 4; ++t) {
+      if (!((m >> t) & 1)) continue;
+      const int x = t & 1 ? q.ix1 : q.ix0, y = t & 2 ? q.iy1 : q.iy0;
+      a0 = x < a0 ? x : a0; a1 = x > a1 ? x : a1;
+      b0 = y < b0 ? y : b0; b1 = y > b1 ? y : b1;
+    }
+    if (x0 != a0 || x1 != a1 || y0 != b0 || y1 != b1) return fail("box", q.ix0, q.iy0, m);
+  }
   std::printf("%ld boxes, %ld windows\n", boxes, fits);
   return 0;
 }
