@@ -990,6 +990,11 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
   constexpr bool kCube = BND == DR_BOUNDARY_CUBE;
   constexpr bool kSameUv = BND == DR_BOUNDARY_WRAP || FILTER == DR_FILTER_NEAREST;
   constexpr bool kOneLevel = kCube || FILTER == DR_FILTER_NEAREST || FILTER == DR_FILTER_LINEAR;
+  // Taps of a footprint.  The nearest filter has one, of weight 1 (its mask
+  // goes into the cotangent): three more of weight 0 would put 0 * inf into
+  // texels that it does not sample, and cost their LDS additions.
+  constexpr int kTaps = FILTER == DR_FILTER_NEAREST ? 1 : 4;
+  constexpr int kRows = kTaps == 1 ? 1 : 2, kRowVals = (kTaps == 1 ? 1 : 2) * CT;  // texel rows
   const bool shared_tex = A.tex_stride == 0;
   const int wave = tid >> 6, lane = tid & 63;
   const int tiles = A.ntx * A.nty;
@@ -1105,7 +1110,18 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
       } else {
         q[li].ix0 = b.ix0; q[li].ix1 = b.ix1; q[li].iy0 = b.iy0; q[li].iy1 = b.iy1;
       }
-      const bool on = valid && q[li].scale != 0.0f;
+      bool on = valid && q[li].scale != 0.0f;
+      if constexpr (FILTER == DR_FILTER_NEAREST) {
+        bool any = false;  // a nonzero value, or NaN (0 * inf outside the image)
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+          g[c] *= b.w00;
+          any = any || g[c] != 0.0f;
+        }
+        on = on && any;
+        w00 = 1.0f;
+        w10 = w01 = w11 = 0.0f;
+      }
       q[li].w00 = on ? w00 : 0.0f; q[li].w10 = on ? w10 : 0.0f;
       q[li].w01 = on ? w01 : 0.0f; q[li].w11 = on ? w11 : 0.0f;
       // A footprint collapsed onto one texel (clamped at a corner; every
@@ -1251,7 +1267,7 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
         }
         const float z = wave_sum4(x);  // lane l: total of value l & 3
         const float zc = __shfl(z, (lane >> 2) & 3, kWave);
-        if (kSameUv) {  // lane 4c + t: channel c, tap t
+        if (kSameUv && kTaps == 4) {  // lane 4c + t: channel c, tap t
           const float wt = leader_weight(q[0], leader, lane & 3);
           if (lane < 4 * CT) acc.v += wt * zc;
         } else {
@@ -1332,10 +1348,10 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
     // -- accumulate: runs of one footprint along a pixel row are summed
     //    first (lanes of one LDS atomic on one address are serialised), the
     //    run's last lane adds the totals ----------------------------------------
-    // Slot li's run totals v (tap-major, 4 * CT values, all zero in a lane
+    // Slot li's run totals v (tap-major, kTaps * CT values, all zero in a lane
     // that is not the tail of a run of `u` lanes' footprints); whether this
     // lane is one.  Every lane executes it.
-    auto run_totals = [&](int li, bool u, float (&v)[4 * CT]) -> bool {
+    auto run_totals = [&](int li, bool u, float (&v)[kTaps * CT]) -> bool {
       const float sc = mip ? q[li].scale : 1.0f;
       // level and the four texel coordinates (each < 32767 on the window
       // path) fix the taps; an unused slot gets a key no footprint has
@@ -1354,9 +1370,9 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
 #pragma unroll
       for (int c = 0; c < CT; ++c) gs[c] = !u ? 0.0f : g[c] * sc;
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < kTaps; ++t)
 #pragma unroll
-        for (int c = 0; c < CT; ++c) v[t * CT + c] = wt[t] * gs[c];
+        for (int c = 0; c < CT; ++c) v[t * CT + c] = kTaps == 1 ? gs[c] : wt[t] * gs[c];
       row_run_scan_n(run, v, maxlen);
       return u && run.tail;
     };
@@ -1368,7 +1384,7 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
       // the window of level k (every lane executes the permutes)
       const int sxy = __builtin_amdgcn_ds_bpermute(k << 2, wxy);
       const int ssz = __builtin_amdgcn_ds_bpermute(k << 2, wsz);
-      float v[4 * CT];
+      float v[kTaps * CT];
       const bool adds = run_totals(li, u, v);
       if (adds && ssz != 0) {
         // window indices of the four taps.  The box holds every tap with a
@@ -1384,7 +1400,7 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
         const int r1 = sbase + min(max(q[li].iy1 - wy, 0), wh - 1) * ww;
         const int o[4] = {r0 + cx0, r0 + cx1, r1 + cx0, r1 + cx1};  // < sbase + area
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
+        for (int t = 0; t < kTaps; ++t)
 #pragma unroll
           for (int c = 0; c < CT; ++c)
             atomicAdd(win + c * kWinTexels + o[t], (double)v[t * CT + c]);
@@ -1462,7 +1478,7 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
       const int bw = -unpack16_hi(px) - x0 + 1, bh = -unpack16_hi(py) - y0 + 1;
       const int rows = win_rows(bw, kWinTexels);
       if (rows * kWinBands >= bh) {  // (rows 0: too wide)
-        float v[4 * CT];
+        float v[kTaps * CT];
         const bool adds = run_totals(0, use0, v);
         const int cx0 = min(max(q[0].ix0 - x0, 0), bw - 1);
         const int cx1 = min(max(q[0].ix1 - x0, 0), bw - 1);
@@ -1474,13 +1490,14 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
           const int nr = min(rows, bh - b0);
           __syncthreads();  // the pool is written out (and cleared)
 #pragma unroll
-          for (int row = 0; row < 2; ++row) {
+          for (int row = 0; row < kRows; ++row) {
             const int r = (row == 0 ? cy0 : cy1) - b0;
             if (adds && (unsigned)r < (unsigned)nr) {
 #pragma unroll
               for (int c = 0; c < CT; ++c) {
-                atomicAdd(win + c * kWinTexels + r * bw + cx0, (double)v[row * 2 * CT + c]);
-                atomicAdd(win + c * kWinTexels + r * bw + cx1, (double)v[row * 2 * CT + CT + c]);
+                atomicAdd(win + c * kWinTexels + r * bw + cx0, (double)v[row * kRowVals + c]);
+                if constexpr (kTaps == 4)
+                  atomicAdd(win + c * kWinTexels + r * bw + cx1, (double)v[row * kRowVals + CT + c]);
               }
             }
           }
@@ -1491,7 +1508,7 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
       }
     }
     // -- levels without a window: each run's two texel rows straight to
-    //    memory.  A wave lays a row's 2 * CT totals of its 64 lanes out in
+    //    memory.  A wave lays a row's kRowVals totals of its 64 lanes out in
     //    its part of the pool and issues them with consecutive lanes on
     //    consecutive addresses (one cache-line request a row instead of one a
     //    value: the atomic units take requests, about 21 G/s), so a minified
@@ -1507,7 +1524,7 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
         const int k = q[li].k;
         const bool u = (li == 0 ? use0 : use1) && ((nowin >> k) & 1);
         if (__ballot(u) == 0) continue;
-        float v[4 * CT];
+        float v[kTaps * CT];
         const bool adds = run_totals(li, u, v);
         const int Wk = level_w(k), Hk = level_h(k);
         const int X0 = win_texel<BND>(q[li].ix0, Wk), X1 = win_texel<BND>(q[li].ix1, Wk);
@@ -1519,7 +1536,7 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
         if (__popcll(__ballot(adds)) <= kWinFewRuns) {
           if (adds) {
 #pragma unroll
-            for (int t = 0; t < 4; ++t)
+            for (int t = 0; t < kTaps; ++t)
 #pragma unroll
               for (int c = 0; c < CT; ++c) {
                 const float x = v[t * CT + c];
@@ -1530,16 +1547,16 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
         }
         staged = true;
 #pragma unroll
-        for (int row = 0; row < 2; ++row) {
+        for (int row = 0; row < kRows; ++row) {
           const uint64_t p = (uint64_t)(lv + (row == 0 ? o0 : o1));
 #pragma unroll
-          for (int j = 0; j < 2 * CT; ++j)
-            st[lane * 2 * CT + j] = adds ? (double)v[row * 2 * CT + j] : 0.0;
+          for (int j = 0; j < kRowVals; ++j)
+            st[lane * kRowVals + j] = adds ? (double)v[row * kRowVals + j] : 0.0;
           __builtin_amdgcn_wave_barrier();  // (LDS is ordered within a wave)
           __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
 #pragma unroll 1
-          for (int i = 0; i < 2 * CT; ++i) {
-            const int e = (i * 64 + lane) / (2 * CT), j = (i * 64 + lane) - e * 2 * CT;
+          for (int i = 0; i < kRowVals; ++i) {
+            const int e = (i * 64 + lane) / kRowVals, j = (i * 64 + lane) - e * kRowVals;
             const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute(e << 2, (int)(uint32_t)p);
             const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_bpermute(e << 2, (int)(p >> 32));
             const int ed = __builtin_amdgcn_ds_bpermute(e << 2, dx);
@@ -1553,7 +1570,7 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
       }
       if (staged) {  // zero again before the next barrier
 #pragma unroll
-        for (int j = 0; j < 2 * CT; ++j) st[lane * 2 * CT + j] = 0.0;
+        for (int j = 0; j < kRowVals; ++j) st[lane * kRowVals + j] = 0.0;
       }
     }
   }
@@ -1665,8 +1682,9 @@ struct ManyHot {
   float w00, w10, w01, w11;
 };
 
+template <int TAPS>
 __device__ __forceinline__ void hot_flush(const ManyHot& h, int C, const double* s) {
-  for (int i = lane_id(); i < 4 * C; i += 64) {
+  for (int i = lane_id(); i < TAPS * C; i += 64) {
     const int t = i / C, c = i - t * C;
     const float w = t == 0 ? h.w00 : t == 1 ? h.w10 : t == 2 ? h.w01 : h.w11;
     const float v = (float)((double)w * s[c]);
@@ -1690,6 +1708,7 @@ __global__ void __launch_bounds__(256, 3) k_tex_bwd_many(TexBwdArgs A, int total
   __syncthreads();
   constexpr bool kCube = BND == DR_BOUNDARY_CUBE;
   constexpr bool mip = FILTER == DR_FILTER_LINEAR_MIPMAP_LINEAR || FILTER == DR_FILTER_LINEAR_MIPMAP_NEAREST;
+  constexpr int kTaps = FILTER == DR_FILTER_NEAREST ? 1 : 4;  // (k_tex_bwd_win)
   const MipDesc& md = A.md;
   const int C = A.C;
   // texels are read for the gradients of uv and the LOD only
@@ -1802,7 +1821,7 @@ __global__ void __launch_bounds__(256, 3) k_tex_bwd_many(TexBwdArgs A, int total
         float* base = dlevel_ptr(lk);
         if (!(hot.on && hot.ux == lux && hot.uy == luy && hot.base == base)) {
           if (hot.on) {
-            hot_flush(hot, C, s_hot[wave]);
+            hot_flush<kTaps>(hot, C, s_hot[wave]);
             for (int c = lane; c < C; c += 64) s_hot[wave][c] = 0.0;
           }
           hot.on = true;
@@ -1968,13 +1987,24 @@ __global__ void __launch_bounds__(256, 3) k_tex_bwd_many(TexBwdArgs A, int total
               }
             }
           }
+          if constexpr (FILTER == DR_FILTER_NEAREST && BND == DR_BOUNDARY_ZERO) {
+            // outside the image: 0 * g is 0, or NaN where g is not finite
+            if (valid && mask[0] == 0) {
+              float* p = dlevel_ptr(0) + ((int64_t)ty0[0] * A.Wt + tx0[0]) * C + c;
+#pragma unroll
+              for (int j = 0; j < 4; ++j) {
+                const float x = 0.0f * g[j];
+                if (x != 0.0f) unsafeAtomicAdd(p + j, x);
+              }
+            }
+          }
           const bool us = li == 0 ? use0 : use1;
           if (__ballot(us) == 0ull) continue;
           const float sc = mip ? q[li].scale : 1.0f;
           const float wt[4] = {q[li].w00, q[li].w10, q[li].w01, q[li].w11};
-          float v[16];
+          float v[kTaps * 4];
 #pragma unroll
-          for (int t = 0; t < 4; ++t)
+          for (int t = 0; t < kTaps; ++t)
 #pragma unroll
             for (int j = 0; j < 4; ++j) v[t * 4 + j] = us ? wt[t] * (g[j] * sc) : 0.0f;
           row_run_scan_n(run[li], v, maxlen[li]);
@@ -1984,7 +2014,7 @@ __global__ void __launch_bounds__(256, 3) k_tex_bwd_many(TexBwdArgs A, int total
             for (int j = 0; j < 4; ++j) {
               if (j < nc) {
 #pragma unroll
-                for (int t = 0; t < 4; ++t) atomicAdd(w + j * texels + o[li][t], (double)v[t * 4 + j]);
+                for (int t = 0; t < kTaps; ++t) atomicAdd(w + j * texels + o[li][t], (double)v[t * 4 + j]);
               }
             }
           }
@@ -2148,7 +2178,7 @@ __global__ void __launch_bounds__(256, 3) k_tex_bwd_many(TexBwdArgs A, int total
       for (int c = lane; c < C; c += 64) s_hot[wave][c] += s_hot[w][c];
   __builtin_amdgcn_wave_barrier();  // (LDS is ordered within a wave)
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  hot_flush(hot, C, s_hot[wave]);
+  hot_flush<kTaps>(hot, C, s_hot[wave]);
 }
 
 // Texture.swift:156: level k = 2x2 mean of level k-1.  Builds up to five

@@ -148,3 +148,39 @@ def test_scattered_wrap(filt, C):
     da = rng.uniform(0.9, 1.1, size=(2, 17, 33, 4)).astype(np.float32) * np.float32(1.1 / S)
     tex = rng.random((1, S, S, C)).astype(np.float32)
     check(rng, tex, uv, da, filt, "wrap")
+
+
+def nonfinite(rng, g):
+    """g with a few infinities and NaNs."""
+    g = g.copy()
+    flat = g.reshape(-1)
+    at = rng.choice(flat.size, size=24, replace=False)
+    flat[at[:9]], flat[at[9:18]], flat[at[18:]] = np.inf, -np.inf, np.nan
+    return g
+
+
+def assert_same_nonfinite(got, ref, what):
+    """NaN and infinities where the oracle has them, close elsewhere."""
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(ref), err_msg=what)
+    np.testing.assert_array_equal(got[np.isinf(ref)], ref[np.isinf(ref)], err_msg=what)
+    fin = np.isfinite(ref)
+    assert_grad_close(got[fin], ref[fin], what)
+
+
+# a cotangent that is not finite reaches the texel that was sampled and no
+# other; outside the zero boundary's image it is masked to 0 * inf
+@pytest.mark.parametrize("C", [1, 3, 4, 6, 129])
+@pytest.mark.parametrize("bnd", ["wrap", "clamp", "zero"])
+@pytest.mark.parametrize("texels", [0.3, 3.0, 12.0])
+def test_nearest_nonfinite_cotangent(C, bnd, texels):
+    torch_dev()
+    from diffrast import DiffRast
+    rng = np.random.default_rng(C)
+    Hi, Wi, Ht, Wt = 33, 50, 160, 192
+    uv, _ = smooth_uv(rng, 2, Hi, Wi, texels * Wi / Wt / 1.5, 0.2, (0.0, 0.0))
+    tex = rng.random((1, Ht, Wt, C)).astype(np.float32)
+    g = nonfinite(rng, rng.normal(size=(2, Hi, Wi, C)).astype(np.float32))
+    t = dev(tex).requires_grad_(True)
+    DiffRast.texture(t, dev(uv), filterMode="nearest", boundaryMode=bnd).backward(dev(g))
+    ref = O.texture_vjp(tex, uv, g, filterMode="nearest", boundaryMode=bnd)[0]
+    assert_same_nonfinite(host(t.grad), ref, "d_tex")
