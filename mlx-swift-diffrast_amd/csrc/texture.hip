@@ -1582,7 +1582,7 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
 // four channels of a pixel, consecutive threads consecutive channels, so
 // texel reads and output writes are whole cache lines; one thread per pixel
 // walking its channels read four bytes a lane at a stride of C floats
-// (2 x 768^2 x 16, trilinear: 286 -> 40 us).
+// (2 x 768^2 x 16, trilinear: 286 -> 49 us, 42 without the level of weight 0).
 // ---------------------------------------------------------------------------
 
 // The bilinear sample of channels [c, c + nc) of one level, in tex_fwd_px's
@@ -1643,12 +1643,11 @@ __global__ void __launch_bounds__(256) k_tex_fwd_many(
           return sample_chunk(lv, Wk, C, bilin(uvp.x, uvp.y, Wk, Hk, BND), c, nc);
         };
         const float w0 = 1.0f - ld.frac, w1 = ld.frac;
-        o = level(ld.k0);
-        o = make_float4(w0 * o.x, w0 * o.y, w0 * o.z, w0 * o.w);
-        if (w1 != 0.0f) {  // (a zero-weight level is not read)
-          const float4 p = level(ld.k1);
-          o = make_float4(o.x + w1 * p.x, o.y + w1 * p.y, o.z + w1 * p.z, o.w + w1 * p.w);
-        }
+        // (a level of weight 0 counts where its texels are not finite: 0 * inf
+        // is NaN; it is read unless it is the first level again)
+        const float4 s0 = level(ld.k0), s1 = ld.k1 != ld.k0 ? level(ld.k1) : s0;
+        o = make_float4(w0 * s0.x + w1 * s1.x, w0 * s0.y + w1 * s1.y, w0 * s0.z + w1 * s1.z,
+                        w0 * s0.w + w1 * s1.w);
       }
     }
     st_chunk(out + pix * C + c, o, nc);
@@ -1662,7 +1661,9 @@ __global__ void __launch_bounds__(256) k_tex_fwd_many(
 // a texel's channels as one run of memory.  One footprint set-up serves all
 // channels, and d_uv and the LOD's gradient sum over them in registers.  The
 // general kernel's wave probes and one device atomic per tap and channel
-// took 3,453 us at 2 x 768^2 x 16, trilinear; this takes 180 (188 with the
+// took 3,453 us at 2 x 768^2 x 16, trilinear; this takes 191 (182 without the
+// terms of weight 0, which matter for texels that are not finite; there, 188
+// with the
 // direct way's cotangents loaded one pixel at a time; 264 at four waves per
 // SIMD, which spills 46 registers; 211 with two and a pool twice the size).
 // Cube maps: k is the face, one level each.
@@ -1751,7 +1752,6 @@ __global__ void __launch_bounds__(256, 3) k_tex_bwd_many(TexBwdArgs A, int total
     float s = 1.0f;
     const bool scaled = mip && (A.bias_map != nullptr || A.has_bias);
     float2 uvp = make_float2(0.0f, 0.0f);
-    bool need1 = false;
     q[0].k = q[1].k = 0;
     q[0].scale = 1.0f;
     q[1].scale = 0.0f;
@@ -1771,7 +1771,6 @@ __global__ void __launch_bounds__(256, 3) k_tex_bwd_many(TexBwdArgs A, int total
       q[0].scale = 1.0f - ld.frac;
       q[1].k = ld.k1;
       q[1].scale = ld.frac;
-      need1 = ld.frac != 0.0f || (FILTER == DR_FILTER_LINEAR_MIPMAP_LINEAR && ld.k0 != 0);
     }
 #pragma unroll
     for (int li = 0; li < (mip ? 2 : 1); ++li) {
@@ -1948,7 +1947,6 @@ __global__ void __launch_bounds__(256, 3) k_tex_bwd_many(TexBwdArgs A, int total
 
     // -- channels: d_uv and the LOD samples, the windows' sums, their flush -----
     float dfx_total = 0.0f, dfy_total = 0.0f, samp[2] = {0.0f, 0.0f};
-    const bool lod0 = FILTER != DR_FILTER_LINEAR_MIPMAP_LINEAR || (q[0].k == 0 && q[1].scale == 0.0f);
     float dfx[2] = {0.0f, 0.0f}, dfy[2] = {0.0f, 0.0f};
 #pragma unroll 1
     for (int c0 = 0; c0 < C; c0 += cap_c) {
@@ -1960,8 +1958,9 @@ __global__ void __launch_bounds__(256, 3) k_tex_bwd_many(TexBwdArgs A, int total
         const float g[4] = {g4.x, g4.y, g4.z, g4.w};
 #pragma unroll
         for (int li = 0; li < (mip ? 2 : 1); ++li) {
-          const bool flat = BND != DR_BOUNDARY_ZERO && tx0[li] == tx1[li] && ty0[li] == ty1[li] && lod0;
-          if (want && valid && (li == 0 || need1) && !flat) {
+          // (also a level of weight 0, and a footprint on one texel: their
+          // terms are 0 unless a texel is not finite)
+          if (want && valid) {
             const int k = q[li].k, Wk = level_w(k);
             const float* lv = level_ptr(k) + c;
             const uint32_t ra = (uint32_t)ty0[li] * (uint32_t)Wk, rb = (uint32_t)ty1[li] * (uint32_t)Wk;
@@ -1975,8 +1974,8 @@ __global__ void __launch_bounds__(256, 3) k_tex_bwd_many(TexBwdArgs A, int total
             const float sc = mip ? q[li].scale : 1.0f;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-              const float t00 = (mask[li] & 1) ? a0[j] : 0.0f, t10 = (mask[li] & 2) ? a1[j] : 0.0f;
-              const float t01 = (mask[li] & 4) ? a2[j] : 0.0f, t11 = (mask[li] & 8) ? a3[j] : 0.0f;
+              const float t00 = a0[j] * (float)(mask[li] & 1), t10 = a1[j] * (float)((mask[li] >> 1) & 1);
+              const float t01 = a2[j] * (float)((mask[li] >> 2) & 1), t11 = a3[j] * (float)(mask[li] >> 3);
               const float gc = g[j] * sc;
               dfx[li] += gc * ((1.0f - v) * (t10 - t00) + v * (t11 - t01));
               dfy[li] += gc * ((1.0f - u) * (t01 - t00) + u * (t11 - t10));

@@ -184,3 +184,30 @@ def test_nearest_nonfinite_cotangent(C, bnd, texels):
     DiffRast.texture(t, dev(uv), filterMode="nearest", boundaryMode=bnd).backward(dev(g))
     ref = O.texture_vjp(tex, uv, g, filterMode="nearest", boundaryMode=bnd)[0]
     assert_same_nonfinite(host(t.grad), ref, "d_tex")
+
+
+# texels that are not finite, also under weights of zero: outside the zero
+# boundary's image, on the level a magnified surface does not use, and under
+# footprints that fall on one texel
+@pytest.mark.parametrize("filt", ["linear", "linear-mipmap-linear", "linear-mipmap-nearest"])
+@pytest.mark.parametrize("bnd", ["wrap", "clamp", "zero"])
+@pytest.mark.parametrize("lod", [1e-3, 1.3, 100.0])
+def test_many_channels_nonfinite_texels(filt, bnd, lod):
+    torch_dev()
+    from diffrast import DiffRast
+    rng = np.random.default_rng(5)
+    Hi, Wi, Ht, Wt, C = 33, 40, 32, 64, 6
+    uv, _ = smooth_uv(rng, 2, Hi, Wi, 0.9, 0.3, (0.0, 0.0))
+    uv[:, -3:, -3:] = 4.0
+    da = np.full((2, Hi, Wi, 4), lod / Wt, np.float32) * np.float32([1, 0.9, 0.4, 0.45])
+    tex = rng.random((1, Ht, Wt, C)).astype(np.float32)
+    tex[0, 0, 0, 1], tex[0, 20, 31, 2], tex[0, Ht - 1, Wt - 1, 4] = np.inf, np.nan, -np.inf
+    g = rng.normal(size=(2, Hi, Wi, C)).astype(np.float32)
+    kw = dict(filterMode=filt, boundaryMode=bnd)
+    mip = "mipmap" in filt
+    u = dev(uv).requires_grad_(True)
+    out = DiffRast.texture(dev(tex), u, uvDA=dev(da) if mip else None, **kw)
+    out.backward(dev(g))
+    assert_same_nonfinite(host(out), O.texture(tex, uv, uvDA=da if mip else None, **kw), "out")
+    ref = O.texture_vjp(tex, uv, g, uvDA=da if mip else None, **kw)[1]
+    assert_same_nonfinite(host(u.grad), ref, "d_uv")
