@@ -958,6 +958,10 @@ __device__ __forceinline__ int wrap_up(int t, int size) {
   return t < size ? t : t % size;
 }
 
+// a * b, 0 where a is 0 whatever b (an infinity, NaN): one instruction, whose
+// intrinsic has no builtin in this compiler.
+__device__ float mul0(float a, float b) __asm("llvm.amdgcn.fmul.legacy");
+
 // Weight `tap` (0..3: 00, 10, 01, 11) of the wave-uniform lane `leader`.
 __device__ __forceinline__ float leader_weight(const TapSlot& q, int leader, int tap) {
   const int a = __builtin_amdgcn_readlane(__float_as_int(q.w00), leader);
@@ -994,6 +998,10 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
   // goes into the cotangent): three more of weight 0 would put 0 * inf into
   // texels that it does not sample, and cost their LDS additions.
   constexpr int kTaps = FILTER == DR_FILTER_NEAREST ? 1 : 4;
+  // A tap of weight zero may lie outside its box, and has a clamped place
+  // there: it adds 0 (mul0), and what 0 * g is where a cotangent is not
+  // finite goes to the tap's own texel, apart from the windows.
+  constexpr bool kOwnTaps = kTaps == 4 && (kCube || BND == DR_BOUNDARY_WRAP);
   constexpr int kRows = kTaps == 1 ? 1 : 2, kRowVals = (kTaps == 1 ? 1 : 2) * CT;  // texel rows
   const bool shared_tex = A.tex_stride == 0;
   const int wave = tid >> 6, lane = tid & 63;
@@ -1372,7 +1380,8 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
 #pragma unroll
       for (int t = 0; t < kTaps; ++t)
 #pragma unroll
-        for (int c = 0; c < CT; ++c) v[t * CT + c] = kTaps == 1 ? gs[c] : wt[t] * gs[c];
+        for (int c = 0; c < CT; ++c)
+          v[t * CT + c] = kTaps == 1 ? gs[c] : kOwnTaps ? mul0(wt[t], gs[c]) : wt[t] * gs[c];
       row_run_scan_n(run, v, maxlen);
       return u && run.tail;
     };
@@ -1407,6 +1416,30 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
       }
     }
     __syncthreads();
+
+    if constexpr (kOwnTaps) {
+      bool bad = false;  // a cotangent that is not finite
+#pragma unroll
+      for (int c = 0; c < CT; ++c) bad = bad || 0.0f * g[c] != 0.0f;
+      if (__ballot(bad) != 0ull) {  // uniform
+#pragma unroll
+        for (int li = 0; li < (mip ? 2 : 1); ++li) {
+          const TapSlot& ql = q[li];
+          if (!(bad && (li == 0 ? use0 : use1))) continue;
+          const int k = ql.k, Wk = level_w(k), Hk = level_h(k);
+#pragma unroll 1
+          for (int t = 0; t < 4; ++t) {
+            if ((t == 0 ? ql.w00 : t == 1 ? ql.w10 : t == 2 ? ql.w01 : ql.w11) != 0.0f) continue;
+            const int X = win_texel<BND>((t & 1) ? ql.ix1 : ql.ix0, Wk);
+            const int Y = win_texel<BND>((t & 2) ? ql.iy1 : ql.iy0, Hk);
+            float* p = dlevel_ptr(k) + ((int64_t)Y * Wk + X) * CT;
+#pragma unroll
+            for (int c = 0; c < CT; ++c)
+              if (0.0f * g[c] != 0.0f) unsafeAtomicAdd(p + c, 0.0f * g[c]);
+          }
+        }
+      }
+    }
 
     // -- write the windows out, row by row -----------------------------------
     // Level k's window of bw x bh texels from window coordinates (x0, y0),
@@ -1661,11 +1694,11 @@ __global__ void __launch_bounds__(256) k_tex_fwd_many(
 // a texel's channels as one run of memory.  One footprint set-up serves all
 // channels, and d_uv and the LOD's gradient sum over them in registers.  The
 // general kernel's wave probes and one device atomic per tap and channel
-// took 3,453 us at 2 x 768^2 x 16, trilinear; this takes 191 (182 without the
-// terms of weight 0, which matter for texels that are not finite; there, 188
-// with the
-// direct way's cotangents loaded one pixel at a time; 264 at four waves per
-// SIMD, which spills 46 registers; 211 with two and a pool twice the size).
+// took 3,453 us at 2 x 768^2 x 16, trilinear; this takes 194 (182 without
+// zero_taps and the terms of weight 0, which matter for values that are not
+// finite; there, 188 with the direct way's cotangents loaded one pixel at a
+// time, 264 at four waves per SIMD, which spills 46 registers, 211 with two and
+// a pool twice the size).
 // Cube maps: k is the face, one level each.
 // ---------------------------------------------------------------------------
 
@@ -1692,6 +1725,62 @@ __device__ __forceinline__ void hot_flush(const ManyHot& h, int C, const double*
     if (v != 0.0f)
       unsafeAtomicAdd(h.base + ((int64_t)((t & 2) ? h.iy1 : h.iy0) * h.Wk +
                                 ((t & 1) ? h.ix1 : h.ix0)) * C + c, v);
+  }
+}
+
+// The taps of weight zero of one pixel's footprints (a border's merged ones, a
+// texel centre's, those outside the image; slot 0's unless it is in the hot
+// sum): 0 * g is 0, or NaN where a cotangent is not finite, and then belongs
+// to the tap's own texel, which need not be in any window.  Computed from the
+// inputs again, so that nothing of it is kept in registers through the
+// channels (k_tex_bwd_many spills already).
+template <int FILTER, int BND>
+__device__ __forceinline__ void zero_taps(const TexBwdArgs& A, int n, int64_t pix, bool in_hot) {
+  constexpr bool kCube = BND == DR_BOUNDARY_CUBE;
+  constexpr bool mip = FILTER == DR_FILTER_LINEAR_MIPMAP_LINEAR || FILTER == DR_FILTER_LINEAR_MIPMAP_NEAREST;
+  constexpr int kTaps = FILTER == DR_FILTER_NEAREST ? 1 : 4;
+  asm volatile("" : "+v"(pix));  // (not the values computed before)
+  const float* gp = A.d_out + pix * A.C;
+  bool bad = false;
+  for (int c = 0; c < A.C; ++c) bad = bad || 0.0f * gp[c] != 0.0f;
+  if (!bad) return;
+  Lod ld;
+  ld.k0 = ld.k1 = 0;
+  ld.frac = 0.0f;
+  if (mip) {
+    float4 da = *reinterpret_cast<const float4*>(A.uv_da + pix * 4);
+    if (A.bias_map || A.has_bias) {
+      const float s = bias_scale(A.bias_map, pix, A.scale_bias, A.has_bias != 0);
+      da = make_float4(da.x * s, da.y * s, da.z * s, da.w * s);
+    }
+    ld = mip_lod(da, A.Ht, A.Wt, A.md.L, FILTER == DR_FILTER_LINEAR_MIPMAP_LINEAR);
+  }
+#pragma unroll 1
+  for (int li = in_hot ? 1 : 0; li < (mip ? 2 : 1); ++li) {
+    if (li == 1 && ld.frac == 0.0f) continue;
+    int k = li == 0 ? ld.k0 : ld.k1;
+    const int Wk = kCube ? A.Wt : mip_w(A.md, k), Hk = kCube ? A.Ht : mip_h(A.md, k);
+    Bilin b;
+    if (kCube) {
+      k = cube_bilin(A.uv[pix * 3 + 0], A.uv[pix * 3 + 1], A.uv[pix * 3 + 2], Wk, Hk, b);
+    } else {
+      const float u = A.uv[pix * 2 + 0], v = A.uv[pix * 2 + 1];
+      b = FILTER == DR_FILTER_NEAREST ? nearest_tap(u, v, Wk, Hk, BND) : bilin(u, v, Wk, Hk, BND);
+    }
+    if (b.ix1 == b.ix0) { b.w00 += b.w10; b.w01 += b.w11; b.w10 = 0.0f; b.w11 = 0.0f; }
+    if (b.iy1 == b.iy0) { b.w00 += b.w01; b.w10 += b.w11; b.w01 = 0.0f; b.w11 = 0.0f; }
+    float* lv = kCube || k == 0 ? A.d_tex + n * A.tex_stride + (int64_t)k * Hk * Wk * A.C
+                                : A.d_pyr + mip_off(A.md, k) +
+                                      (A.tex_stride == 0 ? 0 : (int64_t)n * Hk * Wk * A.C);
+#pragma unroll
+    for (int t = 0; t < kTaps; ++t) {
+      if ((t == 0 ? b.w00 : t == 1 ? b.w10 : t == 2 ? b.w01 : b.w11) != 0.0f) continue;
+      float* p = lv + ((int64_t)((t & 2) ? b.iy1 : b.iy0) * Wk + ((t & 1) ? b.ix1 : b.ix0)) * A.C;
+      for (int c = 0; c < A.C; ++c) {
+        const float x = 0.0f * gp[c];
+        if (x != 0.0f) unsafeAtomicAdd(p + c, x);
+      }
+    }
   }
 }
 
@@ -1847,6 +1936,14 @@ __global__ void __launch_bounds__(256, 3) k_tex_bwd_many(TexBwdArgs A, int total
       }
     }
 
+    // taps of weight zero (zero_taps), other than the hot sum's
+    bool zeros = false;
+#pragma unroll
+    for (int li = 0; li < (mip ? 2 : 1); ++li)
+      zeros = zeros || (valid && q[li].scale != 0.0f && !(li == 0 && in_hot) &&
+                        (q[li].w00 == 0.0f ||
+                         (kTaps == 4 && (q[li].w10 == 0.0f || q[li].w01 == 0.0f || q[li].w11 == 0.0f))));
+
     // -- boxes of the levels in use, and their windows (k_tex_bwd_win) -----------
     {
       const int lm = wave_or((use0 ? 1 << q[0].k : 0) | (use1 ? 1 << q[1].k : 0));
@@ -1986,17 +2083,6 @@ __global__ void __launch_bounds__(256, 3) k_tex_bwd_many(TexBwdArgs A, int total
               }
             }
           }
-          if constexpr (FILTER == DR_FILTER_NEAREST && BND == DR_BOUNDARY_ZERO) {
-            // outside the image: 0 * g is 0, or NaN where g is not finite
-            if (valid && mask[0] == 0) {
-              float* p = dlevel_ptr(0) + ((int64_t)ty0[0] * A.Wt + tx0[0]) * C + c;
-#pragma unroll
-              for (int j = 0; j < 4; ++j) {
-                const float x = 0.0f * g[j];
-                if (x != 0.0f) unsafeAtomicAdd(p + j, x);
-              }
-            }
-          }
           const bool us = li == 0 ? use0 : use1;
           if (__ballot(us) == 0ull) continue;
           const float sc = mip ? q[li].scale : 1.0f;
@@ -2005,7 +2091,7 @@ __global__ void __launch_bounds__(256, 3) k_tex_bwd_many(TexBwdArgs A, int total
 #pragma unroll
           for (int t = 0; t < kTaps; ++t)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) v[t * 4 + j] = us ? wt[t] * (g[j] * sc) : 0.0f;
+            for (int j = 0; j < 4; ++j) v[t * 4 + j] = us ? mul0(wt[t], g[j] * sc) : 0.0f;
           row_run_scan_n(run[li], v, maxlen[li]);
           if (adds[li]) {
             double* w = win + (c - c0) * texels;
@@ -2096,6 +2182,8 @@ __global__ void __launch_bounds__(256, 3) k_tex_bwd_many(TexBwdArgs A, int total
         }
       }
     }
+
+    if (zeros) zero_taps<FILTER, BND>(A, n, pix, in_hot);
 
     // -- d_uv, d_uvDA, d_bias (Texture.swift:500-520, :979-1102) -----------------
     if (kCube) {

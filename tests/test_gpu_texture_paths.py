@@ -186,6 +186,41 @@ def test_nearest_nonfinite_cotangent(C, bnd, texels):
     assert_same_nonfinite(host(t.grad), ref, "d_tex")
 
 
+# cotangents that are not finite on footprints at texel centres, whose taps
+# of weight zero (0 * inf) lie outside the boxes of the weighted ones
+@pytest.mark.parametrize("C,bnd,filt", [(1, "wrap", "linear"), (3, "wrap", "linear"),
+                                        (4, "wrap", "linear-mipmap-linear"), (3, "cube", "linear"),
+                                        (6, "wrap", "linear"), (6, "clamp", "linear"),
+                                        (6, "zero", "linear"), (6, "cube", "linear"),
+                                        (6, "clamp", "linear-mipmap-linear")])
+@pytest.mark.parametrize("step", [1, 4, 16])  # texels a pixel
+def test_zero_weight_taps_nonfinite_cotangent(C, bnd, filt, step):
+    torch_dev()
+    from diffrast import DiffRast
+    rng = np.random.default_rng(C + step)
+    Hi = Wi = 33
+    S = 256
+    i = (np.arange(Hi) * step + 40) % S  # (no texel at a border, where taps merge)
+    y, x = np.meshgrid(i, i, indexing="ij")
+    if bnd == "cube":  # exact in fp32: every quotient is by 1
+        y, x = np.clip(y, 1, S - 2), np.clip(x, 1, S - 2)
+        uv = np.stack([(2 * x + 1) / S - 1, -((2 * y + 1) / S - 1), np.ones_like(x)], -1)
+    else:
+        uv = np.stack([(x + 0.5) / S, (y + 0.5) / S], -1)
+        if bnd == "zero":
+            uv[:5] += 2.0  # outside the image
+    uv = np.stack([uv, uv[::-1]]).astype(np.float32)
+    tex = rng.random((1, 6, S, S, C) if bnd == "cube" else (1, S, S, C)).astype(np.float32)
+    g = nonfinite(rng, rng.normal(size=(2, Hi, Wi, C)).astype(np.float32))
+    kw = dict(filterMode=filt, boundaryMode=bnd)
+    # (between two levels: of a level of weight zero no tap is added)
+    da = np.full((2, Hi, Wi, 4), 1.3 / S, np.float32) if "mipmap" in filt else None
+    t = dev(tex).requires_grad_(True)
+    DiffRast.texture(t, dev(uv), uvDA=None if da is None else dev(da), **kw).backward(dev(g))
+    ref = O.texture_vjp(tex, uv, g, uvDA=da, **kw)[0]
+    assert_same_nonfinite(host(t.grad), ref, "d_tex")
+
+
 # texels that are not finite, also under weights of zero: outside the zero
 # boundary's image, on the level a magnified surface does not use, and under
 # footprints that fall on one texel
