@@ -313,21 +313,33 @@ __device__ __forceinline__ int dpp_shift(int v) {
   return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true);
 }
 
+template <int CTRL>
+__device__ __forceinline__ float dpp_shift_of(float v) {
+  return __int_as_float(dpp_shift<CTRL>(__float_as_int(v)));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_shift_of(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)dpp_shift<CTRL>((int)(uint32_t)b);
+  const uint32_t hi = (uint32_t)dpp_shift<CTRL>((int)(uint32_t)(b >> 32));
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
 // Step D of the scan, masked on the sending side: lane l's value reaches
 // lane l + D when both lie in one run (run start of l + D <= l); any other
 // lane sends +0.  The receiver then adds unconditionally, so the shift
 // fuses into the add (one DPP instruction per value) and the sums equal a
 // conditional add's.
-template <int D, int M>
-__device__ __forceinline__ void run_scan_step(int li, int s, float (&v)[M]) {
+template <int D, int M, typename T>
+__device__ __forceinline__ void run_scan_step(int li, int s, T (&v)[M]) {
   const int s_to = dpp_shift<0x100 + D>(s);  // run start of lane l + D
   const bool send = li + D <= 15 && s_to <= li;
-  float w[M];  // all masks first: a DPP read right after the VALU write of its
+  T w[M];  // all masks first: a DPP read right after the VALU write of its
                // source waits two cycles
 #pragma unroll
-  for (int i = 0; i < M; ++i) w[i] = send ? v[i] : 0.0f;
+  for (int i = 0; i < M; ++i) w[i] = send ? v[i] : T(0);
 #pragma unroll
-  for (int i = 0; i < M; ++i) v[i] += __int_as_float(dpp_shift<0x110 + D>(__float_as_int(w[i])));
+  for (int i = 0; i < M; ++i) v[i] += dpp_shift_of<0x110 + D>(w[i]);
 }
 
 __device__ __forceinline__ int wave_max(int v) {
@@ -374,8 +386,8 @@ __device__ __forceinline__ RowRun row_run(uint64_t key) {
   return r;
 }
 
-template <int M>
-__device__ __forceinline__ void row_run_scan(const RowRun& r, float (&v)[M]) {
+template <int M, typename T>
+__device__ __forceinline__ void row_run_scan(const RowRun& r, T (&v)[M]) {
   run_scan_step<1>(r.li, r.s, v);
   run_scan_step<2>(r.li, r.s, v);
   run_scan_step<4>(r.li, r.s, v);
@@ -385,16 +397,16 @@ __device__ __forceinline__ void row_run_scan(const RowRun& r, float (&v)[M]) {
 // The same scan with only as many steps as the longest run in the wave
 // needs (`maxlen`, wave-uniform): a run of length r is summed after
 // ceil(log2 r) steps.
-template <int M>
-__device__ __forceinline__ void row_run_scan_n(const RowRun& r, float (&v)[M], int maxlen) {
+template <int M, typename T>
+__device__ __forceinline__ void row_run_scan_n(const RowRun& r, T (&v)[M], int maxlen) {
   if (maxlen > 1) run_scan_step<1>(r.li, r.s, v);
   if (maxlen > 2) run_scan_step<2>(r.li, r.s, v);
   if (maxlen > 4) run_scan_step<4>(r.li, r.s, v);
   if (maxlen > 8) run_scan_step<8>(r.li, r.s, v);
 }
 
-template <int M>
-__device__ __forceinline__ bool row_run_sum(uint64_t key, float (&v)[M]) {
+template <int M, typename T>
+__device__ __forceinline__ bool row_run_sum(uint64_t key, T (&v)[M]) {
   const RowRun r = row_run(key);
   row_run_scan_n(r, v, wave_max(r.li - r.s + 1));
   return r.tail;
@@ -630,8 +642,8 @@ __device__ __forceinline__ void lds_table_clear(LdsTableU<NV, CAP>& u) {
   if (threadIdx.x == 0) u.n = 0;
 }
 
-template <int NV, int CAP, typename D>
-__device__ __forceinline__ void lds_table_add(LdsTableU<NV, CAP>& u, D* dst, const float* v) {
+template <int NV, int CAP, typename D, typename V>
+__device__ __forceinline__ void lds_table_add(LdsTableU<NV, CAP>& u, D* dst, const V* v) {
   static_assert(CAP <= 65536, "slots are 16-bit");
   auto& t = u.t;
   bool any = false;

@@ -8,6 +8,8 @@
 //              :370-417 (d_rast_db)
 // u weights vertex 1, v weights vertex 2, bw = 1 - u - v weights vertex 0
 // (CONVENTIONS.md of the reference).
+#include <type_traits>
+
 #include "common.h"
 
 namespace dr {
@@ -367,7 +369,9 @@ __global__ void __launch_bounds__(256) k_interp_bwd(
   }
   // d_attr (Interpolate.swift:231-264, :269-324), summed per vertex row in
   // LDS before the global atomics.
-  float rv[3 * AT];  // rows of i0, i1, i2
+  // rows of i0, i1, i2, their runs summed in fp32; in fp64 for one attribute,
+  // where the three sums are few enough for it (4 x 720 x 1280: 37 -> 38 us)
+  std::conditional_t<AT == 1, double, float> rv[3 * AT];
 #pragma unroll
   for (int q = 0; q < 3 * AT; ++q) rv[q] = 0.0f;
   if (valid) {
@@ -406,12 +410,14 @@ __global__ void __launch_bounds__(256) k_interp_bwd(
 // and d_rast_db sum over them in registers.  Element by element, each
 // attribute of each vertex searched a table of 256 single values by itself
 // and, once that was full, became a device atomic (4 x 720 x 1280, A = 8,
-// K = 2: 320 us, now 95).
+// K = 2: 320 us, now 115).  The runs are summed in fp64, as the table is (in
+// fp32: 103 us, and a term 2^24 times smaller than its neighbours' is lost).
+// Six waves per SIMD: 115 us against 118 with five and 177 with eight.
 constexpr int kAnyRows = 256;   // table entries: vertex rows of a tile
 constexpr int kAnyChunk = 4;
 constexpr int kAnyNone = 0xffff;  // no entry: the row goes to memory
 
-__global__ void __launch_bounds__(256) k_interp_bwd_any(
+__global__ void __launch_bounds__(256, 6) k_interp_bwd_any(
     const float* __restrict__ attr, int64_t attr_stride, const float* __restrict__ rast,
     const float* __restrict__ rast_db, const int32_t* __restrict__ tri,
     DiffIdx diff, int K, const float* __restrict__ d_out,
@@ -497,23 +503,24 @@ __global__ void __launch_bounds__(256) k_interp_bwd_any(
 #pragma unroll 1
   for (int c = 0; c < A; c += kAnyChunk) {
     const int nc = min(kAnyChunk, A - c);
-    float rv[3 * kAnyChunk];
+    float ga[kAnyChunk];                  // cotangents of the attributes,
+    double gu[kAnyChunk], gv[kAnyChunk];  // and of the derivatives' u and v terms
 #pragma unroll
-    for (int j = 0; j < 3 * kAnyChunk; ++j) rv[j] = 0.0f;
+    for (int j = 0; j < kAnyChunk; ++j) {
+      ga[j] = 0.0f;
+      gu[j] = gv[j] = 0.0;
+    }
     if (valid) {
       const float4 g4 = ld_chunk(g + c, nc);
       const float4 x = ld_chunk(at + o0 + c, nc), y = ld_chunk(at + o1 + c, nc),
                    z = ld_chunk(at + o2 + c, nc);
-      const float ga[4] = {g4.x, g4.y, g4.z, g4.w};
+      ga[0] = g4.x; ga[1] = g4.y; ga[2] = g4.z; ga[3] = g4.w;
       const float d01[4] = {y.x - x.x, y.y - x.y, y.z - x.z, y.w - x.w};
       const float d02[4] = {z.x - x.x, z.y - x.y, z.z - x.z, z.w - x.w};
 #pragma unroll
       for (int j = 0; j < kAnyChunk; ++j) {
         du += d01[j] * ga[j];
         dv += d02[j] * ga[j];
-        rv[j] = bw * ga[j];
-        rv[kAnyChunk + j] = u * ga[j];
-        rv[2 * kAnyChunk + j] = v * ga[j];
       }
       // derivative outputs of this chunk's attributes (indices are uniform)
 #pragma unroll 1
@@ -530,24 +537,29 @@ __global__ void __launch_bounds__(256) k_interp_bwd_any(
           d_udy += d01[j] * gy;
           d_vdx += d02[j] * gx;
           d_vdy += d02[j] * gy;
-          rv[j] += -u_term - v_term;
-          rv[kAnyChunk + j] += u_term;
-          rv[2 * kAnyChunk + j] += v_term;
+          gu[j] += (double)u_term;
+          gv[j] += (double)v_term;
         }
       }
     }
-    row_run_scan_n(run, rv, maxlen);
-    if (tail) {
+    // a vertex at a time: its four sums along the runs, in fp64 as in the table
 #pragma unroll
-      for (int i = 0; i < 3; ++i) {
+    for (int i = 0; i < 3; ++i) {
+      const float w = i == 0 ? bw : i == 1 ? u : v;
+      double rv[kAnyChunk];
+#pragma unroll
+      for (int j = 0; j < kAnyChunk; ++j)
+        rv[j] = valid ? (double)(w * ga[j]) + (i == 0 ? -gu[j] - gv[j] : i == 1 ? gu[j] : gv[j]) : 0.0;
+      row_run_scan_n(run, rv, maxlen);
+      if (tail) {
 #pragma unroll
         for (int j = 0; j < kAnyChunk; ++j) {
-          const float x = rv[i * kAnyChunk + j];
-          if (j >= nc || x == 0.0f) continue;
+          const double x = rv[j];
+          if (j >= nc || x == 0.0) continue;
           if (slot[i] != kAnyNone)
-            atomicAdd(&s_sum[j][slot[i]], (double)x);
+            atomicAdd(&s_sum[j][slot[i]], x);
           else
-            unsafeAtomicAdd(da + (int64_t)vi[i] * A + c + j, x);
+            unsafeAtomicAdd(da + (int64_t)vi[i] * A + c + j, (float)x);
         }
       }
     }

@@ -45,3 +45,45 @@ def test_any_shape(A, diff, shared, level, H, W):
         d_attr, d_rast, _ = O.interpolate_vjp(attr, rast, sc["tri"], g)
     assert_grad_close(host(r.grad), d_rast, "d_rast", rtol=1e-5)
     assert_grad_close(host(a.grad), d_attr, "d_attr")
+
+
+@pytest.mark.parametrize("A,diff", [(1, None), (5, None), (8, [0, 1]), (6, "all"), (1, "all")])
+def test_sums_of_a_tile_are_exact(A, diff):
+    """A tile's d_attr terms are summed in fp64: cotangents of +-2^26 that
+    cancel within a pixel row leave the ones between them, which fp32 sums of
+    the row would lose.  One triangle everywhere at u = v = 0, so vertex 0
+    takes every cotangent whole and the derivatives' u terms (db = (1, 0, 0,
+    0)) go to vertices 0 and 1."""
+    torch = torch_dev()
+    from diffrast import DiffRast
+    rng = np.random.default_rng(A)
+    N, H, W = 1, 64, 80
+    rast = np.zeros((N, H, W, 4), np.float32)
+    rast[..., 3] = 1.0
+    db = np.zeros_like(rast)
+    db[..., 0] = 1.0
+
+    def cotangent(n):
+        g = rng.integers(-3, 4, size=(N, H, W, n)).astype(np.float32)
+        at = rng.integers(0, 8, size=(N, H, W // 16, n))
+        big = g.reshape(N, H, W // 16, 16, n)
+        np.put_along_axis(big, at[:, :, :, None], np.float32(2 ** 26), 3)
+        np.put_along_axis(big, 8 + at[:, :, :, None], np.float32(-2 ** 26), 3)
+        return g
+    attr = dev(rng.normal(size=(1, 3, A)).astype(np.float32)).requires_grad_(True)
+    tri = dev(np.array([[0, 1, 2]], np.int32))
+    g = cotangent(A)
+    ref = np.zeros((3, A))
+    ref[0] = g.astype(np.float64).sum((0, 1, 2))
+    if diff is None:
+        out, _ = DiffRast.interpolate(attr, dev(rast), tri)
+        out.backward(dev(g))
+    else:
+        idx = list(range(A)) if diff == "all" else diff
+        gda = cotangent(2 * len(idx))
+        out, da = DiffRast.interpolate(attr, dev(rast), tri, rastDB=dev(db), diffAttrs=diff)
+        torch.autograd.backward([out, da], [dev(g), dev(gda)])
+        u_term = gda[..., 0::2].astype(np.float64).sum((0, 1, 2))
+        ref[0, idx] -= u_term
+        ref[1, idx] += u_term
+    np.testing.assert_array_equal(host(attr.grad)[0], ref)
