@@ -422,6 +422,14 @@ __device__ __forceinline__ float dpp_movf(float v) {
   return __int_as_float(dpp_mov<CTRL>(__float_as_int(v)));
 }
 
+template <int CTRL>
+__device__ __forceinline__ double dpp_movf(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)dpp_mov<CTRL>((int)(uint32_t)b);
+  const uint32_t hi = (uint32_t)dpp_mov<CTRL>((int)(uint32_t)(b >> 32));
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
 // v + (v of lane l ^ 32) and v + (v of lane l ^ 16), with the gfx950 lane
 // swaps (one VALU instruction each, no LDS round trip).  permlane32_swap
 // exchanges lanes 32..63 of its first operand with lanes 0..31 of its
@@ -435,6 +443,20 @@ __device__ __forceinline__ float add_xor32(float v) {
 __device__ __forceinline__ float add_xor16(float v) {
   const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ double add_xor32(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const auto l = __builtin_amdgcn_permlane32_swap((uint32_t)b, (uint32_t)b, false, false);
+  const auto h = __builtin_amdgcn_permlane32_swap((uint32_t)(b >> 32), (uint32_t)(b >> 32), false, false);
+  return __builtin_bit_cast(double, ((uint64_t)h[0] << 32) | l[0]) +
+         __builtin_bit_cast(double, ((uint64_t)h[1] << 32) | l[1]);
+}
+__device__ __forceinline__ double add_xor16(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const auto l = __builtin_amdgcn_permlane16_swap((uint32_t)b, (uint32_t)b, false, false);
+  const auto h = __builtin_amdgcn_permlane16_swap((uint32_t)(b >> 32), (uint32_t)(b >> 32), false, false);
+  return __builtin_bit_cast(double, ((uint64_t)h[0] << 32) | l[0]) +
+         __builtin_bit_cast(double, ((uint64_t)h[1] << 32) | l[1]);
 }
 
 // Sixteen wave sums at once.  A transposing butterfly (row mirror, half-row
@@ -464,14 +486,15 @@ __device__ __forceinline__ float wave_sum16(const float (&a)[16]) {
 // with value (l & 3) summed over its quad, row rotations by 4 and 8 add the
 // row's four quads, and the lane swaps the four rows.  Every lane returns
 // the total of value (lane & 3).  All 64 lanes must execute this.
-__device__ __forceinline__ float wave_sum4(const float (&a)[4]) {
+template <typename T>
+__device__ __forceinline__ T wave_sum4(const T (&a)[4]) {
   const int l = lane_id();
   const bool b1 = (l >> 1) & 1, b0 = l & 1;
-  float v2[2];
+  T v2[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i)  // quad_perm [2,3,0,1]
     v2[i] = (b1 ? a[i + 2] : a[i]) + dpp_movf<0x4E>(b1 ? a[i] : a[i + 2]);
-  float v = (b0 ? v2[1] : v2[0]) + dpp_movf<0xB1>(b0 ? v2[0] : v2[1]);  // quad_perm [1,0,3,2]
+  T v = (b0 ? v2[1] : v2[0]) + dpp_movf<0xB1>(b0 ? v2[0] : v2[1]);  // quad_perm [1,0,3,2]
   v += dpp_movf<0x124>(v);  // row_ror:4
   v += dpp_movf<0x128>(v);  // row_ror:8
   return add_xor32(add_xor16(v));

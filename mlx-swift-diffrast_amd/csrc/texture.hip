@@ -356,29 +356,30 @@ __global__ void __launch_bounds__(256) k_tex_fwd(
 // same clamped texel) adds its wave-summed values here instead of issuing
 // atomics; the accumulator is written out when a different footprint takes
 // its place and when the wave has finished all its tiles.  Wave-uniform.
-template <int CT>
+// (V: double where the sums are fp64 all the way, k_tex_bwd_win.)
+template <int CT, typename V = float>
 struct FootAcc {
   float* p[4];  // the footprint's four texels (wave-uniform)
-  float v;      // lane j < 4*CT: running sum of value j = 4 * channel + tap
+  V v;          // lane j < 4*CT: running sum of value j = 4 * channel + tap
   bool on;
 };
 
-template <int CT>
-__device__ __forceinline__ void acc_init(FootAcc<CT>& a) {
+template <int CT, typename V>
+__device__ __forceinline__ void acc_init(FootAcc<CT, V>& a) {
   a.on = false;
 #pragma unroll
   for (int i = 0; i < 4; ++i) a.p[i] = nullptr;
-  a.v = 0.0f;
+  a.v = 0;
 }
 
-template <int CT>
-__device__ __forceinline__ void acc_flush(FootAcc<CT>& a) {
+template <int CT, typename V>
+__device__ __forceinline__ void acc_flush(FootAcc<CT, V>& a) {
   if (!a.on) return;
   const int l = lane_id();
-  if (l < 4 * CT && a.v != 0.0f) {
+  if (l < 4 * CT && a.v != 0) {
     const int tap = l & 3;
     float* q = tap == 0 ? a.p[0] : tap == 1 ? a.p[1] : tap == 2 ? a.p[2] : a.p[3];
-    unsafeAtomicAdd(q + (l >> 2), a.v);
+    unsafeAtomicAdd(q + (l >> 2), (float)a.v);
   }
   a.on = false;
 }
@@ -390,20 +391,20 @@ __device__ __forceinline__ void acc_flush(FootAcc<CT>& a) {
 // serialised (about 80 M/s) just as the workgroups end: one per workgroup
 // instead of one per wave (bilinear, 4 x 1000^2 x 3: 215 -> 193 us; 8 x 1024^2
 // trilinear, whose waves end further apart: no change).
-template <int CT, int W>
+template <int CT, int W, typename V = float>
 struct FootAccLds {
   uint64_t p[W][4];
-  float v[W][4 * CT];
+  V v[W][4 * CT];
 };
 
-template <int CT, int W>
-__device__ __forceinline__ void acc_flush_group(const FootAcc<CT>& a, FootAccLds<CT, W>& s) {
+template <int CT, int W, typename V>
+__device__ __forceinline__ void acc_flush_group(const FootAcc<CT, V>& a, FootAccLds<CT, W, V>& s) {
   const int wave = (int)threadIdx.x >> 6, l = lane_id();
   if (l < 4) {
     float* q = l == 0 ? a.p[0] : l == 1 ? a.p[1] : l == 2 ? a.p[2] : a.p[3];
     s.p[wave][l] = a.on ? (uint64_t)q : 0ull;
   }
-  if (l < 4 * CT) s.v[wave][l] = a.on ? a.v : 0.0f;
+  if (l < 4 * CT) s.v[wave][l] = a.on ? a.v : V(0);
   __syncthreads();
   if (!a.on) return;
   auto same = [&](int w) {
@@ -915,7 +916,7 @@ __global__ void __launch_bounds__(256) k_tex_bwd(TexBwdArgs A, int total_tiles) 
 // 4 x 1000^2 x 3 at 1-3 texels a pixel: 960 us, now 189; at 8 x 1024^2
 // trilinear with 1.3% of them, no change: 238 us).  Cube maps and the nearest
 // filter took the 512-entry hash table for all taps (cube, 4 x 800^2 x 3:
-// 94 us, now 49; nearest, 4 x 800 x 700 x 4: 86, now 49).
+// 94 us, now 55; nearest, 4 x 800 x 700 x 4: 86, now 51).
 // ---------------------------------------------------------------------------
 
 constexpr int kWinWaves = 4;                  // waves per workgroup; a tile is 16 x (4 * kWinWaves) pixels
@@ -982,8 +983,15 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
   __shared__ double win[kWinTexels * CT];
   __shared__ __align__(16) int s_lmask[kWinWaves];  // per wave: the levels in use (bit mask)
   __shared__ int2 s_lbox[kWinWaves][kMaxLevels];     // per wave and level: packed box
-  __shared__ FootAccLds<CT, kWinWaves> s_acc;
-  FootAcc<CT> acc;
+  // Sums that are fp64 from the first term on: the nearest filter's and the
+  // bilinear cube maps' runs, and their and the wrap mode's empty pixels
+  // (other runs and empty pixels are summed in fp32 first).  Against fp32 sums:
+  // cube, 4 x 800^2 x 3, 49 -> 55 us; nearest and bilinear wrap, no change.
+  constexpr bool kWide = FILTER == DR_FILTER_NEAREST || BND == DR_BOUNDARY_CUBE;
+  using RunT = std::conditional_t<kWide, double, float>;
+  using AccT = std::conditional_t<kWide || BND == DR_BOUNDARY_WRAP, double, float>;
+  __shared__ FootAccLds<CT, kWinWaves, AccT> s_acc;
+  FootAcc<CT, AccT> acc;
   acc_init(acc);
   const int tid = threadIdx.x;
   for (int i = tid; i < kWinTexels * CT; i += kWinThreads) win[i] = 0.0;
@@ -1262,19 +1270,19 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
           acc_flush(acc);
 #pragma unroll
           for (int t = 0; t < 4; ++t) acc.p[t] = (float*)uni((uint64_t)lp[t]);
-          acc.v = 0.0f;
+          acc.v = 0;
           acc.on = true;
         }
         // all the weight is on tap 0 (one texel; wrap mode: the group has one
         // set of four weights): four sums, one per channel
-        float x[4];
+        AccT x[4];
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
           const float gc = g[c < CT ? c : 0] * q[0].scale;
           x[c] = (c < CT && same) ? (kSameUv ? gc : q[0].w00 * gc) : 0.0f;
         }
-        const float z = wave_sum4(x);  // lane l: total of value l & 3
-        const float zc = __shfl(z, (lane >> 2) & 3, kWave);
+        const AccT z = wave_sum4(x);  // lane l: total of value l & 3
+        const AccT zc = __shfl(z, (lane >> 2) & 3, kWave);
         if (kSameUv && kTaps == 4) {  // lane 4c + t: channel c, tap t
           const float wt = leader_weight(q[0], leader, lane & 3);
           if (lane < 4 * CT) acc.v += wt * zc;
@@ -1356,11 +1364,9 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
     // -- accumulate: runs of one footprint along a pixel row are summed
     //    first (lanes of one LDS atomic on one address are serialised), the
     //    run's last lane adds the totals ----------------------------------------
-    // Slot li's run totals v (tap-major, kTaps * CT values, all zero in a lane
-    // that is not the tail of a run of `u` lanes' footprints); whether this
-    // lane is one.  Every lane executes it.
-    auto run_totals = [&](int li, bool u, float (&v)[kTaps * CT]) -> bool {
-      const float sc = mip ? q[li].scale : 1.0f;
+    // The runs of slot li's footprints in the `u` lanes, and the longest one in
+    // the wave.  Every lane executes it.
+    auto slot_runs = [&](int li, bool u, int& maxlen) -> RowRun {
       // level and the four texel coordinates (each < 32767 on the window
       // path) fix the taps; an unused slot gets a key no footprint has
       const uint64_t key =
@@ -1372,19 +1378,28 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
                    ((uint64_t)q[li].ix1 << 30) | ((uint64_t)q[li].iy0 << 15) |
                    (uint64_t)q[li].iy1;
       const RowRun run = row_run(key);
-      const int maxlen = wave_max(run.li - run.s + 1);  // longest run in the wave
+      maxlen = wave_max(run.li - run.s + 1);
+      return run;
+    };
+    // Their totals of taps t0, t0 + 1, ... (v: tap-major, CT values a tap), in
+    // a run's last lane; zero in a lane without `u`.  Every lane executes it.
+    auto run_totals = [&](int li, bool u, const RowRun& run, int maxlen, int t0, auto& v) {
+      constexpr int n = sizeof(v) / sizeof(v[0]) / CT;
+      const float sc = mip ? q[li].scale : 1.0f;
       const float wt[4] = {q[li].w00, q[li].w10, q[li].w01, q[li].w11};
       float gs[CT];
 #pragma unroll
       for (int c = 0; c < CT; ++c) gs[c] = !u ? 0.0f : g[c] * sc;
 #pragma unroll
-      for (int t = 0; t < kTaps; ++t)
+      for (int t = 0; t < n; ++t)
 #pragma unroll
         for (int c = 0; c < CT; ++c)
-          v[t * CT + c] = kTaps == 1 ? gs[c] : kOwnTaps ? mul0(wt[t], gs[c]) : wt[t] * gs[c];
+          v[t * CT + c] = kTaps == 1 ? gs[c] : kOwnTaps ? mul0(wt[t0 + t], gs[c]) : wt[t0 + t] * gs[c];
       row_run_scan_n(run, v, maxlen);
-      return u && run.tail;
     };
+    // Taps summed at once: all four in fp32, one in fp64, whose four would
+    // need twice the registers (cube, 4 x 800^2 x 4: 61 us, 76 with all four).
+    constexpr int kAtOnce = kWide ? 1 : kTaps;
 #pragma unroll
     for (int li = 0; li < 2; ++li) {
       const bool u = li == 0 ? use0 : use1;
@@ -1393,9 +1408,11 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
       // the window of level k (every lane executes the permutes)
       const int sxy = __builtin_amdgcn_ds_bpermute(k << 2, wxy);
       const int ssz = __builtin_amdgcn_ds_bpermute(k << 2, wsz);
-      float v[kTaps * CT];
-      const bool adds = run_totals(li, u, v);
-      if (adds && ssz != 0) {
+      int maxlen;
+      const RowRun run = slot_runs(li, u, maxlen);
+      const bool adds = u && run.tail && ssz != 0;
+      int o[4] = {0, 0, 0, 0};
+      if (adds) {
         // window indices of the four taps.  The box holds every tap with a
         // nonzero weight in some lane of the run; a tap whose weight is zero
         // in all of them (a texel column or row with zero weight, outside
@@ -1407,12 +1424,19 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
         const int cx1 = min(max(q[li].ix1 - wx, 0), ww - 1);
         const int r0 = sbase + min(max(q[li].iy0 - wy, 0), wh - 1) * ww;
         const int r1 = sbase + min(max(q[li].iy1 - wy, 0), wh - 1) * ww;
-        const int o[4] = {r0 + cx0, r0 + cx1, r1 + cx0, r1 + cx1};  // < sbase + area
+        o[0] = r0 + cx0; o[1] = r0 + cx1; o[2] = r1 + cx0; o[3] = r1 + cx1;  // < sbase + area
+      }
 #pragma unroll
-        for (int t = 0; t < kTaps; ++t)
+      for (int t0 = 0; t0 < kTaps; t0 += kAtOnce) {
+        RunT v[kAtOnce * CT];
+        run_totals(li, u, run, maxlen, t0, v);
+        if (adds) {
 #pragma unroll
-          for (int c = 0; c < CT; ++c)
-            atomicAdd(win + c * kWinTexels + o[t], (double)v[t * CT + c]);
+          for (int t = 0; t < kAtOnce; ++t)
+#pragma unroll
+            for (int c = 0; c < CT; ++c)
+              atomicAdd(win + c * kWinTexels + o[t0 + t], (double)v[t * CT + c]);
+        }
       }
     }
     __syncthreads();
@@ -1511,8 +1535,11 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
       const int bw = -unpack16_hi(px) - x0 + 1, bh = -unpack16_hi(py) - y0 + 1;
       const int rows = win_rows(bw, kWinTexels);
       if (rows * kWinBands >= bh) {  // (rows 0: too wide)
-        float v[kTaps * CT];
-        const bool adds = run_totals(0, use0, v);
+        int maxlen;
+        const RowRun run = slot_runs(0, use0, maxlen);
+        const bool adds = use0 && run.tail;
+        RunT v[kTaps * CT];
+        run_totals(0, use0, run, maxlen, 0, v);
         const int cx0 = min(max(q[0].ix0 - x0, 0), bw - 1);
         const int cx1 = min(max(q[0].ix1 - x0, 0), bw - 1);
         // (a zero-weight row outside the box is clamped into it: adds 0)
@@ -1557,8 +1584,9 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
         const int k = q[li].k;
         const bool u = (li == 0 ? use0 : use1) && ((nowin >> k) & 1);
         if (__ballot(u) == 0) continue;
-        float v[kTaps * CT];
-        const bool adds = run_totals(li, u, v);
+        int maxlen;
+        const RowRun run = slot_runs(li, u, maxlen);
+        const bool adds = u && run.tail;
         const int Wk = level_w(k), Hk = level_h(k);
         const int X0 = win_texel<BND>(q[li].ix0, Wk), X1 = win_texel<BND>(q[li].ix1, Wk);
         const int Y0 = win_texel<BND>(q[li].iy0, Hk), Y1 = win_texel<BND>(q[li].iy1, Hk);
@@ -1566,25 +1594,26 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
         const uint32_t o0 = ((uint32_t)Y0 * (uint32_t)Wk + (uint32_t)X0) * CT;
         const uint32_t o1 = ((uint32_t)Y1 * (uint32_t)Wk + (uint32_t)X0) * CT;
         const int dx = (X1 - X0) * CT;
-        if (__popcll(__ballot(adds)) <= kWinFewRuns) {
-          if (adds) {
-#pragma unroll
-            for (int t = 0; t < kTaps; ++t)
-#pragma unroll
-              for (int c = 0; c < CT; ++c) {
-                const float x = v[t * CT + c];
-                if (x != 0.0f) unsafeAtomicAdd(lv + ((t & 2) ? o1 : o0) + ((t & 1) ? dx : 0) + c, x);
-              }
-          }
-          continue;
-        }
-        staged = true;
+        const bool few = __popcll(__ballot(adds)) <= kWinFewRuns;  // uniform
+        staged = staged || !few;
 #pragma unroll
         for (int row = 0; row < kRows; ++row) {
-          const uint64_t p = (uint64_t)(lv + (row == 0 ? o0 : o1));
+          RunT v[kRowVals];
+          run_totals(li, u, run, maxlen, row * 2, v);
+          float* const pr = lv + (row == 0 ? o0 : o1);
+          if (few) {
+            if (adds) {
 #pragma unroll
-          for (int j = 0; j < kRowVals; ++j)
-            st[lane * kRowVals + j] = adds ? (double)v[row * kRowVals + j] : 0.0;
+              for (int j = 0; j < kRowVals; ++j) {
+                const float x = (float)v[j];
+                if (x != 0.0f) unsafeAtomicAdd(pr + (j < CT ? j : dx + j - CT), x);
+              }
+            }
+            continue;
+          }
+          const uint64_t p = (uint64_t)pr;
+#pragma unroll
+          for (int j = 0; j < kRowVals; ++j) st[lane * kRowVals + j] = adds ? (double)v[j] : 0.0;
           __builtin_amdgcn_wave_barrier();  // (LDS is ordered within a wave)
           __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
 #pragma unroll 1

@@ -246,3 +246,43 @@ def test_many_channels_nonfinite_texels(filt, bnd, lod):
     assert_same_nonfinite(host(out), O.texture(tex, uv, uvDA=da if mip else None, **kw), "out")
     ref = O.texture_vjp(tex, uv, g, uvDA=da if mip else None, **kw)[1]
     assert_same_nonfinite(host(u.grad), ref, "d_uv")
+
+
+# a tile's d_tex terms are summed in fp64 from the first on: cotangents of
+# +-2^26 that cancel within four pixels of a texel leave the small ones, which
+# fp32 sums of a pixel row would lose (weights are 1, or 1/4 under a constant
+# uv, so every product is exact)
+@pytest.mark.parametrize("C", [1, 3, 4])
+@pytest.mark.parametrize("kind", ["nearest", "nearest-constant", "cube", "wrap-constant"])
+def test_sums_of_a_tile_are_exact(kind, C):
+    torch_dev()
+    from diffrast import DiffRast
+    rng = np.random.default_rng(C)
+    N, Hi, Wi, S = 2, 48, 64, 64
+    y, x = np.meshgrid(np.arange(Hi) + 8, np.arange(Wi) // 4 + 8, indexing="ij")
+    g = rng.integers(-3, 4, size=(N, Hi, Wi // 4, 4, C)).astype(np.float32) * 4
+    at = rng.integers(0, 2, size=(N, Hi, Wi // 4, 1, C))
+    np.put_along_axis(g, at, np.float32(2 ** 26), 3)
+    np.put_along_axis(g, 2 + at, np.float32(-2 ** 26), 3)
+    g = g.reshape(N, Hi, Wi, C)
+    ref = np.zeros((S, S, C))
+    if kind.startswith("nearest"):
+        if kind == "nearest-constant":
+            x, y = np.full_like(x, 5), np.full_like(y, 9)
+        uv = np.stack([(x + 0.5) / S, (y + 0.5) / S], -1)
+        kw = dict(filterMode="nearest", boundaryMode="wrap")
+        np.add.at(ref, (y, x), g.astype(np.float64).sum(0))
+    elif kind == "cube":
+        uv = np.stack([(2 * x + 1) / S - 1, -((2 * y + 1) / S - 1), np.ones(x.shape)], -1)
+        kw = dict(filterMode="linear", boundaryMode="cube")
+        np.add.at(ref, (y, x), g.astype(np.float64).sum(0))
+    else:  # the four corner texels
+        uv = np.zeros((Hi, Wi, 2))
+        kw = dict(filterMode="linear", boundaryMode="wrap")
+        ref[np.ix_([0, S - 1], [0, S - 1])] = g.astype(np.float64).sum((0, 1, 2)) / 4
+    uv = np.broadcast_to(uv, (N,) + uv.shape).astype(np.float32)
+    shape = (1, 6, S, S, C) if kind == "cube" else (1, S, S, C)
+    t = dev(rng.random(shape).astype(np.float32)).requires_grad_(True)
+    DiffRast.texture(t, dev(uv), **kw).backward(dev(g))
+    got = host(t.grad)[0]
+    np.testing.assert_array_equal(got[4] if kind == "cube" else got, ref)
