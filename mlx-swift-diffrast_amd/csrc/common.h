@@ -792,6 +792,19 @@ inline hipError_t fill2_async(T* p0, int64_t n0, T* p1, int64_t n1, T v, hipStre
   return fill_async(p1, v, n1, s);
 }
 
+// A launch of `blocks` workgroups of 256 threads over x and y: one dimension
+// holds fewer than 2^32 threads (more are not all run, without an error).  The
+// workgroup's index is block_xy(); the last row may hold some past `blocks`.
+constexpr int kGridRowLog = 23;
+inline dim3 grid_xy(int64_t blocks) {
+  constexpr int64_t row = 1ll << kGridRowLog;
+  if (blocks <= row) return dim3((unsigned)blocks);
+  return dim3((unsigned)row, (unsigned)((blocks + row - 1) >> kGridRowLog));
+}
+__device__ __forceinline__ int64_t block_xy() {
+  return ((int64_t)blockIdx.y << kGridRowLog) + blockIdx.x;
+}
+
 inline unsigned grid_for(int64_t n, int block) {
   return (unsigned)((n + block - 1) / block);
 }

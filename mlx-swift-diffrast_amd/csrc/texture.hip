@@ -2308,14 +2308,15 @@ constexpr int kMipPatchLog = 5, kMipPatch = 1 << kMipPatchLog;
 
 __global__ void __launch_bounds__(256) k_mip_block(const float* __restrict__ src,
                                                    float* __restrict__ pyr, MipDesc md, int s,
-                                                   int m, int C) {
+                                                   int m, int C, int64_t blocks) {
   __shared__ float buf[2][256 * kMipMaxC];
+  if (block_xy() >= blocks) return;
   const int Ws = md.w[s];
   const int nbx = (Ws + kMipPatch - 1) / kMipPatch;
   const int per_n = nbx * ((md.h[s] + kMipPatch - 1) / kMipPatch);
   const int chunks = (C + kMipMaxC - 1) / kMipMaxC;
-  int blk = (int)blockIdx.x / chunks;
-  const int c0 = ((int)blockIdx.x - blk * chunks) * kMipMaxC, nc = min(kMipMaxC, C - c0);
+  int blk = (int)block_xy() / chunks;
+  const int c0 = ((int)block_xy() - blk * chunks) * kMipMaxC, nc = min(kMipMaxC, C - c0);
   const int n = blk / per_n;
   blk -= n * per_n;
   const int by = blk / nbx, bx = blk - by * nbx;
@@ -2359,12 +2360,13 @@ __global__ void __launch_bounds__(256) k_mip_block(const float* __restrict__ src
 // loads and stores, the same sums in the same order.
 __global__ void __launch_bounds__(256) k_mip_block_c4(const float* __restrict__ src,
                                                       float* __restrict__ pyr, MipDesc md, int s,
-                                                      int m) {
+                                                      int m, int64_t blocks) {
   __shared__ float4 buf[2][256];
+  if (block_xy() >= blocks) return;
   const int Ws = md.w[s];
   const int nbx = (Ws + kMipPatch - 1) / kMipPatch;
   const int per_n = nbx * ((md.h[s] + kMipPatch - 1) / kMipPatch);
-  const int n = (int)blockIdx.x / per_n, blk = (int)blockIdx.x - n * per_n;
+  const int n = (int)block_xy() / per_n, blk = (int)block_xy() - n * per_n;
   const int by = blk / nbx, bx = blk - by * nbx;
   const float4* lvl = reinterpret_cast<const float4*>(src) + (int64_t)n * md.h[s] * Ws;
   auto mean4 = [](float4 a, float4 b, float4 d, float4 f) {
@@ -2406,24 +2408,45 @@ __global__ void __launch_bounds__(256) k_mip_block_c4(const float* __restrict__ 
 // d_tex (which already holds level 0's own gradient).  Two passes: level 1's
 // totals in place (each of its values walks its chain of ancestors), then
 // level 0 adds a quarter of its parent's total.  A workgroup takes 256
-// values, or vectors of V = 4 where C is a multiple of 4, of one row, so
-// consecutive threads read consecutive memory; one thread per texel walking
-// the whole chain for each of its channels took 71 us at 512^2 x 16, this
-// takes 16.
+// values, or vectors of V = 4 where C is a multiple of 4, of one row (or
+// several whole rows, where they are shorter), so consecutive threads read
+// consecutive memory; one thread per texel walking the whole chain for each of
+// its channels took 71 us at 512^2 x 16, this takes 16.
 template <int V>
 struct alignas(4 * V) VecF {
   float v[V];
 };
 
+// How a level's rows of `vals` values are dealt to workgroups: 2^log threads a
+// row (at most 256), bpr workgroups for each 256 >> log rows.
+struct CollapseGrid {
+  int64_t rows, vals, blocks;
+  int log, bpr;
+};
+
+// i / d, i below n (uniform): in 32 bits where n allows.
+__device__ __forceinline__ int64_t div_n(int64_t i, int64_t n, int d) {
+  return n < (1ll << 31) ? (int)i / d : i / d;
+}
+
+// A thread's row and its value of the row; false: none.
+__device__ __forceinline__ bool collapse_place(const CollapseGrid& g, int64_t& row, int64_t& i) {
+  const int64_t b = block_xy();
+  const int64_t r = g.bpr == 1 ? b : div_n(b, g.blocks, g.bpr);
+  const int part = (int)(b - r * g.bpr);
+  row = (r << (8 - g.log)) + ((int)threadIdx.x >> g.log);
+  i = ((int64_t)part << g.log) + ((int)threadIdx.x & ((1 << g.log) - 1));
+  return row < g.rows && i < g.vals;
+}
+
 template <int V>
 __global__ void __launch_bounds__(256) k_mip_collapse1(float* __restrict__ d_pyr, MipDesc md,
-                                                       int G, int bpr) {
-  const int row = (int)blockIdx.x / bpr;  // n * H1 + y
-  const int i = ((int)blockIdx.x - row * bpr) * 256 + (int)threadIdx.x;  // value of the row
-  const int W1 = md.w[1], H1 = md.h[1];
-  if (i >= W1 * G) return;
-  const int x = i / G, c = i - x * G;
-  const int n = row / H1, y = row - n * H1;
+                                                       int G, CollapseGrid cg) {
+  int64_t row, i;  // row: n * H1 + y
+  if (!collapse_place(cg, row, i)) return;
+  const int H1 = md.h[1];
+  const int x = (int)div_n(i, cg.vals, G), c = (int)(i - (int64_t)x * G);
+  const int n = (int)div_n(row, cg.rows, H1), y = (int)(row - (int64_t)n * H1);
   VecF<V>* d = reinterpret_cast<VecF<V>*>(d_pyr);
   auto at = [&](int k) -> VecF<V>& {
     const int sh = k - 1;
@@ -2440,16 +2463,16 @@ __global__ void __launch_bounds__(256) k_mip_collapse1(float* __restrict__ d_pyr
 
 template <int V>
 __global__ void __launch_bounds__(256) k_mip_collapse0(const float* __restrict__ d_pyr, MipDesc md,
-                                                       int G, int bpr, float* __restrict__ d_tex) {
-  const int64_t row = (int64_t)blockIdx.x / bpr;  // n * H + y
-  const int i = ((int)blockIdx.x - (int)row * bpr) * 256 + (int)threadIdx.x;
-  const int W = md.w[0], H = md.h[0];
-  if (i >= W * G) return;
-  const int x = i / G, c = i - x * G;
-  const int n = (int)row / H, y = (int)row - n * H;
+                                                       int G, CollapseGrid cg,
+                                                       float* __restrict__ d_tex) {
+  int64_t row, i;  // row: n * H + y
+  if (!collapse_place(cg, row, i)) return;
+  const int H = md.h[0];
+  const int x = (int)div_n(i, cg.vals, G), c = (int)(i - (int64_t)x * G);
+  const int n = (int)div_n(row, cg.rows, H), y = (int)(row - (int64_t)n * H);
   const VecF<V> t = reinterpret_cast<const VecF<V>*>(
       d_pyr)[md.off[1] / V + (((int64_t)n * md.h[1] + (y >> 1)) * md.w[1] + (x >> 1)) * G + c];
-  VecF<V>* dp = reinterpret_cast<VecF<V>*>(d_tex) + row * W * G + i;
+  VecF<V>* dp = reinterpret_cast<VecF<V>*>(d_tex) + row * cg.vals + i;
   VecF<V> d = *dp;
 #pragma unroll
   for (int j = 0; j < V; ++j) d.v[j] += t.v[j] * 0.25f;
@@ -3029,11 +3052,11 @@ extern "C" int dr_texture_build_mip(const float* tex, int Nt, int H, int W, int 
     {
       DR_TIMED("k_mip_block", stream);
       if (C == 4 && (((uintptr_t)src | (uintptr_t)pyramid) & 15) == 0)
-        hipLaunchKernelGGL(k_mip_block_c4, dim3((unsigned)blocks), dim3(256), 0, stream, src,
-                           pyramid, md, sl, m);
+        hipLaunchKernelGGL(k_mip_block_c4, grid_xy(blocks), dim3(256), 0, stream, src, pyramid, md,
+                           sl, m, blocks);
       else
-        hipLaunchKernelGGL(k_mip_block, dim3((unsigned)blocks), dim3(256), 0, stream, src, pyramid,
-                           md, sl, m, C);
+        hipLaunchKernelGGL(k_mip_block, grid_xy(blocks), dim3(256), 0, stream, src, pyramid, md, sl,
+                           m, C, blocks);
     }
     DR_CHECK_LAUNCH();
     sl += m;
@@ -3094,21 +3117,30 @@ static int mip_collapse(float* d_pyr, const MipDesc& md, int ntex, int Ht, int W
   DR_TIMED("k_mip_collapse", stream);
   const bool vec = C % 4 == 0 && (((uintptr_t)d_pyr | (uintptr_t)d_tex) & 15) == 0;
   const int G = vec ? C / 4 : C;  // values of a texel
+  auto deal = [&](int h, int w) {
+    CollapseGrid g;
+    g.rows = (int64_t)ntex * h;
+    g.vals = (int64_t)w * G;
+    g.log = 0;
+    while (g.log < 8 && (1 << g.log) < g.vals) ++g.log;
+    g.bpr = (int)((g.vals + (1 << g.log) - 1) >> g.log);
+    const int per = 256 >> g.log;  // rows of a workgroup
+    g.blocks = (g.rows + per - 1) / per * g.bpr;
+    return g;
+  };
   if (md.L >= 3) {
-    const int bpr = (int)(((int64_t)md.w[1] * G + 255) / 256);
-    const dim3 grid((unsigned)((int64_t)ntex * md.h[1] * bpr));
+    const CollapseGrid g = deal(md.h[1], md.w[1]);
     if (vec)
-      hipLaunchKernelGGL(k_mip_collapse1<4>, grid, dim3(256), 0, stream, d_pyr, md, G, bpr);
+      hipLaunchKernelGGL(k_mip_collapse1<4>, grid_xy(g.blocks), dim3(256), 0, stream, d_pyr, md, G, g);
     else
-      hipLaunchKernelGGL(k_mip_collapse1<1>, grid, dim3(256), 0, stream, d_pyr, md, G, bpr);
+      hipLaunchKernelGGL(k_mip_collapse1<1>, grid_xy(g.blocks), dim3(256), 0, stream, d_pyr, md, G, g);
     DR_CHECK_LAUNCH();
   }
-  const int bpr = (int)(((int64_t)Wt * G + 255) / 256);
-  const dim3 grid((unsigned)((int64_t)ntex * Ht * bpr));
+  const CollapseGrid g = deal(Ht, Wt);
   if (vec)
-    hipLaunchKernelGGL(k_mip_collapse0<4>, grid, dim3(256), 0, stream, d_pyr, md, G, bpr, d_tex);
+    hipLaunchKernelGGL(k_mip_collapse0<4>, grid_xy(g.blocks), dim3(256), 0, stream, d_pyr, md, G, g, d_tex);
   else
-    hipLaunchKernelGGL(k_mip_collapse0<1>, grid, dim3(256), 0, stream, d_pyr, md, G, bpr, d_tex);
+    hipLaunchKernelGGL(k_mip_collapse0<1>, grid_xy(g.blocks), dim3(256), 0, stream, d_pyr, md, G, g, d_tex);
   DR_CHECK_LAUNCH();
   return DR_OK;
 }

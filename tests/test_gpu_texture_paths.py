@@ -286,3 +286,30 @@ def test_sums_of_a_tile_are_exact(kind, C):
     DiffRast.texture(t, dev(uv), **kw).backward(dev(g))
     got = host(t.grad)[0]
     np.testing.assert_array_equal(got[4] if kind == "cube" else got, ref)
+
+
+# the pyramid's backward on rows shorter and longer than a workgroup
+@pytest.mark.parametrize("C", [1, 3, 4, 8])
+@pytest.mark.parametrize("Ht,Wt", [(64, 2), (6, 2), (48, 16), (8, 520)])
+@pytest.mark.parametrize("Nt", [1, 3])
+def test_pyramid_backward_rows(C, Ht, Wt, Nt):
+    torch_dev()
+    rng = np.random.default_rng(Ht + Wt + C)
+    uv = rng.uniform(0.0, 1.0, size=(3, 17, 19, 2)).astype(np.float32)
+    da = rng.uniform(0.9, 1.1, size=(3, 17, 19, 4)).astype(np.float32) * np.float32(1.6 / max(Ht, Wt))
+    tex = rng.random((Nt, Ht, Wt, C)).astype(np.float32)
+    check(rng, tex, uv, da, "linear-mipmap-linear", "clamp")
+
+
+def test_pyramid_of_more_rows_than_a_grid():
+    """2^24 + 2 texel rows: as one workgroup of 256 threads a row, the
+    pyramid's backward would be a grid of more than 2^32 threads, of which a
+    launch runs a part (the general kernel's sides above 32,767 too)."""
+    torch_dev()
+    rng = np.random.default_rng(0)
+    Ht, Wt = 2 ** 24 + 2, 2
+    uv = rng.uniform(0.0, 1.0, size=(1, 16, 16, 2)).astype(np.float32)
+    da = np.full((1, 16, 16, 4), 1.4 / Ht, np.float32)
+    da[..., :2] = 0.0
+    tex = rng.random((1, Ht, Wt, 1)).astype(np.float32)
+    check(rng, tex, uv, da, "linear-mipmap-linear", "clamp")
