@@ -137,6 +137,12 @@ Tensor cotangent(const Tensor& g, at::IntArrayRef sizes, const Tensor& like) {
   return g.defined() ? f32(g) : zeros(sizes, like);
 }
 
+// A side input is read by the kernels that run on the main input's device.
+void check_device(const char* what, const Tensor& t, const Tensor& main) {
+  TORCH_CHECK_VALUE(t.is_cuda() && t.device() == main.device(), what, " must be on the device of ",
+                    "the other tensors (got ", t.device(), " and ", main.device(), ")");
+}
+
 void check_tri(const char* op, const Tensor& tri) {
   TORCH_CHECK_VALUE(tri.dim() == 2 && tri.size(1) == 3, op, ": tri must be [T, 3] (got ",
                     tri.sizes(), ")");
@@ -389,6 +395,7 @@ std::tuple<Tensor, Tensor> interpolate_op(const Tensor& attr, const Tensor& rast
   TORCH_CHECK_VALUE(rast_db.has_value(), "interpolate: rastDB is required when diffAttrs is set");
   TORCH_CHECK_VALUE(rast_db->sizes() == rast.sizes(), "interpolate: rastDB must match rast shape (got ",
                     rast_db->sizes(), " vs ", rast.sizes(), ")");
+  check_device("interpolate: rastDB", *rast_db, rast);
   Tensor diff_dev;
   if (mode == 2) {
     TORCH_CHECK_VALUE(!diff.empty(), "interpolate: diffAttrs.indices must be non-empty");
@@ -468,6 +475,7 @@ Tensor bias_map_of(const OptTensor& m, const Tensor& uv) {
                         m->sizes().slice(0, 3) == uv.sizes().slice(0, 3),
                     "texture: mipLevelBiasMap must be [N, H_img, W_img] or [N, H_img, W_img, 1] (got ",
                     m->sizes(), ")");
+  check_device("texture: mipLevelBiasMap", *m, uv);
   return f32(*m);
 }
 
@@ -497,6 +505,7 @@ Tensor texture_op(const Tensor& tex, const Tensor& uv, const OptTensor& uv_da, i
     TORCH_CHECK_VALUE(da_fits && uv_da->size(3) == 6,
                       "texture: cube mipmap filterModes require uvDA [N, H_img, W_img, 6] "
                       "(direction derivatives)");
+    check_device("texture: uvDA", *uv_da, uvf);
     return TextureFn::apply(texf, uvf, OptTensor(f32(*uv_da)), some(bias_map_of(bias_map, uvf)),
                             filt, boundary, bias, (int64_t)0, OptTensor(), dir_grad);
   }
@@ -512,6 +521,7 @@ Tensor texture_op(const Tensor& tex, const Tensor& uv, const OptTensor& uv_da, i
   TORCH_CHECK_VALUE(uv_da.has_value(), "texture: mipmap filterModes require uvDA");
   TORCH_CHECK_VALUE(da_fits && uv_da->size(3) == 4,
                     "texture: uvDA must be [N, H_img, W_img, 4] (got ", uv_da->sizes(), ")");
+  check_device("texture: uvDA", *uv_da, uvf);
   return TextureFn::apply(texf, uvf, OptTensor(f32(*uv_da)), some(bias_map_of(bias_map, uvf)), filt,
                           boundary, bias, levels, pyramid, false);
 }
@@ -574,11 +584,16 @@ Tensor antialias_op(const Tensor& color, const Tensor& rast, const Tensor& pos, 
                     pos.sizes(), ")");
   TORCH_CHECK_VALUE(color.is_cuda() && rast.is_cuda() && pos.is_cuda(),
                     "antialias: tensors must be on a ROCm device");
+  // (read per image and per triangle)
+  TORCH_CHECK_VALUE(pos.size(0) >= color.size(0), "antialias: pos must have color's batch (got ",
+                    pos.sizes(), " for ", color.size(0), " images)");
   const Tensor tri32 = tri_of(tri, color.device());
   check_tri("antialias", tri32);
   Tensor topo;
   if (topology.has_value()) {
     topo = tri_of(*topology, color.device());
+    TORCH_CHECK_VALUE(topo.numel() >= tri32.numel(), "antialias: topologyHash must be [T, 3] (got ",
+                      topo.sizes(), " for ", tri32.size(0), " triangles)");
   } else {
     topo = at::empty_like(tri32);
     check(api.dr_antialias_topology(i32(tri32), (int)tri32.size(0), (int32_t*)topo.data_ptr(),

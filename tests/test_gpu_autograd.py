@@ -112,3 +112,34 @@ def test_threads_and_streams():
     [t.start() for t in ts]
     [t.join() for t in ts]
     assert not bad, bad[0]
+
+
+def test_side_inputs_are_checked():
+    """Inputs beside the main ones that are on the host, or too small for
+    what the kernels read of them, are ValueErrors before any launch."""
+    torch = torch_dev()
+    from diffrast import DiffRast
+    pos, tri, uv, tex = scene()
+    rast, db = DiffRast.rasterize(pos, tri, (40, 36))
+    a, da = DiffRast.interpolate(uv, rast, tri, rastDB=db, diffAttrs="all")
+    mip = dict(filterMode="linear-mipmap-linear")
+    d = torch.nn.functional.pad(a, (0, 1), value=1.0)
+    cube = torch.rand(1, 6, 8, 8, 3, device="cuda")
+    bias = torch.zeros(a.shape[:3])
+    for call, msg in [
+            (lambda: DiffRast.interpolate(uv, rast, tri, rastDB=db.cpu(), diffAttrs="all"), "rastDB"),
+            (lambda: DiffRast.interpolate(uv, rast, tri, rastDB=db.cpu(), diffAttrs=[0]), "rastDB"),
+            (lambda: DiffRast.texture(tex, a, uvDA=da.cpu(), **mip), "uvDA"),
+            (lambda: DiffRast.texture(tex, a, uvDA=da, mipLevelBiasMap=bias, **mip), "mipLevelBiasMap"),
+            (lambda: DiffRast.texture(cube, d, uvDA=torch.zeros(*a.shape[:3], 6), boundaryMode="cube",
+                                      **mip), "uvDA")]:
+        with pytest.raises(ValueError, match=msg + " must be on the device"):
+            call()
+    col = DiffRast.texture(tex, a)
+    with pytest.raises(ValueError, match="color's batch"):
+        DiffRast.antialias(col, rast, pos[:1], tri)
+    with pytest.raises(ValueError, match="topologyHash must be"):
+        DiffRast.antialias(col, rast, pos, tri, topologyHash=tri[:4])
+    topo = DiffRast.antialiasConstructTopologyHash(tri)
+    out = DiffRast.antialias(col, rast, pos, tri, topologyHash=topo)
+    np.testing.assert_array_equal(host(out), host(DiffRast.antialias(col, rast, pos, tri)))
