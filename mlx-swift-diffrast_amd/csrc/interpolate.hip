@@ -214,8 +214,16 @@ __global__ void __launch_bounds__(256) k_interp_fwd_any(
   const int ty = tile / ntx, tx = tile - ty * ntx;
   const int G = (A + 3) >> 2;
   const float* at = attr + (int64_t)img * attr_stride;
-  for (int i = (int)threadIdx.x; i < 256 * G; i += 256) {
-    const int lp = i / G, g = i - lp * G, a = g * 4;
+  // (pixel, chunk) of item i = threadIdx.x, + 256, ... of 256 * G, which need
+  // not fit 32 bits
+  const int step = 256 / G, rest = 256 - step * G;
+  int lp = (int)threadIdx.x / G, g = (int)threadIdx.x - lp * G;
+  for (; lp < 256; lp += step, g += rest) {
+    if (g >= G) {
+      g -= G;
+      if (++lp >= 256) break;
+    }
+    const int a = g * 4;
     const int pw = tx * 16 + (lp & 15), ph = ty * 16 + (lp >> 4);
     if (pw >= W || ph >= H) continue;
     const int64_t pix = ((int64_t)img * H + ph) * W + pw;

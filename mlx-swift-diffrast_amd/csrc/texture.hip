@@ -1671,8 +1671,16 @@ __global__ void __launch_bounds__(256) k_tex_fwd_many(
   const int ty = tile / ntx, tx = tile - ty * ntx;
   const int G = (C + 3) >> 2;  // chunks of four channels
   const bool shared = tex_stride == 0;
-  for (int i = (int)threadIdx.x; i < 256 * G; i += 256) {
-    const int lp = i / G, c = (i - lp * G) * 4;  // tile pixel, first channel
+  // (pixel, chunk) of item i = threadIdx.x, + 256, ... of 256 * G, which need
+  // not fit 32 bits
+  const int step = 256 / G, rest = 256 - step * G;
+  int lp = (int)threadIdx.x / G, g = (int)threadIdx.x - lp * G;
+  for (; lp < 256; lp += step, g += rest) {
+    if (g >= G) {
+      g -= G;
+      if (++lp >= 256) break;
+    }
+    const int c = g * 4;  // first channel
     const int ph = ty * 16 + (lp >> 4), pw = tx * 16 + (lp & 15);
     if (ph >= Hi || pw >= Wi) continue;
     const int64_t pix = ((int64_t)n * Hi + ph) * Wi + pw;

@@ -87,3 +87,17 @@ def test_sums_of_a_tile_are_exact(A, diff):
         ref[0, idx] -= u_term
         ref[1, idx] += u_term
     np.testing.assert_array_equal(host(attr.grad)[0], ref)
+
+
+def test_more_attributes_than_a_tile_counts_in_32_bits():
+    """2^25 + 5 attributes: the forward's 256 pixels times chunks of four are
+    more than 2^31 items."""
+    torch = torch_dev()
+    from diffrast import DiffRast
+    A = 2 ** 25 + 5
+    attr = torch.rand(1, 3, A, device="cuda")
+    rast = torch.tensor([0.25, 0.5, 0.0, 1.0], device="cuda").reshape(1, 1, 1, 4)
+    tri = torch.tensor([[0, 1, 2]], dtype=torch.int32, device="cuda")
+    out = DiffRast.interpolate(attr, rast, tri)[0].reshape(-1)
+    want = 0.25 * attr[0, 0] + 0.25 * attr[0, 1] + 0.5 * attr[0, 2]
+    assert float((out - want).abs().max()) < 1e-6

@@ -313,3 +313,15 @@ def test_pyramid_of_more_rows_than_a_grid():
     da[..., :2] = 0.0
     tex = rng.random((1, Ht, Wt, 1)).astype(np.float32)
     check(rng, tex, uv, da, "linear-mipmap-linear", "clamp")
+
+
+def test_more_channels_than_a_tile_counts_in_32_bits():
+    """2^25 + 5 channels: 256 pixels times chunks of four are more than 2^31
+    items."""
+    torch = torch_dev()
+    from diffrast import DiffRast
+    C = 2 ** 25 + 5
+    tex = torch.rand(1, 1, 2, C, device="cuda")
+    uv = torch.tensor([0.5, 0.5], device="cuda").reshape(1, 1, 1, 2)
+    out = DiffRast.texture(tex, uv, filterMode="linear", boundaryMode="clamp").reshape(-1)
+    assert float((out - tex[0, 0].mean(0)).abs().max()) < 1e-6
