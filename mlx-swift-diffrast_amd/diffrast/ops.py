@@ -112,16 +112,16 @@ class MipPyramid(list):
         self.source_version = tex._version
 
 
-def _packed_pyramid(levels, tex, tex_arg):
+def _packed_pyramid(levels, tex):
     """(L, packed levels 1..L-1) of a `textureConstructMip` list: its levels
     are views of one buffer in the library's packing, used as they are; any
     other list of [Nt, Hk, Wk, C] levels is packed by a copy.  A
-    `MipPyramid` must still describe `tex_arg` as it is now."""
+    `MipPyramid` must still describe `tex` as it is now."""
     if isinstance(levels, MipPyramid):
-        if tex_arg.data_ptr() != levels.source_ptr:
+        if tex.data_ptr() != levels.source_ptr:
             raise ValueError("texture: mip was built from another texture tensor "
                              "(textureConstructMip(tex) of the tex passed here)")
-        if tex_arg._version != levels.source_version:
+        if tex._version != levels.source_version:
             raise ValueError("texture: tex was modified in place after textureConstructMip; "
                              "rebuild mip from the current texture")
     levels = list(levels)
@@ -275,7 +275,7 @@ class DiffRast:
         if mip is not None and (bnd == BoundaryMode.cube or filt >= FilterMode.linearMipmapNearest):
             if bnd == BoundaryMode.cube:
                 raise ValueError("texture: a prebuilt `mip` is for 2D textures")
-            levels, pyramid = _packed_pyramid(mip, tex.to(torch.float32).contiguous(), tex)
+            levels, pyramid = _packed_pyramid(mip, tex)
         return _lib.ops().texture(tex, uv, uvDA, int(filt), int(bnd), float(mipLevelBias),
                                   mipLevelBiasMap, levels, pyramid, bool(dirGrad))
 

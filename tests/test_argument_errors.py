@@ -28,3 +28,15 @@ TRI = torch.zeros((1, 3), dtype=torch.int32)
 def test_value_errors(call, msg):
     with pytest.raises(ValueError, match=msg):
         call()
+
+
+def test_prebuilt_mip_converts_nothing(monkeypatch):
+    """A prebuilt pyramid is matched against the texture's shape; the texture
+    itself is converted once, by the compiled node."""
+    def refuse(*_, **__):
+        raise AssertionError("converted")
+    tex = torch.zeros(1, 4, 4, 3, dtype=torch.float16)
+    monkeypatch.setattr(torch.Tensor, "to", refuse)
+    with pytest.raises(ValueError, match="ROCm device"):
+        DiffRast.texture(tex, torch.zeros(1, 2, 2, 2), uvDA=torch.zeros(1, 2, 2, 4),
+                         filterMode="linear-mipmap-linear", mip=[tex])
