@@ -1366,14 +1366,17 @@ static int bin_lds_chunks(int N, int tiles, int64_t max_items) {
   return (int)chunks;
 }
 
-// Allows the binning kernels more than 64 KiB of dynamic LDS (images of more
-// than 16,384 tiles, which are never balanced: kBinBalTiles).
-static void bin_lds_large() {
-  const int bytes = kBinLdsTiles * (int)sizeof(int);
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k_bin_lds<true, false>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k_bin_lds<false, false>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+// Allows the binning kernel of a pass more than 64 KiB of dynamic LDS (images
+// of more than 16,384 tiles, which are never balanced: kBinBalTiles); false
+// where that is refused.
+static bool bin_lds_large(bool fill) {
+  const void* f = fill ? reinterpret_cast<const void*>(k_bin_lds<true, false>)
+                       : reinterpret_cast<const void*>(k_bin_lds<false, false>);
+  if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                          kBinLdsTiles * (int)sizeof(int)) == hipSuccess)
+    return true;
+  (void)hipGetLastError();
+  return false;
 }
 
 // Per-tile counts (FILL false) or counts and lists (FILL true) of the items.
@@ -1387,11 +1390,11 @@ static int64_t launch_binning(bool fill, const Items& it, int64_t n_items, int64
                               int cap, hipStream_t stream, int64_t* wstats = nullptr,
                               int64_t wcap = 0, bool bal = false) {
   if (n_items == 0) return 0;
-  const int chunks = bin_lds_chunks(N, tiles, max_items);
+  int chunks = bin_lds_chunks(N, tiles, max_items);
+  const size_t lds = (size_t)((tiles + 3) / 4) * sizeof(int4);
+  if (chunks > 0 && lds > 64 * 1024 && !bin_lds_large(fill)) chunks = 0;  // counters in memory
   if (chunks > 0) {
     const dim3 grid((unsigned)((int64_t)N * chunks));
-    const size_t lds = (size_t)((tiles + 3) / 4) * sizeof(int4);
-    if (lds > 64 * 1024) bin_lds_large();
     if (fill) {
       const int64_t waves = (int64_t)N * chunks * (kBinThreads / 64);
       if (waves > wcap) wstats = nullptr;
