@@ -252,10 +252,10 @@ def test_cached_pyramid_stale():
     assert_fwd_close(host(out), ref)
 
 
-@pytest.mark.parametrize("C", [4, 5])
+@pytest.mark.parametrize("C", [4, 5, 129])
 def test_level_above_2g_elements(C):
-    """A texture level of more than 2^31 floats (C = 4: the windowed
-    backward, sides up to 32767; C = 5: the tiled backward): texel offsets
+    """A texture level of more than 2^31 floats (C = 4 and 5: the windowed
+    backwards, sides up to 32767; C = 129: the general one): texel offsets
     are formed in 64 bits (32 bits where a level stays below 2^32 floats).
     16 pixels sample the last 8x8 texels; their outputs and gradients equal
     those of the same texels as a texture of their own (the pixels' uv
@@ -263,7 +263,7 @@ def test_level_above_2g_elements(C):
     and d_tex is zero away from them."""
     torch = torch_dev()
     from diffrast import DiffRast
-    S = 23200 if C == 4 else 20800
+    S = {4: 23200, 5: 20800, 129: 4100}[C]
     assert S * S * C > 2 ** 31
     gen = torch.Generator(device="cuda").manual_seed(C)
     tex = torch.rand((1, S, S, C), device="cuda", generator=gen).requires_grad_(True)

@@ -325,3 +325,21 @@ def test_more_channels_than_a_tile_counts_in_32_bits():
     uv = torch.tensor([0.5, 0.5], device="cuda").reshape(1, 1, 1, 2)
     out = DiffRast.texture(tex, uv, filterMode="linear", boundaryMode="clamp").reshape(-1)
     assert float((out - tex[0, 0].mean(0)).abs().max()) < 1e-6
+
+
+# a side above 32,767, where windows' 16-bit coordinates end: the general
+# kernel at every compiled channel count, and the run-time one
+@pytest.mark.parametrize("C", [1, 2, 3, 4, 6])
+@pytest.mark.parametrize("filt,bnd", [("nearest", "wrap"), ("nearest", "zero"), ("linear", "clamp"),
+                                      ("linear", "wrap"), ("linear-mipmap-linear", "zero"),
+                                      ("linear-mipmap-nearest", "clamp")])
+@pytest.mark.parametrize("Ht,Wt", [(2, 40000), (32768, 4)])
+def test_long_sides(C, filt, bnd, Ht, Wt):
+    torch_dev()
+    rng = np.random.default_rng(C + Ht)
+    uv = rng.uniform(-0.2, 1.2, size=(2, 18, 23, 2)).astype(np.float32)
+    uv[:, 4:9] = uv[:, 4:5, :1]  # and pixels of one footprint
+    da = rng.uniform(0.9, 1.1, size=(2, 18, 23, 4)).astype(np.float32)
+    da *= np.float32([1.3 / Wt, 1.2 / Wt, 1.0 / Ht, 0.9 / Ht])
+    tex = rng.random((1, Ht, Wt, C)).astype(np.float32)
+    check(rng, tex, uv, da, filt, bnd)
