@@ -280,8 +280,10 @@ std::tuple<Tensor, Tensor> rasterize_op(const Tensor& pos, const Tensor& tri, in
                     "rasterize: maxPerTile must be in [0, 1024] (0: no limit)");
   const Tensor posc = posf.contiguous();
   // Reuse (peel layers only): the same pos and tri tensors as the previous
-  // call on this stream, read in place and unchanged since.
-  const bool in_place = posc.const_data_ptr() == pos.const_data_ptr() && tri.is_cuda() &&
+  // call on this stream, read in place and unchanged since.  (A transform's
+  // wrapper has no storage: apply() refuses it by name.)
+  const bool in_place = pos.has_storage() && tri32.has_storage() && tri.is_cuda() &&
+                        posc.const_data_ptr() == pos.const_data_ptr() &&
                         tri32.const_data_ptr() == tri.const_data_ptr();
   const Where at_ = place_of(posc);
   bool again = false;

@@ -57,13 +57,32 @@ def test_in_place_change_is_refused():
 
 
 def test_transforms_are_refused():
+    """vmap, functorch's gradients and forward mode pass autograd nodes by:
+    each op refuses them by name (and takes the same call without)."""
     torch = torch_dev()
     from diffrast import DiffRast
+    from diffrast.fit import mse_loss
+    import torch.autograd.forward_ad as forward_ad
     pos, tri, uv, tex = scene()
-    with pytest.raises(Exception):
-        torch.func.vmap(lambda t: DiffRast.rasterize(t, tri, (8, 8))[0])(pos[None])
-    with pytest.raises(Exception):
-        torch.func.jvp(lambda t: DiffRast.rasterize(t, tri, (8, 8))[0], (pos,), (pos,))
+    rast, db = DiffRast.rasterize(pos, tri, (8, 8))
+    a, _ = DiffRast.interpolate(uv, rast, tri)
+    col = DiffRast.texture(tex, a)
+    topo = DiffRast.antialiasConstructTopologyHash(tri)
+    ops = [(lambda t: DiffRast.rasterize(t, tri, (8, 8))[0], pos),
+           (lambda t: DiffRast.interpolate(t, rast, tri)[0], uv),
+           (lambda t: DiffRast.texture(t, a), tex),
+           (lambda t: DiffRast.antialias(t, rast, pos, tri, topologyHash=topo), col),
+           (lambda t: mse_loss(t, col), col.clone())]
+    for op, x in ops:
+        assert torch.isfinite(op(x)).all()
+        for call in (lambda: torch.func.vmap(op)(x[None]),
+                     lambda: torch.func.grad(lambda t: op(t).sum())(x),
+                     lambda: torch.func.jvp(op, (x,), (x,))):
+            with pytest.raises(RuntimeError, match="torch::autograd::Function with functorch"):
+                call()
+        with forward_ad.dual_level():
+            with pytest.raises(RuntimeError, match="jvp is not implemented"):
+                op(forward_ad.make_dual(x, x))
 
 
 def test_partial_cotangents():
