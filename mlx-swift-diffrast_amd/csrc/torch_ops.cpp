@@ -171,18 +171,24 @@ struct LastRaster {
   std::vector<int32_t> ranges;
 };
 // The last rasterize forward per (device, stream): its pos and tri buffers
-// (address, shape, strides) and pos's version.  A backward whose pos and tri
-// are those buffers, pos at that version, differentiates a forward over the
-// same data (autograd has checked that its saved pos is unchanged since its
-// own forward; a later in-place change would have bumped the version), so it
-// may reuse the per-triangle values the last forward stored
-// (DR_RASTERIZE_BWD_REUSE; the peel layers of one pos all qualify).
+// (storage, address, shape, strides) and pos's version.  A backward whose pos
+// and tri are those buffers, pos at that version, differentiates a forward
+// over the same data (autograd has checked that its saved pos is unchanged
+// since its own forward; a later in-place change would have bumped the
+// version), so it may reuse the per-triangle values the last forward stored
+// (DR_RASTERIZE_BWD_REUSE; the peel layers of one pos all qualify).  The
+// storages are weak references: an address alone may by then be that of
+// another tensor (a hook on saved tensors brings pos back in new memory).
+using WeakStorage = c10::weak_intrusive_ptr<c10::StorageImpl>;
 struct FwdKey {
+  WeakStorage pos_storage, tri_storage;
   const void *pos, *tri;
   int64_t version;
   std::vector<int64_t> pos_sizes, pos_strides, tri_sizes;
   bool operator==(const FwdKey& o) const {
-    return pos == o.pos && tri == o.tri && version == o.version && pos_sizes == o.pos_sizes &&
+    return pos_storage._unsafe_get_target() == o.pos_storage._unsafe_get_target() &&
+           tri_storage._unsafe_get_target() == o.tri_storage._unsafe_get_target() &&
+           pos == o.pos && tri == o.tri && version == o.version && pos_sizes == o.pos_sizes &&
            pos_strides == o.pos_strides && tri_sizes == o.tri_sizes;
   }
 };
@@ -191,7 +197,8 @@ std::map<Where, LastRaster> g_last_raster;
 std::map<Where, FwdKey> g_last_fwd;
 
 FwdKey fwd_key(const Tensor& pos, const Tensor& tri) {
-  return {pos.const_data_ptr(), tri.const_data_ptr(), (int64_t)pos._version(), pos.sizes().vec(),
+  return {pos.storage().getWeakStorageImpl(), tri.storage().getWeakStorageImpl(),
+          pos.const_data_ptr(), tri.const_data_ptr(), (int64_t)pos._version(), pos.sizes().vec(),
           pos.strides().vec(), tri.sizes().vec()};
 }
 
@@ -212,7 +219,7 @@ struct RasterizeFn : torch::autograd::Function<RasterizeFn> {
     {
       FwdKey key = fwd_key(pos, tri);
       std::lock_guard<std::mutex> lk(g_mu);
-      g_last_fwd[place_of(pos)] = std::move(key);
+      g_last_fwd.insert_or_assign(place_of(pos), std::move(key));
     }
     ctx->set_materialize_grads(false);
     ctx->save_for_backward({pos, tri, rast});

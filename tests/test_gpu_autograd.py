@@ -162,3 +162,44 @@ def test_side_inputs_are_checked():
     topo = DiffRast.antialiasConstructTopologyHash(tri)
     out = DiffRast.antialias(col, rast, pos, tri, topologyHash=topo)
     np.testing.assert_array_equal(host(out), host(DiffRast.antialias(col, rast, pos, tri)))
+
+
+def test_saved_pos_back_at_another_tensors_address():
+    """The backward of a forward whose saved pos a hook brings back in new
+    memory, at the address of the last forward's pos by then freed: it must
+    not take that forward's per-triangle values for its own."""
+    torch = torch_dev()
+    from diffrast import DiffRast
+    rng = np.random.default_rng(3)
+    V, T = 1_000_000, 40  # 16 MB: a block of the allocator's own
+    tri = dev(np.arange(3 * T, dtype=np.int32).reshape(T, 3))
+
+    def vertices():
+        p = rng.uniform(-1, 1, size=(1, V, 4)).astype(np.float32)
+        p[..., 3] = 1.0
+        return dev(p)
+    a, b = vertices().requires_grad_(True), vertices()
+    g = torch.randn(1, 64, 64, 4, device="cuda")
+    at = {}
+
+    def pack(t):
+        return t.cpu() if t.shape == a.shape else t.detach()
+
+    def unpack(t):
+        if t.is_cuda:
+            return t
+        t = t.cuda()
+        at["unpacked"] = t.data_ptr()
+        return t
+    ref = torch.autograd.grad(DiffRast.rasterize(a * 1.0, tri, (64, 64))[0], a, g)[0]
+    torch.cuda.synchronize()
+    with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+        rast = DiffRast.rasterize(a * 1.0, tri, (64, 64))[0]
+    with torch.no_grad():
+        other = b * 1.0
+        at["other"] = other.data_ptr()
+        DiffRast.rasterize(other, tri, (64, 64))
+        del other
+    got = torch.autograd.grad(rast, a, g)[0]
+    assert at["unpacked"] == at["other"]  # the case that is meant
+    np.testing.assert_array_equal(host(got), host(ref))
