@@ -904,8 +904,9 @@ __global__ void __launch_bounds__(256) k_tex_bwd(TexBwdArgs A, int total_tiles) 
 
 // ---------------------------------------------------------------------------
 // Windowed backward, C in 1..4: every 2D filter, and bilinear cube maps (a
-// face in the place of a level).  Per 16x16 pixel tile the texel bounding box of the footprints on
-// each level in use is taken, and contributions are summed into dense fp64
+// face in the place of a level).  Per 16x16 pixel tile the texel bounding box
+// of the footprints on each level in use is taken (window_box.h), and
+// contributions are summed into dense fp64
 // LDS windows over those boxes (direct indexing, no hashing; the windows
 // share one pool).  The windows are written out row by row, so consecutive
 // lanes issue atomics to consecutive addresses.  Groups of lanes on one
@@ -1212,8 +1213,8 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
       // flat footprints only (all the weight on one texel: every background
       // pixel), in groups of any size: a few background pixels kept out of
       // the windows keep a tile that mixes them with the object from boxes
-      // spanning both, which the windows cannot hold (their taps then went to
-      // the hash table: 0.299 -> 0.294 ms at 8 x 1024^2); other footprints,
+      // spanning both, which the windows cannot hold (0.299 -> 0.294 ms at 8 x
+      // 1024^2, when such boxes' taps took an LDS hash table); other footprints,
       // however many lanes share them, take the windows' run sums
       // Wrap mode: an empty pixel's footprint (uv = 0) is the texture's four
       // corner texels, so pixels of one uv are grouped instead: those at uv
@@ -3267,8 +3268,8 @@ static int dpyr_get(const DPyrBuf& buf, int64_t np, hipStream_t stream, float*& 
   return d_pyr ? DR_OK : scratch_fail();
 }
 
-// The cube extension's backward: one thread per pixel, d_tex / d_pyramid by
-// global atomics, then the pyramid collapse over the Nt*6 faces.  The first
+// The cube extension's backward: k_cube_bwd (a tile's d_tex and d_pyramid sums
+// in an LDS table), then the pyramid collapse over the Nt*6 faces.  The first
 // `zero_tex` floats of d_tex are cleared first (0: accumulate), after the
 // pyramid gradient's buffer is known to fit, so a refused call leaves d_tex
 // untouched.
