@@ -1948,7 +1948,11 @@ __global__ void __launch_bounds__(256, 3) k_tex_bwd_many(TexBwdArgs A, int total
         if (!(hot.on && hot.ux == lux && hot.uy == luy && hot.base == base)) {
           if (hot.on) {
             hot_flush<kTaps>(hot, C, s_hot[wave]);
+            __builtin_amdgcn_wave_barrier();  // (other lanes' reads, then writes)
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
             for (int c = lane; c < C; c += 64) s_hot[wave][c] = 0.0;
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
           }
           hot.on = true;
           hot.ux = lux;
