@@ -267,7 +267,7 @@ struct AATile {
 // Triangle id of a rast pixel from its fourth channel; ids outside [0, T)
 // read as empty.
 __device__ __forceinline__ int aa_id(float w, int T) {
-  const int id = f2i(w) - 1;
+  const int id = dec(f2i(w));
   return (unsigned)id < (unsigned)T ? id : -1;
 }
 

@@ -194,6 +194,13 @@ __device__ __forceinline__ int f2i(float x) {
   return r;
 }
 
+// i + 1 and i - 1 of a converted float, which may be the largest or smallest
+// int: they wrap.  Of a signed overflow the compiler may assume that it does
+// not happen and check one form of the value, then use the other (a clamped
+// texel column of u * W >= 2^31 was read at -2^31 so).
+__device__ __forceinline__ int inc(int i) { return (int)((unsigned)i + 1u); }
+__device__ __forceinline__ int dec(int i) { return (int)((unsigned)i - 1u); }
+
 // q = i / d, r = i % d for 0 <= i and 0 < d: a 32-bit division while i fits
 // in 31 bits (several times cheaper than the 64-bit one).
 __device__ __forceinline__ void divmod64(int64_t i, int d, int64_t& q, int& r) {

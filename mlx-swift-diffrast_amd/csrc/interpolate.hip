@@ -104,7 +104,7 @@ __global__ void __launch_bounds__(256) k_interp_fwd(
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int q = 0; q < PX; ++q) {
-    t[q] = in[q] ? f2i(r[q].w) - 1 : -1;
+    t[q] = in[q] ? dec(f2i(r[q].w)) : -1;
     if (t[q] >= T) t[q] = -1;  // not a triangle of this mesh: empty
   }
   bool any = false;
@@ -229,7 +229,7 @@ __global__ void __launch_bounds__(256) k_interp_fwd_any(
     const int64_t pix = ((int64_t)img * H + ph) * W + pw;
     const int na = min(4, A - a);
     const float4 r = *reinterpret_cast<const float4*>(rast + pix * 4);
-    int t = f2i(r.w) - 1;
+    int t = dec(f2i(r.w));
     int i0 = 0, i1 = 0, i2 = 0;
     if ((unsigned)t < (unsigned)T) {
       i0 = tri[t * 3 + 0];
@@ -296,7 +296,7 @@ __global__ void __launch_bounds__(256) k_interp_bwd(
   const int64_t pix = ((int64_t)n * H + min(ph, H - 1)) * W + min(pw, W - 1);
 
   const float4 r = *reinterpret_cast<const float4*>(rast + pix * 4);
-  const int t = f2i(r.w) - 1;
+  const int t = dec(f2i(r.w));
   bool valid = inside && t >= 0 && t < T;
   {
     const uint64_t any = __ballot(valid);
@@ -447,7 +447,7 @@ __global__ void __launch_bounds__(256, 6) k_interp_bwd_any(
   const bool inside = pw < W && ph < H;
   const int64_t pix = ((int64_t)n * H + min(ph, H - 1)) * W + min(pw, W - 1);
   const float4 r = *reinterpret_cast<const float4*>(rast + pix * 4);
-  const int t = f2i(r.w) - 1;
+  const int t = dec(f2i(r.w));
   bool valid = inside && t >= 0 && t < T;
   {
     const uint64_t any = __ballot(valid);

@@ -1152,7 +1152,7 @@ __global__ void __launch_bounds__(256) k_raster_bwd(
   bool valid = pw < W && ph < H;
   const int64_t pix = ((int64_t)n * H + min(ph, H - 1)) * W + min(pw, W - 1);
   const float4 r = *reinterpret_cast<const float4*>(rast + pix * 4);
-  const int t = f2i(r.w) - 1;
+  const int t = dec(f2i(r.w));
   valid = valid && t >= 0 && t < T;
   RBwdRec R;
   float4 dr = make_float4(0.f, 0.f, 0.f, 0.f), ddb = dr;

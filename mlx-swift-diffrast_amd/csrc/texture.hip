@@ -85,7 +85,7 @@ __device__ __forceinline__ void wrap_pair(int t, int size, int& i0, int& i1) {
   } else {
     float unused;
     i0 = apply_boundary(t, size, DR_BOUNDARY_WRAP, unused);
-    i1 = apply_boundary(t + 1, size, DR_BOUNDARY_WRAP, unused);
+    i1 = apply_boundary(inc(t), size, DR_BOUNDARY_WRAP, unused);
   }
 }
 
@@ -101,7 +101,7 @@ __device__ __forceinline__ Bilin bilin(float u, float v, int Wk, int Hk, int mod
   const float tx = u * (float)Wk - 0.5f;
   const float ty = v * (float)Hk - 0.5f;
   const int tx0 = f2i(floorf(tx)), ty0 = f2i(floorf(ty));
-  const int tx1 = tx0 + 1, ty1 = ty0 + 1;
+  const int tx1 = inc(tx0), ty1 = inc(ty0);
   b.fx = tx - (float)tx0;
   b.fy = ty - (float)ty0;
   b.tx0 = tx0;
@@ -166,7 +166,7 @@ __device__ __forceinline__ int cube_bilin(float x, float y, float z, int Wt, int
   const float txr = u * (float)Wt - 0.5f;
   const float tyr = v * (float)Ht - 0.5f;
   const int tx0 = f2i(floorf(txr)), ty0 = f2i(floorf(tyr));
-  const int tx1 = tx0 + 1, ty1 = ty0 + 1;
+  const int tx1 = inc(tx0), ty1 = inc(ty0);
   const float fx = txr - (float)tx0, fy = tyr - (float)ty0;
   b.fx = fx;
   b.fy = fy;

@@ -176,3 +176,30 @@ def test_triangle_count_above_32bit_indexing_is_refused():
     rc = lib.dr_antialias_fwd(p, p, p, t, t, 1, 8, 8, 1, 3, T, p, _stream())
     assert rc == L.DR_ERR_ARGUMENT and b"715827882" in lib.dr_get_last_error()
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("A", [2, 5])
+def test_ids_beyond_32_bits_read_as_empty(A):
+    """A rast whose fourth channel is not finite, or beyond the integers."""
+    torch = torch_dev()
+    from diffrast import DiffRast
+    pos, tri, H, W = _scene()
+    rast, _ = O.rasterize(pos, tri, (H, W), max_per_tile=0)
+    for k, value in enumerate([np.inf, -np.inf, np.nan, 3e9, -3e9, -2.0 ** 31, 2.0 ** 31]):
+        rast[:, 30 + k, 30:46, 3] = value
+    empty = rast.copy()
+    empty[:, 30:37, 30:46, 3] = 0.0
+    rng = np.random.default_rng(A)
+    attr = rng.normal(size=(pos.shape[1], A)).astype(np.float32)
+    g = rng.normal(size=(2, H, W, A)).astype(np.float32)
+    color = rng.random((2, H, W, 3)).astype(np.float32)
+    got = []
+    for r in (rast, empty):
+        a, rr, p = dev(attr).requires_grad_(True), dev(r).requires_grad_(True), dev(pos).requires_grad_(True)
+        out = DiffRast.interpolate(a, rr, dev(tri))[0]
+        d = torch.autograd.grad(out, [a, rr], dev(g))
+        aa = DiffRast.antialias(dev(color), dev(r), p, dev(tri))
+        got.append([host(x) for x in (out, *d, aa)])
+    for x, y in zip(*got):
+        assert np.isfinite(x).all()
+        assert_grad_close(x, y, rtol=1e-6)

@@ -343,3 +343,28 @@ def test_long_sides(C, filt, bnd, Ht, Wt):
     da *= np.float32([1.3 / Wt, 1.2 / Wt, 1.0 / Ht, 0.9 / Ht])
     tex = rng.random((1, Ht, Wt, C)).astype(np.float32)
     check(rng, tex, uv, da, filt, bnd)
+
+
+# texel coordinates beyond 32 bits saturate, and the second one of a footprint
+# wraps: every tap is inside the texture
+@pytest.mark.parametrize("C", [1, 3, 4, 6])
+@pytest.mark.parametrize("bnd", ["wrap", "clamp", "zero"])
+@pytest.mark.parametrize("filt", ["nearest", "linear", "linear-mipmap-linear"])
+def test_coordinates_beyond_32_bits(C, bnd, filt):
+    torch_dev()
+    from diffrast import DiffRast
+    rng = np.random.default_rng(C)
+    uv = rng.uniform(0.1, 0.9, size=(1, 9, 17, 2)).astype(np.float32)
+    for k, value in enumerate([np.inf, -np.inf, np.nan, 5e7, -5e7, 3.4e7, 1e30]):
+        uv[0, k, k + 2, k % 2] = value
+        uv[0, k, k + 7] = value
+    da = np.full((1, 9, 17, 4), 1.3 / 64, np.float32) if "mipmap" in filt else None
+    tex = rng.random((1, 64, 64, C)).astype(np.float32)
+    kw = dict(filterMode=filt, boundaryMode=bnd)
+    t = dev(tex).requires_grad_(True)
+    out = DiffRast.texture(t, dev(uv), uvDA=None if da is None else dev(da), **kw)
+    assert_same_nonfinite(host(out), O.texture(tex, uv, uvDA=da, **kw), "out")
+    g = rng.normal(size=out.shape).astype(np.float32)
+    out.backward(dev(g))
+    ref = O.texture_vjp(tex, uv, g, uvDA=da, **kw)[0]
+    assert_same_nonfinite(host(t.grad), ref, "d_tex")
