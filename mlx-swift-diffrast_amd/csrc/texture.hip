@@ -960,8 +960,8 @@ __device__ __forceinline__ int wrap_up(int t, int size) {
   return t < size ? t : t % size;
 }
 
-// a * b, 0 where a is 0 whatever b (an infinity, NaN): one instruction, whose
-// intrinsic has no builtin in this compiler.
+// a * b, 0 where either is 0 whatever the other (an infinity, NaN): one
+// instruction, whose intrinsic has no builtin in this compiler.
 __device__ float mul0(float a, float b) __asm("llvm.amdgcn.fmul.legacy");
 
 // Weight `tap` (0..3: 00, 10, 01, 11) of the wave-uniform lane `leader`.
@@ -1009,7 +1009,8 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
   constexpr int kTaps = FILTER == DR_FILTER_NEAREST ? 1 : 4;
   // A tap of weight zero may lie outside its box, and has a clamped place
   // there: it adds 0 (mul0), and what 0 * g is where a cotangent is not
-  // finite goes to the tap's own texel, apart from the windows.
+  // finite goes to the tap's own texel, apart from the windows.  (So does the
+  // product of a cotangent of zero and a weight that is not finite.)
   constexpr bool kOwnTaps = kTaps == 4 && (kCube || BND == DR_BOUNDARY_WRAP);
   constexpr int kRows = kTaps == 1 ? 1 : 2, kRowVals = (kTaps == 1 ? 1 : 2) * CT;  // texel rows
   const bool shared_tex = A.tex_stride == 0;
@@ -1443,9 +1444,13 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
     __syncthreads();
 
     if constexpr (kOwnTaps) {
-      bool bad = false;  // a cotangent that is not finite
+      // what mul0 left out: 0 * g, and w * 0, where the other is not finite
+      bool bad = false;
 #pragma unroll
       for (int c = 0; c < CT; ++c) bad = bad || 0.0f * g[c] != 0.0f;
+#pragma unroll
+      for (int li = 0; li < (mip ? 2 : 1); ++li)
+        bad = bad || 0.0f * (q[li].w00 + q[li].w10 + q[li].w01 + q[li].w11) != 0.0f;
       if (__ballot(bad) != 0ull) {  // uniform
 #pragma unroll
         for (int li = 0; li < (mip ? 2 : 1); ++li) {
@@ -1454,13 +1459,15 @@ __global__ void __launch_bounds__(kWinThreads, 5) k_tex_bwd_win(TexBwdArgs A, in
           const int k = ql.k, Wk = level_w(k), Hk = level_h(k);
 #pragma unroll 1
           for (int t = 0; t < 4; ++t) {
-            if ((t == 0 ? ql.w00 : t == 1 ? ql.w10 : t == 2 ? ql.w01 : ql.w11) != 0.0f) continue;
+            const float w = t == 0 ? ql.w00 : t == 1 ? ql.w10 : t == 2 ? ql.w01 : ql.w11;
             const int X = win_texel<BND>((t & 1) ? ql.ix1 : ql.ix0, Wk);
             const int Y = win_texel<BND>((t & 2) ? ql.iy1 : ql.iy0, Hk);
             float* p = dlevel_ptr(k) + ((int64_t)Y * Wk + X) * CT;
 #pragma unroll
-            for (int c = 0; c < CT; ++c)
-              if (0.0f * g[c] != 0.0f) unsafeAtomicAdd(p + c, 0.0f * g[c]);
+            for (int c = 0; c < CT; ++c) {
+              const float x = w * g[c];
+              if ((w == 0.0f || g[c] == 0.0f) && x != 0.0f) unsafeAtomicAdd(p + c, x);
+            }
           }
         }
       }
@@ -1769,9 +1776,10 @@ __device__ __forceinline__ void hot_flush(const ManyHot& h, int C, const double*
 // The taps of weight zero of one pixel's footprints (a border's merged ones, a
 // texel centre's, those outside the image; slot 0's unless it is in the hot
 // sum): 0 * g is 0, or NaN where a cotangent is not finite, and then belongs
-// to the tap's own texel, which need not be in any window.  Computed from the
-// inputs again, so that nothing of it is kept in registers through the
-// channels (k_tex_bwd_many spills already).
+// to the tap's own texel, which need not be in any window.  So does NaN of a
+// weight that is not finite and a cotangent of zero.  Computed from the inputs
+// again, so that nothing of it is kept in registers through the channels
+// (k_tex_bwd_many spills already).
 template <int FILTER, int BND>
 __device__ __forceinline__ void zero_taps(const TexBwdArgs& A, int n, int64_t pix, bool in_hot) {
   constexpr bool kCube = BND == DR_BOUNDARY_CUBE;
@@ -1779,9 +1787,6 @@ __device__ __forceinline__ void zero_taps(const TexBwdArgs& A, int n, int64_t pi
   constexpr int kTaps = FILTER == DR_FILTER_NEAREST ? 1 : 4;
   asm volatile("" : "+v"(pix));  // (not the values computed before)
   const float* gp = A.d_out + pix * A.C;
-  bool bad = false;
-  for (int c = 0; c < A.C; ++c) bad = bad || 0.0f * gp[c] != 0.0f;
-  if (!bad) return;
   Lod ld;
   ld.k0 = ld.k1 = 0;
   ld.frac = 0.0f;
@@ -1812,11 +1817,12 @@ __device__ __forceinline__ void zero_taps(const TexBwdArgs& A, int n, int64_t pi
                                       (A.tex_stride == 0 ? 0 : (int64_t)n * Hk * Wk * A.C);
 #pragma unroll
     for (int t = 0; t < kTaps; ++t) {
-      if ((t == 0 ? b.w00 : t == 1 ? b.w10 : t == 2 ? b.w01 : b.w11) != 0.0f) continue;
+      const float w = t == 0 ? b.w00 : t == 1 ? b.w10 : t == 2 ? b.w01 : b.w11;
+      if (w != 0.0f && 0.0f * w == 0.0f) continue;
       float* p = lv + ((int64_t)((t & 2) ? b.iy1 : b.iy0) * Wk + ((t & 1) ? b.ix1 : b.ix0)) * A.C;
       for (int c = 0; c < A.C; ++c) {
-        const float x = 0.0f * gp[c];
-        if (x != 0.0f) unsafeAtomicAdd(p + c, x);
+        const float gc = gp[c], x = w * gc;
+        if ((w == 0.0f || gc == 0.0f) && x != 0.0f) unsafeAtomicAdd(p + c, x);
       }
     }
   }
@@ -1978,13 +1984,15 @@ __global__ void __launch_bounds__(256, 3) k_tex_bwd_many(TexBwdArgs A, int total
       }
     }
 
-    // taps of weight zero (zero_taps), other than the hot sum's
+    // taps of weight zero, or not finite (zero_taps), other than the hot sum's
     bool zeros = false;
 #pragma unroll
     for (int li = 0; li < (mip ? 2 : 1); ++li)
       zeros = zeros || (valid && q[li].scale != 0.0f && !(li == 0 && in_hot) &&
                         (q[li].w00 == 0.0f ||
-                         (kTaps == 4 && (q[li].w10 == 0.0f || q[li].w01 == 0.0f || q[li].w11 == 0.0f))));
+                         (kTaps == 4 &&
+                          (q[li].w10 == 0.0f || q[li].w01 == 0.0f || q[li].w11 == 0.0f ||
+                           0.0f * (q[li].w00 + q[li].w10 + q[li].w01 + q[li].w11) != 0.0f))));
 
     // -- boxes of the levels in use, and their windows (k_tex_bwd_win) -----------
     {

@@ -368,3 +368,31 @@ def test_coordinates_beyond_32_bits(C, bnd, filt):
     out.backward(dev(g))
     ref = O.texture_vjp(tex, uv, g, uvDA=da, **kw)[0]
     assert_same_nonfinite(host(t.grad), ref, "d_tex")
+
+
+# uv that is not finite gives weights that are not: their products with
+# cotangents of zero are NaN too
+@pytest.mark.parametrize("C,bnd,filt", [(1, "wrap", "linear"), (3, "wrap", "linear"),
+                                        (4, "wrap", "linear-mipmap-linear"), (3, "cube", "linear"),
+                                        (6, "wrap", "linear"), (6, "clamp", "linear"),
+                                        (6, "zero", "linear"), (6, "cube", "linear"),
+                                        (6, "clamp", "linear-mipmap-linear"), (3, "wrap", "nearest"),
+                                        (6, "zero", "nearest")])
+@pytest.mark.parametrize("zero", ["all", "one"])
+def test_nonfinite_uv_zero_cotangent(C, bnd, filt, zero):
+    torch_dev()
+    from diffrast import DiffRast
+    rng = np.random.default_rng(C)
+    Hi, Wi, S = 33, 50, 64
+    g = rng.normal(size=(2, Hi, Wi, C)).astype(np.float32)
+    uv = rng.uniform(0.1, 0.9, size=(2, Hi, Wi, 3 if bnd == "cube" else 2)).astype(np.float32)
+    for n, y, x, value in [(0, 3, 7, np.nan), (0, 20, 31, np.inf), (1, 9, 40, -np.inf), (1, 32, 49, np.nan)]:
+        uv[n, y, x, 0] = value
+        g[n, y, x, :C if zero == "all" else 1] = 0.0
+    tex = rng.random((1, 6, S, S, C) if bnd == "cube" else (1, S, S, C)).astype(np.float32)
+    kw = dict(filterMode=filt, boundaryMode=bnd)
+    da = np.full((2, Hi, Wi, 4), 1.3 / S, np.float32) if "mipmap" in filt else None
+    t = dev(tex).requires_grad_(True)
+    DiffRast.texture(t, dev(uv), uvDA=None if da is None else dev(da), **kw).backward(dev(g))
+    ref = O.texture_vjp(tex, uv, g, uvDA=da, **kw)[0]
+    assert_same_nonfinite(host(t.grad), ref, "d_tex")
