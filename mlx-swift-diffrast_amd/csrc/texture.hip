@@ -1739,7 +1739,7 @@ __global__ void __launch_bounds__(256) k_tex_fwd_many(
 // a texel's channels as one run of memory.  One footprint set-up serves all
 // channels, and d_uv and the LOD's gradient sum over them in registers.  The
 // general kernel's wave probes and one device atomic per tap and channel
-// took 3,453 us at 2 x 768^2 x 16, trilinear; this takes 194 (182 without
+// took 3,453 us at 2 x 768^2 x 16, trilinear; this takes 186 (181 without
 // zero_taps and the terms of weight 0, which matter for values that are not
 // finite; there, 188 with the direct way's cotangents loaded one pixel at a
 // time, 264 at four waves per SIMD, which spills 46 registers, 211 with two and
@@ -1984,11 +1984,13 @@ __global__ void __launch_bounds__(256, 3) k_tex_bwd_many(TexBwdArgs A, int total
       }
     }
 
-    // taps of weight zero, or not finite (zero_taps), other than the hot sum's
-    bool zeros = false;
+    // Whether zero_taps has anything to add: a cotangent or a weight that is
+    // not finite makes the uv gradient's terms so too, and where there are none
+    // it looks itself at taps of weight zero, or not finite.
+    bool odd = false;
 #pragma unroll
     for (int li = 0; li < (mip ? 2 : 1); ++li)
-      zeros = zeros || (valid && q[li].scale != 0.0f && !(li == 0 && in_hot) &&
+      odd = odd || (!want && valid && q[li].scale != 0.0f && !(li == 0 && in_hot) &&
                         (q[li].w00 == 0.0f ||
                          (kTaps == 4 &&
                           (q[li].w10 == 0.0f || q[li].w01 == 0.0f || q[li].w11 == 0.0f ||
@@ -2233,7 +2235,8 @@ __global__ void __launch_bounds__(256, 3) k_tex_bwd_many(TexBwdArgs A, int total
       }
     }
 
-    if (zeros) zero_taps<FILTER, BND>(A, n, pix, in_hot);
+    if (want) odd = valid && 0.0f * (dfx[0] + dfy[0] + dfx[1] + dfy[1]) != 0.0f;
+    if (odd) zero_taps<FILTER, BND>(A, n, pix, in_hot);
 
     // -- d_uv, d_uvDA, d_bias (Texture.swift:500-520, :979-1102) -----------------
     if (kCube) {

@@ -194,7 +194,8 @@ def test_nearest_nonfinite_cotangent(C, bnd, texels):
                                         (6, "zero", "linear"), (6, "cube", "linear"),
                                         (6, "clamp", "linear-mipmap-linear")])
 @pytest.mark.parametrize("step", [1, 4, 16])  # texels a pixel
-def test_zero_weight_taps_nonfinite_cotangent(C, bnd, filt, step):
+@pytest.mark.parametrize("uv_grad", [False, True])
+def test_zero_weight_taps_nonfinite_cotangent(C, bnd, filt, step, uv_grad):
     torch_dev()
     from diffrast import DiffRast
     rng = np.random.default_rng(C + step)
@@ -215,8 +216,8 @@ def test_zero_weight_taps_nonfinite_cotangent(C, bnd, filt, step):
     kw = dict(filterMode=filt, boundaryMode=bnd)
     # (between two levels: of a level of weight zero no tap is added)
     da = np.full((2, Hi, Wi, 4), 1.3 / S, np.float32) if "mipmap" in filt else None
-    t = dev(tex).requires_grad_(True)
-    DiffRast.texture(t, dev(uv), uvDA=None if da is None else dev(da), **kw).backward(dev(g))
+    t, u = dev(tex).requires_grad_(True), dev(uv).requires_grad_(uv_grad)
+    DiffRast.texture(t, u, uvDA=None if da is None else dev(da), **kw).backward(dev(g))
     ref = O.texture_vjp(tex, uv, g, uvDA=da, **kw)[0]
     assert_same_nonfinite(host(t.grad), ref, "d_tex")
 
@@ -379,7 +380,8 @@ def test_coordinates_beyond_32_bits(C, bnd, filt):
                                         (6, "clamp", "linear-mipmap-linear"), (3, "wrap", "nearest"),
                                         (6, "zero", "nearest")])
 @pytest.mark.parametrize("zero", ["all", "one"])
-def test_nonfinite_uv_zero_cotangent(C, bnd, filt, zero):
+@pytest.mark.parametrize("uv_grad", [False, True])
+def test_nonfinite_uv_zero_cotangent(C, bnd, filt, zero, uv_grad):
     torch_dev()
     from diffrast import DiffRast
     rng = np.random.default_rng(C)
@@ -392,7 +394,7 @@ def test_nonfinite_uv_zero_cotangent(C, bnd, filt, zero):
     tex = rng.random((1, 6, S, S, C) if bnd == "cube" else (1, S, S, C)).astype(np.float32)
     kw = dict(filterMode=filt, boundaryMode=bnd)
     da = np.full((2, Hi, Wi, 4), 1.3 / S, np.float32) if "mipmap" in filt else None
-    t = dev(tex).requires_grad_(True)
-    DiffRast.texture(t, dev(uv), uvDA=None if da is None else dev(da), **kw).backward(dev(g))
+    t, u = dev(tex).requires_grad_(True), dev(uv).requires_grad_(uv_grad)
+    DiffRast.texture(t, u, uvDA=None if da is None else dev(da), **kw).backward(dev(g))
     ref = O.texture_vjp(tex, uv, g, uvDA=da, **kw)[0]
     assert_same_nonfinite(host(t.grad), ref, "d_tex")
